@@ -380,11 +380,26 @@ __device__ __forceinline__ void single_fit(const LDS& L, const ColourSet& cs, in
     }
 }
 
-// range.rs: clamp to [0,1] then snap to the 565 grid
+// A constant kept in a vector register.  As an operand of a VOP3 form (which
+// takes no literal) the compiler would put it in a scalar register, and a
+// scalar operand halves the issue rate of FP32 instructions (v_fma_f32 with
+// two vector sources and an inline constant: 21.8 lanes per clock and SIMD at
+// 4 waves, with a scalar source 13.8).
+__device__ __forceinline__ float vector_const(float c)
+{
+    asm("" : "+v"(c));
+    return c;
+}
+
+// range.rs: clamp to [0,1] then snap to the 565 grid, trunc(grid * v + 0.5)
+// * rcp.  The product and the sum are one fused operation: for both grids (31
+// and 63) trunc(fma(grid, v, 0.5)) equals trunc(fl(fl(grid * v) + 0.5)) for
+// every binary32 v in [0, 1] (both are monotone in v, and each of the 31 / 63
+// steps falls on the same v; the test suite checks every step).
 __device__ __forceinline__ float snap(float v, float grid, float rcp)
 {
     v = fminf(1.0f, fmaxf(0.0f, v));
-    return truncf(grid * v + 0.5f) * rcp;
+    return truncf(__builtin_fmaf(grid, v, 0.5f)) * rcp;
 }
 
 // range.rs:44-192
@@ -478,6 +493,12 @@ __device__ __forceinline__ void range_fit(const LDS& L, const ColourSet& cs, int
     if (do4 && error4 < best) write_colour(true, s0, s1, s2, e0, e1, e2, cs.remap < 0 ? 3u : mine4, l, lo, hi);
 }
 
+// The two snap grids in vector registers, made once ahead of a split loop.
+struct SnapGrids {
+    float g5, g6;
+};
+__device__ __forceinline__ SnapGrids snap_grids() { return SnapGrids{vector_const(31.0f), vector_const(63.0f)}; }
+
 // The three prefix sums a split reads: part0 = S[0][i], part1, part2.
 struct SplitSums {
     float4 p0, p1, p2;
@@ -501,8 +522,9 @@ __device__ __forceinline__ SplitSums load_split(const GroupLds& L, uint32_t code
 // unit-weight table entry of this candidate, which holds exactly the values
 // the expressions below produce when every point weight is 1.
 template <int NC, bool UNIT = false>
-__device__ __forceinline__ float eval_split(const SplitSums& s, const float4& xs, const FitParams& fp, float (&a)[3],
-                                            float (&b)[3], const txt::UnitSplit& u = txt::UnitSplit{})
+__device__ __forceinline__ float eval_split(const SplitSums& s, const float4& xs, const FitParams& fp,
+                                            const SnapGrids& sg, float (&a)[3], float (&b)[3],
+                                            const txt::UnitSplit& u = txt::UnitSplit{})
 {
     const float4 p0 = s.p0;
     const float4 p1 = s.p1;
@@ -569,7 +591,7 @@ __device__ __forceinline__ float eval_split(const SplitSums& s, const float4& xs
         }
     }
     const float factor = UNIT ? u.factor : 1.0f / ((a2 * b2) - ab * ab);
-    const float grid[3] = {31.0f, 63.0f, 31.0f};
+    const float grid[3] = {sg.g5, sg.g6, sg.g5};
     const float rcp[3] = {1.0f / 31.0f, 1.0f / 63.0f, 1.0f / 31.0f};
     const float wts[3] = {fp.wr, fp.wg, fp.wb};
     float e5[3];
@@ -727,6 +749,7 @@ __device__ __forceinline__ void search_loop(const GroupLds& L, int l, uint32_t m
     const uint32_t limA = mylen > (uint32_t)l ? mylen - (uint32_t)l : 0u;
     const uint32_t limB = mylen > (uint32_t)l + 16u ? mylen - (uint32_t)l - 16u : 0u;
     const uint32_t wlen = (uint32_t)__builtin_amdgcn_readfirstlane((int)wave_max_of_groups(mylen));
+    const SnapGrids sg = snap_grids();
     be = __builtin_huge_valf();
     bc = 0xFFFFFFFFu;
     auto keep = [&](float err, uint32_t c) {
@@ -748,14 +771,14 @@ __device__ __forceinline__ void search_loop(const GroupLds& L, int l, uint32_t m
         if (UNIT) uB = unit_at(ub + 256);
         if (base < limA) {
             float a[3], b[3];
-            keep(eval_split<NC, UNIT>(sA, xs, fp, a, b, uA), cA);
+            keep(eval_split<NC, UNIT>(sA, xs, fp, sg, a, b, uA), cA);
         }
         const uint32_t cB2 = code_at(so + 192);
         sA = load_split<NC>(L, cA2);
         if (UNIT) uA = unit_at(ub + 512);
         if (base < limB) {
             float a[3], b[3];
-            keep(eval_split<NC, UNIT>(sB, xs, fp, a, b, uB), cB);
+            keep(eval_split<NC, UNIT>(sB, xs, fp, sg, a, b, uB), cB);
         }
         cA = cA2;
         cB = cB2;
@@ -787,7 +810,7 @@ template <int NC>
 __device__ __forceinline__ void split_endpoints(const GroupLds& L, int n, uint32_t code, const FitParams& fp,
                                                 float (&sa)[3], float (&sb)[3])
 {
-    eval_split<NC>(load_split<NC>(L, code), L.S[n], fp, sa, sb);
+    eval_split<NC>(load_split<NC>(L, code), L.S[n], fp, snap_grids(), sa, sb);
 }
 
 // Index of this lane's pixel for the winning split (cluster.rs:252-273 /
