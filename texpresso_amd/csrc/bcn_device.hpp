@@ -52,7 +52,7 @@ struct __align__(16) FrontLds {
     __device__ uint32_t pix(int m) const { return pixels[m]; }
 };
 
-// Per-group LDS (one per 4x4 block in flight), 2512 bytes, so that 16
+// Per-group LDS (one per 4x4 block in flight), 2544 bytes, so that 16
 // single-wave workgroups (64 groups) fit in a CU's 160 KiB.  The first 80
 // bytes of the prefix table are also scratch while they hold nothing live:
 // the block's pixels at the start of a block, then, while an ordering is
@@ -62,6 +62,7 @@ struct __align__(16) GroupLds {
     float4 S[txt::kSEntries];  // prefix sums of the weighted ordered points (txt::soff layout)
     float4 pts[16];            // distinct colours: x, y, z, sqrt(weight)
     uint2 ord[8];              // orderings searched so far, 16 four-bit indices each
+    uint32_t keep[8];          // the block's state that a split search does not read (k_pipe_search)
 
     __device__ float* keys() { return reinterpret_cast<float*>(S); }
     __device__ const float* keys() const { return reinterpret_cast<const float*>(S); }
@@ -70,7 +71,7 @@ struct __align__(16) GroupLds {
     __device__ void put_pix(int l, uint32_t px) { keys()[l] = __uint_as_float(px); }
     __device__ uint32_t pix(int m) const { return __float_as_uint(keys()[m]); }
 };
-static_assert(sizeof(GroupLds) == 2512, "group LDS size");
+static_assert(sizeof(GroupLds) == 2544, "group LDS size");
 
 // Device copies of the constexpr tables (one per translation unit: the code
 // objects are built without relocatable device code).
@@ -135,7 +136,7 @@ __device__ __forceinline__ void argmin_step(float& e, uint32_t& c)
 {
     const float e2 = ror16f<N>(e);
     const uint32_t c2 = ror16<N>(c);
-    const bool take = (e2 < e) || (e2 == e && c2 < c);
+    const bool take = (e2 < e) | ((e2 == e) & (c2 < c));
     e = take ? e2 : e;
     c = take ? c2 : c;
 }
@@ -164,12 +165,12 @@ __device__ __forceinline__ uint32_t pack_565(float x, float y, float z)
     return (r << 11) | (g << 5) | b;
 }
 
-// colourblock.rs:58-94.  `idx` is this lane's pixel index; the group's
-// packed block comes back in (lo, hi) on every lane of the group.
-__device__ __forceinline__ void write_colour(bool four, float sx, float sy, float sz, float ex, float ey, float ez,
-                                             uint32_t idx, int l, uint32_t& lo, uint32_t& hi)
+// colourblock.rs:58-94 from packed endpoints.  `idx` is this lane's pixel
+// index; the group's packed block comes back in (lo, hi) on every lane of the
+// group.
+__device__ __forceinline__ void write_packed(bool four, uint32_t a, uint32_t b, uint32_t idx, int l, uint32_t& lo,
+                                             uint32_t& hi)
 {
-    uint32_t a = pack_565(sx, sy, sz), b = pack_565(ex, ey, ez);
     if (!four) {
         if (a > b) {  // write3: a <= b, swap palette slots 0 and 1
             const uint32_t t = a; a = b; b = t;
@@ -185,6 +186,12 @@ __device__ __forceinline__ void write_colour(bool four, float sx, float sy, floa
     }
     lo = a | (b << 16);
     hi = grp_or((idx & 3u) << (2 * l));
+}
+
+__device__ __forceinline__ void write_colour(bool four, float sx, float sy, float sz, float ex, float ey, float ez,
+                                             uint32_t idx, int l, uint32_t& lo, uint32_t& hi)
+{
+    write_packed(four, pack_565(sx, sy, sz), pack_565(ex, ey, ez), idx, l, lo, hi);
 }
 
 // ------------------------------------------------------------ alpha paths
@@ -396,10 +403,35 @@ __device__ __forceinline__ float vector_const(float c)
 // and 63) trunc(fma(grid, v, 0.5)) equals trunc(fl(fl(grid * v) + 0.5)) for
 // every binary32 v in [0, 1] (both are monotone in v, and each of the 31 / 63
 // steps falls on the same v; the test suite checks every step).
-__device__ __forceinline__ float snap(float v, float grid, float rcp)
+__device__ __forceinline__ float snap_level(float v, float grid)
 {
     v = fminf(1.0f, fmaxf(0.0f, v));
-    return truncf(__builtin_fmaf(grid, v, 0.5f)) * rcp;
+    return truncf(__builtin_fmaf(grid, v, 0.5f));
+}
+__device__ __forceinline__ float snap(float v, float grid, float rcp) { return snap_level(v, grid) * rcp; }
+
+// Snapped endpoints as a 565 word, and back: a level m of a grid is the value
+// m * rcp, and pack_565 of that value is m again (31 * fl(m / 31) and
+// 63 * fl(m / 63) round to m for every level).
+__device__ __forceinline__ uint32_t pack_levels(float r, float g, float b)
+{
+    return ((uint32_t)r << 11) | ((uint32_t)g << 5) | (uint32_t)b;
+}
+__device__ __forceinline__ void unpack_levels(uint32_t w, float& x, float& y, float& z)
+{
+    x = (float)(w >> 11) * (1.0f / 31.0f);
+    y = (float)((w >> 5) & 63u) * (1.0f / 63.0f);
+    z = (float)(w & 31u) * (1.0f / 31.0f);
+}
+// The axis of the next ordering: best end - best start (cluster.rs:247-249).
+__device__ __forceinline__ void ends_axis(uint32_t a, uint32_t b, float& x, float& y, float& z)
+{
+    float ax, ay, az, bx, by, bz;
+    unpack_levels(a, ax, ay, az);
+    unpack_levels(b, bx, by, bz);
+    x = bx - ax;
+    y = by - ay;
+    z = bz - az;
 }
 
 // range.rs:44-192
@@ -493,11 +525,11 @@ __device__ __forceinline__ void range_fit(const LDS& L, const ColourSet& cs, int
     if (do4 && error4 < best) write_colour(true, s0, s1, s2, e0, e1, e2, cs.remap < 0 ? 3u : mine4, l, lo, hi);
 }
 
-// The two snap grids in vector registers, made once ahead of a split loop.
-struct SnapGrids {
-    float g5, g6;
-};
-__device__ __forceinline__ SnapGrids snap_grids() { return SnapGrids{vector_const(31.0f), vector_const(63.0f)}; }
+// Entry of a prefix table at a byte offset.
+__device__ __forceinline__ float4 sum_at(const float4* S, uint32_t bytes)
+{
+    return *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(S) + bytes);
+}
 
 // The three prefix sums a split reads: part0 = S[0][i], part1, part2.
 struct SplitSums {
@@ -505,113 +537,162 @@ struct SplitSums {
 };
 
 template <int NC>
-__device__ __forceinline__ SplitSums load_split(const GroupLds& L, uint32_t code)
+__device__ __forceinline__ SplitSums load_split(const GroupLds& L, const txt::SplitOne& e)
 {
     SplitSums s;
-    s.p0 = L.S[(code >> 16) & 15u];
-    s.p1 = L.S[code & 255u];
-    if (NC == 4) s.p2 = L.S[(code >> 8) & 255u];
+    s.p0 = sum_at(L.S, e.key & 0xFFFFu);
+    s.p1 = sum_at(L.S, e.o & 0xFFFFu);
+    if (NC == 4) s.p2 = sum_at(L.S, e.o >> 16);
     else s.p2 = s.p1;
     return s;
 }
 
-// One split of the ClusterFit search (cluster.rs:189-230 for compress3,
-// 320-364 for compress4).  Returns the weighted error; the quantised
-// endpoints come back through a and b.  With UNIT the weight terms
-// (alpha2_sum, beta2_sum, alphabeta_sum, factor) come from `u`, the
-// unit-weight table entry of this candidate, which holds exactly the values
-// the expressions below produce when every point weight is 1.
-template <int NC, bool UNIT = false>
-__device__ __forceinline__ float eval_split(const SplitSums& s, const float4& xs, const FitParams& fp,
-                                            const SnapGrids& sg, float (&a)[3], float (&b)[3],
-                                            const txt::UnitSplit& u = txt::UnitSplit{})
+// What a 4-colour split needs of (j, k) alone and of (i, j) alone: with
+// part3 = xsum - part2 - part1 - part0,
+//   alphax = part2*(1/3,1/3,1/3,1/9) + (part1*(2/3,2/3,2/3,4/9) + part0)
+//   betax  = part1*(1/3,..,1/9) + (part2*(2/3,..,4/9) + part3)
+// (cluster.rs:320-330).  The binary32 constants satisfy 2/3 = 2 * (1/3) and
+// 4/9 = 4 * (1/9) exactly (same significand), and scaling by a power of two
+// commutes with rounding for the normal values summed here, so
+// p * (2/3) + q == fma(2, p * (1/3), q) bit for bit: one product per part
+// serves both alphax and betax.
+struct SplitCol {    // part2
+    float4 q, m, p;  // xsum - part2; part2 * (1/3,1/3,1/3,1/9); part2
+};
+struct SplitRow {          // part0 and part1
+    float4 p0, p1, m, f;   // part1 * (1/3,..,1/9); part1 * (2/3,..,4/9) + part0
+};
+static_assert(2.0f * (1.0f / 3.0f) == 2.0f / 3.0f && 4.0f * (1.0f / 9.0f) == 4.0f / 9.0f,
+              "2/3 and 4/9 are exact multiples of 1/3 and 1/9");
+
+__device__ __forceinline__ SplitCol split_col(const float4& p2, const float4& xs)
 {
-    const float4 p0 = s.p0;
-    const float4 p1 = s.p1;
-    float ax[3], bx[3], a2, b2, ab;
-    if (NC == 4) {
-        const float4 p2 = s.p2;
-        // part3 = xsum - part2 - part1 - part0
-        const float p3x = ((xs.x - p2.x) - p1.x) - p0.x;
-        const float p3y = ((xs.y - p2.y) - p1.y) - p0.y;
-        const float p3z = ((xs.z - p2.z) - p1.z) - p0.z;
-        // alphax = part2*(1/3,1/3,1/3,1/9) + (part1*(2/3,2/3,2/3,4/9) + part0)
-        // betax  = part1*(1/3,..,1/9) + (part2*(2/3,..,4/9) + part3)
-        // The binary32 constants satisfy 2/3 = 2 * (1/3) and 4/9 = 4 * (1/9)
-        // exactly (same significand), and scaling by a power of two commutes
-        // with rounding for the normal values summed here, so
-        // p * (2/3) + q == fma(2, p * (1/3), q) bit for bit: one product per
-        // part serves both alphax and betax.
-        const float t13 = 1.0f / 3.0f, n19 = 1.0f / 9.0f;
-        static_assert(2.0f * (1.0f / 3.0f) == 2.0f / 3.0f && 4.0f * (1.0f / 9.0f) == 4.0f / 9.0f,
-                      "2/3 and 4/9 are exact multiples of 1/3 and 1/9");
-        const float m1x = p1.x * t13, m1y = p1.y * t13, m1z = p1.z * t13;
-        const float m2x = p2.x * t13, m2y = p2.y * t13, m2z = p2.z * t13;
-        ax[0] = m2x + __builtin_fmaf(2.0f, m1x, p0.x);
-        ax[1] = m2y + __builtin_fmaf(2.0f, m1y, p0.y);
-        ax[2] = m2z + __builtin_fmaf(2.0f, m1z, p0.z);
-        bx[0] = m1x + __builtin_fmaf(2.0f, m2x, p3x);
-        bx[1] = m1y + __builtin_fmaf(2.0f, m2y, p3y);
-        bx[2] = m1z + __builtin_fmaf(2.0f, m2z, p3z);
-        if (UNIT) {
-            a2 = u.a2;
-            b2 = u.b2;
-            ab = u.ab;
-        } else {
-            const float p3w = ((xs.w - p2.w) - p1.w) - p0.w;
-            const float w1 = p1.w * n19, w2 = p2.w * n19;
-            a2 = w2 + __builtin_fmaf(4.0f, w1, p0.w);
-            b2 = w1 + __builtin_fmaf(4.0f, w2, p3w);
-            ab = (2.0f / 9.0f) * (p1.w + p2.w);
-        }
+    const float t13 = 1.0f / 3.0f, n19 = 1.0f / 9.0f;
+    return SplitCol{make_float4(xs.x - p2.x, xs.y - p2.y, xs.z - p2.z, xs.w - p2.w),
+                    make_float4(p2.x * t13, p2.y * t13, p2.z * t13, p2.w * n19), p2};
+}
+__device__ __forceinline__ SplitRow split_row(const float4& p0, const float4& p1)
+{
+    const float t13 = 1.0f / 3.0f, n19 = 1.0f / 9.0f;
+    const float4 m = make_float4(p1.x * t13, p1.y * t13, p1.z * t13, p1.w * n19);
+    return SplitRow{p0, p1, m,
+                    make_float4(__builtin_fmaf(2.0f, m.x, p0.x), __builtin_fmaf(2.0f, m.y, p0.y),
+                                __builtin_fmaf(2.0f, m.z, p0.z), __builtin_fmaf(4.0f, m.w, p0.w))};
+}
+
+// alphax_sum, betax_sum and the weight terms of one split.
+struct SplitTerms {
+    float ax[3], bx[3];
+    txt::UnitSplit u;  // alpha2_sum, beta2_sum, alphabeta_sum, factor
+};
+
+// 4-colour terms (cluster.rs:320-335).  With UNIT the weight terms come from
+// `u`, the unit-weight table entry of this split, which holds exactly the
+// values the expressions below produce when every point weight is 1.
+template <bool UNIT>
+__device__ __forceinline__ SplitTerms split_terms4(const SplitRow& r, const SplitCol& c, const txt::UnitSplit& u)
+{
+    SplitTerms t;
+    // part3, then alphax and betax
+    const float p3x = (c.q.x - r.p1.x) - r.p0.x;
+    const float p3y = (c.q.y - r.p1.y) - r.p0.y;
+    const float p3z = (c.q.z - r.p1.z) - r.p0.z;
+    t.ax[0] = c.m.x + r.f.x;
+    t.ax[1] = c.m.y + r.f.y;
+    t.ax[2] = c.m.z + r.f.z;
+    t.bx[0] = r.m.x + __builtin_fmaf(2.0f, c.m.x, p3x);
+    t.bx[1] = r.m.y + __builtin_fmaf(2.0f, c.m.y, p3y);
+    t.bx[2] = r.m.z + __builtin_fmaf(2.0f, c.m.z, p3z);
+    if (UNIT) {
+        t.u = u;
     } else {
-        // part2 = xsum - part1 - part0; alphax = part1*(.5,.5,.5) + part0,
-        // betax = part1*(.5,.5,.5) + part2.  Halving is exact for the normal
-        // prefix sums, so the fused form rounds once exactly as the
-        // product-then-add does.
-        const float p2x = (xs.x - p1.x) - p0.x;
-        const float p2y = (xs.y - p1.y) - p0.y;
-        const float p2z = (xs.z - p1.z) - p0.z;
-        ax[0] = __builtin_fmaf(0.5f, p1.x, p0.x);
-        ax[1] = __builtin_fmaf(0.5f, p1.y, p0.y);
-        ax[2] = __builtin_fmaf(0.5f, p1.z, p0.z);
-        bx[0] = __builtin_fmaf(0.5f, p1.x, p2x);
-        bx[1] = __builtin_fmaf(0.5f, p1.y, p2y);
-        bx[2] = __builtin_fmaf(0.5f, p1.z, p2z);
-        if (UNIT) {
-            a2 = u.a2;
-            b2 = u.b2;
-            ab = u.ab;
-        } else {
-            const float p2w = (xs.w - p1.w) - p0.w;
-            const float hw = p1.w * 0.25f;
-            a2 = hw + p0.w;
-            b2 = hw + p2w;
-            ab = hw;
-        }
+        const float p3w = (c.q.w - r.p1.w) - r.p0.w;
+        t.u.a2 = c.m.w + r.f.w;
+        t.u.b2 = r.m.w + __builtin_fmaf(4.0f, c.m.w, p3w);
+        t.u.ab = (2.0f / 9.0f) * (r.p1.w + c.p.w);
+        t.u.factor = 1.0f / ((t.u.a2 * t.u.b2) - t.u.ab * t.u.ab);
     }
-    const float factor = UNIT ? u.factor : 1.0f / ((a2 * b2) - ab * ab);
+    return t;
+}
+
+// 3-colour terms (cluster.rs:189-202): part2 = xsum - part1 - part0; alphax =
+// part1*(.5,.5,.5) + part0, betax = part1*(.5,.5,.5) + part2.  Halving is
+// exact for the normal prefix sums, so the fused form rounds once exactly as
+// the product-then-add does.
+template <bool UNIT>
+__device__ __forceinline__ SplitTerms split_terms3(const float4& p0, const float4& p1, const float4& xs,
+                                                   const txt::UnitSplit& u)
+{
+    SplitTerms t;
+    const float p2x = (xs.x - p1.x) - p0.x;
+    const float p2y = (xs.y - p1.y) - p0.y;
+    const float p2z = (xs.z - p1.z) - p0.z;
+    t.ax[0] = __builtin_fmaf(0.5f, p1.x, p0.x);
+    t.ax[1] = __builtin_fmaf(0.5f, p1.y, p0.y);
+    t.ax[2] = __builtin_fmaf(0.5f, p1.z, p0.z);
+    t.bx[0] = __builtin_fmaf(0.5f, p1.x, p2x);
+    t.bx[1] = __builtin_fmaf(0.5f, p1.y, p2y);
+    t.bx[2] = __builtin_fmaf(0.5f, p1.z, p2z);
+    if (UNIT) {
+        t.u = u;
+    } else {
+        const float p2w = (xs.w - p1.w) - p0.w;
+        const float hw = p1.w * 0.25f;
+        t.u.a2 = hw + p0.w;
+        t.u.b2 = hw + p2w;
+        t.u.ab = hw;
+        t.u.factor = 1.0f / ((t.u.a2 * t.u.b2) - t.u.ab * t.u.ab);
+    }
+    return t;
+}
+
+// The two snap grids in vector registers, made once ahead of a split loop.
+struct SnapGrids {
+    float g5, g6;
+};
+__device__ __forceinline__ SnapGrids snap_grids() { return SnapGrids{vector_const(31.0f), vector_const(63.0f)}; }
+
+// Least-squares endpoints of a split on one channel (cluster.rs:203-212 /
+// 336-345), as levels of its grid.
+__device__ __forceinline__ void split_levels(const SplitTerms& t, int c, float grid, float& a, float& b)
+{
+    a = snap_level(((t.ax[c] * t.u.b2) - t.bx[c] * t.u.ab) * t.u.factor, grid);
+    b = snap_level(((t.bx[c] * t.u.a2) - t.ax[c] * t.u.ab) * t.u.factor, grid);
+}
+
+// Weighted error of a split with its endpoints snapped (cluster.rs:203-230 /
+// 336-364).
+__device__ __forceinline__ float split_error(const SplitTerms& t, const FitParams& fp, const SnapGrids& sg)
+{
     const float grid[3] = {sg.g5, sg.g6, sg.g5};
     const float rcp[3] = {1.0f / 31.0f, 1.0f / 63.0f, 1.0f / 31.0f};
     const float wts[3] = {fp.wr, fp.wg, fp.wb};
+    const float a2 = t.u.a2, b2 = t.u.b2, ab = t.u.ab;
     float e5[3];
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-        float av = ((ax[c] * b2) - bx[c] * ab) * factor;
-        float bv = ((bx[c] * a2) - ax[c] * ab) * factor;
-        av = snap(av, grid[c], rcp[c]);
-        bv = snap(bv, grid[c], rcp[c]);
-        a[c] = av;
-        b[c] = bv;
+        float av, bv;
+        split_levels(t, c, grid[c], av, bv);
+        av = av * rcp[c];
+        bv = bv * rcp[c];
         const float e1 = (av * av) * a2 + ((bv * bv) * b2);
-        const float e2 = ((av * bv) * ab) - av * ax[c];
-        const float e3 = e2 - bv * bx[c];
+        const float e2 = ((av * bv) * ab) - av * t.ax[c];
+        const float e3 = e2 - bv * t.bx[c];
         // 2 * e3 is exact (a power-of-two scaling of a small finite value),
         // so the fused form rounds once, exactly like the product-then-add
         const float e4 = __builtin_fmaf(2.0f, e3, e1);
         e5[c] = e4 * wts[c];
     }
     return (e5[0] + e5[1]) + e5[2];
+}
+
+// The terms of one split on its own.
+template <int NC, bool UNIT = false>
+__device__ __forceinline__ SplitTerms split_terms(const SplitSums& s, const float4& xs,
+                                                  const txt::UnitSplit& u = txt::UnitSplit{})
+{
+    if (NC == 4) return split_terms4<UNIT>(split_row(s.p0, s.p1), split_col(s.p2, xs), u);
+    return split_terms3<UNIT>(s.p0, s.p1, xs, u);
 }
 
 // LDS hand-off between the lanes of one group.  Groups never share LDS and a
@@ -722,108 +803,230 @@ __device__ __forceinline__ uint32_t wave_max_of_groups(uint32_t v)
     return max(max(a, b), max(c, d));
 }
 
-// Candidate loop of one split search (see search_step).
-template <int NC, bool UNIT>
-__device__ __forceinline__ void search_loop(const GroupLds& L, int l, uint32_t mylen, const float4& xs,
-                                            const FitParams& fp, float& be, uint32_t& bc)
+// A raw buffer over a constant table: reads past its end return 0 (an entry
+// of the prefix table's first rows, loaded ahead but never evaluated).
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t table_rsrc(const void* p, uint32_t bytes)
 {
-    // Trip q covers list entries 32q .. 32q + 31: lane l evaluates entry
-    // 32q + l (A) and 32q + 16 + l (B), each while 32q is below its limit.
-    // Loop control and the trip's offsets are scalar: the code list is read
-    // through a buffer resource with the lane's offset in a vector register
-    // and the trip's in a scalar one (hardware bounds checks: a read past
-    // the end returns 0), the 16-byte unit entries from a scalar base plus
-    // the lane's offset.  Codes are read two half-trips ahead and prefix
-    // sums one half-trip ahead.  The kept minimum is the smallest (error,
-    // code), codes ordered by loop-order rank, so evaluation order does not
-    // matter; the three comparisons are combined without branches.  The
-    // lists are padded past the longest trip: reads need no guard, and
-    // entries at or past `mylen` are loaded but never evaluated.
-    constexpr int kStored = NC == 4 ? txt::kCand4Stored : txt::kCand3Stored;
-    const __amdgpu_buffer_rsrc_t rt =
-        __builtin_amdgcn_make_buffer_rsrc((void*)(NC == 4 ? c_cand.t4 : c_cand.t3), 0, kStored * 4, kBufferFlags);
-    const char* ubase = reinterpret_cast<const char*>(NC == 4 ? c_unit.u4 : c_unit.u3);
-    const uint32_t vo = 4u * (uint32_t)l, uo = 16u * (uint32_t)l;
-    auto code_at = [&](uint32_t soff) { return __builtin_amdgcn_raw_buffer_load_b32(rt, vo, soff, 0); };
-    auto unit_at = [&](const char* base) { return *reinterpret_cast<const txt::UnitSplit*>(base + uo); };
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, kBufferFlags);
+}
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ txt::UnitSplit unit_at(__amdgpu_buffer_rsrc_t r, uint32_t vo, uint32_t so)
+{
+    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, vo, so, 0);
+    return txt::UnitSplit{__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]), __uint_as_float(v[3])};
+}
+
+// (error, key) of the splits a lane has seen: `see` for splits that come in
+// key order (the first strict minimum is kept), `merge` for another lane's
+// or list's.
+struct BestSplit {
+    float e = __builtin_huge_valf();
+    uint32_t c = 0xFFFFFFFFu;
+
+    __device__ __forceinline__ void see(float err, uint32_t key)
+    {
+        const bool take = err < e;
+        e = take ? err : e;
+        c = take ? key : c;
+    }
+    __device__ __forceinline__ void merge(float err, uint32_t key)
+    {
+        const bool take = (err < e) | ((err == e) & (key < c));
+        e = take ? err : e;
+        c = take ? key : c;
+    }
+};
+
+// The single splits of a list (all of a 3-colour search, the odd rows and
+// columns of a 4-colour one).  Trip q covers entries 32q .. 32q + 31: lane l
+// evaluates entry 32q + l (A) and 32q + 16 + l (B), each while 32q is below
+// its limit, so a lane meets its entries in key order.  Loop control and the
+// trip's offsets are scalar: the list is read through a buffer resource with
+// the lane's offset in a vector register and the trip's in a scalar one.
+// Entries are read two half-trips ahead and prefix sums one half-trip ahead.
+template <int NC, bool UNIT>
+__device__ __forceinline__ void search_ones(const GroupLds& L, int l, const txt::SplitList& list, uint32_t wlen,
+                                            const float4& xs, const FitParams& fp, const SnapGrids& sg,
+                                            BestSplit& best)
+{
+    const __amdgpu_buffer_rsrc_t rt = NC == 4 ? table_rsrc(c_cand.one4, sizeof c_cand.one4)
+                                              : table_rsrc(c_cand.one3, sizeof c_cand.one3);
+    const __amdgpu_buffer_rsrc_t ru = NC == 4 ? table_rsrc(c_unit.one4, sizeof c_unit.one4)
+                                              : table_rsrc(c_unit.one3, sizeof c_unit.one3);
+    const uint32_t mylen = list.len;
+    const uint32_t vo = 8u * ((uint32_t)list.start + (uint32_t)l), uo = 16u * (uint32_t)l;
+    auto one_at = [&](uint32_t so) {
+        const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(rt, vo, so, 0);
+        return txt::SplitOne{v[0], v[1]};
+    };
     const uint32_t limA = mylen > (uint32_t)l ? mylen - (uint32_t)l : 0u;
     const uint32_t limB = mylen > (uint32_t)l + 16u ? mylen - (uint32_t)l - 16u : 0u;
-    const uint32_t wlen = (uint32_t)__builtin_amdgcn_readfirstlane((int)wave_max_of_groups(mylen));
-    const SnapGrids sg = snap_grids();
-    be = __builtin_huge_valf();
-    bc = 0xFFFFFFFFu;
-    auto keep = [&](float err, uint32_t c) {
-        const bool take = (err < be) | ((err == be) & (c < bc));
-        be = take ? err : be;
-        bc = take ? c : bc;
-    };
-    uint32_t cA = code_at(0);
-    uint32_t cB = code_at(64);
+    BestSplit mine;
+    txt::SplitOne cA = one_at(0);
+    txt::SplitOne cB = one_at(128);
     SplitSums sA = load_split<NC>(L, cA);
     txt::UnitSplit uA{};
-    if (UNIT) uA = unit_at(ubase);
+    if (UNIT) uA = unit_at(ru, uo, 0);
     for (uint32_t base = 0; base < wlen; base += 32) {
-        const uint32_t so = 4u * base;
-        const char* ub = ubase + 16u * base;
-        const uint32_t cA2 = code_at(so + 128);
+        const uint32_t so = 8u * base, su = 16u * base;
+        const txt::SplitOne cA2 = one_at(so + 256);
         const SplitSums sB = load_split<NC>(L, cB);
         txt::UnitSplit uB{};
-        if (UNIT) uB = unit_at(ub + 256);
+        if (UNIT) uB = unit_at(ru, uo, su + 256);
         if (base < limA) {
-            float a[3], b[3];
-            keep(eval_split<NC, UNIT>(sA, xs, fp, sg, a, b, uA), cA);
+            mine.see(split_error(split_terms<NC, UNIT>(sA, xs, uA), fp, sg), cA.key);
         }
-        const uint32_t cB2 = code_at(so + 192);
+        const txt::SplitOne cB2 = one_at(so + 384);
         sA = load_split<NC>(L, cA2);
-        if (UNIT) uA = unit_at(ub + 512);
+        if (UNIT) uA = unit_at(ru, uo, su + 512);
         if (base < limB) {
-            float a[3], b[3];
-            keep(eval_split<NC, UNIT>(sB, xs, fp, sg, a, b, uB), cB);
+            mine.see(split_error(split_terms<NC, UNIT>(sB, xs, uB), fp, sg), cB.key);
         }
         cA = cA2;
         cB = cB2;
     }
+    best.merge(mine.e, mine.c);
+}
+
+// The 2 x 2 tiles of a 4-colour list, one tile per lane and trip.  The loop is
+// bound by VALU issue; a tile computes what depends on (j, k) alone and on
+// (i, j) alone once for two splits each, decodes one list entry for four and
+// needs no tie compare (each row is met in key order), which takes a split
+// from 130 to 106 VALU instructions (unit weights).  With every load a step
+// ahead of its use (the barriers keep the scheduler from sinking them: without
+// them the loop waits out four table loads a tile and gains nothing), 2048^2
+// BC3 IterativeClusterFit went from 1011 to 937 us.  Other weights need 26
+// more registers, so there the sums are read at the tile's start.
+template <bool UNIT>
+__device__ __forceinline__ void search_tiles(const GroupLds& L, int l, const txt::SplitList& list, uint32_t wlen,
+                                             const float4& xs, const FitParams& fp, const SnapGrids& sg,
+                                             BestSplit& best)
+{
+    const __amdgpu_buffer_rsrc_t rt = table_rsrc(c_cand.tile, sizeof c_cand.tile);
+    const __amdgpu_buffer_rsrc_t ru = table_rsrc(c_unit.tile, sizeof c_unit.tile);
+    constexpr uint32_t kPos = sizeof c_unit.tile[0];  // bytes from one split of the tiles to the next
+    const uint32_t lim = list.len > l ? (uint32_t)list.len - (uint32_t)l : 0u;
+    const uint32_t vo = 12u * ((uint32_t)list.start + (uint32_t)l), uo = 16u * (uint32_t)l;
+    auto tile_at = [&](uint32_t so) { return __builtin_amdgcn_raw_buffer_load_b96(rt, vo, so, 0); };
+    auto unit = [&](uint32_t so) { return UNIT ? unit_at(ru, uo, so) : txt::UnitSplit{}; };
+    auto part0 = [&](uint32_t key, int r) { return sum_at(L.S + r, key & 0xFFFFu); };
+    BestSplit rows[2];  // rows i and i + 1 of the tiles, each met in key order
+    u32x3 t = tile_at(0), t2 = tile_at(192);
+    float4 p0, p1, c0, c1;  // the first row's and the columns' sums
+    auto load_sums = [&]() {
+        p0 = part0(t[2], 0);
+        p1 = sum_at(L.S, t[0] & 0xFFFFu);
+        c0 = sum_at(L.S, t[1] & 0xFFFFu);
+        c1 = sum_at(L.S, t[1] >> 16);
+    };
+    if (UNIT) load_sums();
+    txt::UnitSplit u0 = unit(0);
+    for (uint32_t base = 0; base < wlen; base += 16) {
+        const uint32_t su = 16u * base;
+        const bool live = base < lim;
+        const uint32_t key = t[2];
+        if (!UNIT) load_sums();
+        const float4 q0 = part0(t[2], 1), q1 = sum_at(L.S, t[0] >> 16);
+        txt::UnitSplit u1 = unit(su + kPos);
+        const SplitCol col0 = split_col(c0, xs), col1 = split_col(c1, xs);
+        __builtin_amdgcn_sched_barrier(0);
+        {
+            const SplitRow row = split_row(p0, p1);
+            if (live) rows[0].see(split_error(split_terms4<UNIT>(row, col0, u0), fp, sg), key);
+            u0 = unit(su + 2 * kPos);
+            __builtin_amdgcn_sched_barrier(0);
+            if (live) rows[0].see(split_error(split_terms4<UNIT>(row, col1, u1), fp, sg), key + txt::kKeyNextK);
+            u1 = unit(su + 3 * kPos);
+        }
+        t = t2;
+        t2 = tile_at(12u * base + 384u);
+        if (UNIT) load_sums();
+        __builtin_amdgcn_sched_barrier(0);
+        {
+            const SplitRow row = split_row(q0, q1);
+            if (live) rows[1].see(split_error(split_terms4<UNIT>(row, col0, u0), fp, sg), key);
+            u0 = unit(su + 256);
+            __builtin_amdgcn_sched_barrier(0);
+            if (live) rows[1].see(split_error(split_terms4<UNIT>(row, col1, u1), fp, sg), key + txt::kKeyNextK);
+        }
+    }
+    best.merge(rows[0].e, rows[0].c);
+    best.merge(rows[1].e, rows[1].c + txt::kKeyNextI);
 }
 
 // The split search over the current prefix table: every group with `run`
-// set evaluates its `len` candidates (16 lanes, list entries two rounds and
-// prefix sums one round ahead) and returns the first strict minimum
-// (error, code) on all of its lanes.  Executed by the whole wave.  When
-// every searching group holds 16 points of weight exactly 1, the weight
-// terms come from the unit-weight table (same values, fewer operations).
+// set evaluates its splits and returns the first strict minimum (error, key)
+// on all of its lanes.  Executed by the whole wave.  When every searching
+// group holds 16 points of weight exactly 1, the weight terms come from the
+// unit-weight table (same values, fewer operations).
+template <int NC, bool UNIT>
+__device__ __forceinline__ void search_loop(const GroupLds& L, int l, int n, bool run, const float4& xs,
+                                            const FitParams& fp, float& be, uint32_t& bc)
+{
+    // the tile and single lists of n colours, read together
+    txt::SplitLists lists{};
+    if (run) lists = NC == 4 ? c_cand.lists4[n] : c_cand.lists3[n];
+    auto longest = [&](uint32_t len) {
+        return (uint32_t)__builtin_amdgcn_readfirstlane((int)wave_max_of_groups(len));
+    };
+    const SnapGrids sg = snap_grids();
+    BestSplit best;
+    if (NC == 4) search_tiles<UNIT>(L, l, lists.tiles, longest(lists.tiles.len), xs, fp, sg, best);
+    search_ones<NC, UNIT>(L, l, lists.ones, longest(lists.ones.len), xs, fp, sg, best);
+    be = best.e;
+    bc = best.c;
+}
+
 template <int NC>
 __device__ __forceinline__ void search_step(const GroupLds& L, int l, int n, bool run, const FitParams& fp,
                                             float& be, uint32_t& bc)
 {
-    const uint32_t mylen = run ? (NC == 4 ? c_cand.len4[n] : c_cand.len3[n]) : 0u;
     const float4 xs = L.S[n];  // xsum_wsum = S[0][n]
     const bool unit = n == 16 && grp_min(L.pts[l].w == 1.0f ? 1u : 0u) == 1u;
     if (!wave_any(run && !unit))
-        search_loop<NC, true>(L, l, mylen, xs, fp, be, bc);
+        search_loop<NC, true>(L, l, n, run, xs, fp, be, bc);
     else
-        search_loop<NC, false>(L, l, mylen, xs, fp, be, bc);
+        search_loop<NC, false>(L, l, n, run, xs, fp, be, bc);
     grp_argmin(be, bc);
 }
 
-// Quantised endpoints of split `code` on the current prefix table.
-template <int NC>
-__device__ __forceinline__ void split_endpoints(const GroupLds& L, int n, uint32_t code, const FitParams& fp,
-                                                float (&sa)[3], float (&sb)[3])
+// txt::soff without branches (row a >= 1 of the table starts at entry
+// 17 + 16 (a - 1) - (a - 1) a / 2; row 0 at entry 1).
+__device__ __forceinline__ int sum_entry(int a, int b)
 {
-    eval_split<NC>(load_split<NC>(L, code), L.S[n], fp, snap_grids(), sa, sb);
+    const int row = a == 0 ? 1 : 17 + 16 * (a - 1) - (((a - 1) * a) >> 1);
+    return a == b ? 0 : row + (b - a - 1);
+}
+
+// Quantised endpoints of the split `key` on the current prefix table, packed.
+template <int NC>
+__device__ __forceinline__ void split_endpoints(const GroupLds& L, int n, uint32_t key, uint32_t& a, uint32_t& b)
+{
+    const int i = txt::key_i(key), j = txt::key_j(key), k = txt::key_k(key);
+    SplitSums s;
+    s.p0 = L.S[i];
+    s.p1 = L.S[sum_entry(i, j)];
+    s.p2 = NC == 4 ? L.S[sum_entry(j, k)] : s.p1;
+    const SplitTerms t = split_terms<NC>(s, L.S[n]);
+    float av[3], bv[3];
+    split_levels(t, 0, 31.0f, av[0], bv[0]);
+    split_levels(t, 1, 63.0f, av[1], bv[1]);
+    split_levels(t, 2, 31.0f, av[2], bv[2]);
+    a = pack_levels(av[0], av[1], av[2]);
+    b = pack_levels(bv[0], bv[1], bv[2]);
 }
 
 // Index of this lane's pixel for the winning split (cluster.rs:252-273 /
 // 391-416 followed by remap_indices): the three overwriting loops leave a
 // point with the value of the range holding its largest position q >= i.
 template <int NC>
-__device__ __forceinline__ uint32_t split_index(const GroupLds& L, int n, int remap, uint32_t code, int it)
+__device__ __forceinline__ uint32_t split_index(const GroupLds& L, int n, int remap, uint32_t key, int it)
 {
     if (remap < 0) return 3u;
-    const int i = (int)((code >> 16) & 15u);
-    const uint32_t o1 = code & 255u, o2 = (code >> 8) & 255u;
-    const int j = o1 ? (int)c_cand.off_b[o1] : i;
-    const int k = NC == 4 ? (o2 ? (int)c_cand.off_b[o2] : j) : 0;
+    const int i = txt::key_i(key), j = txt::key_j(key), k = txt::key_k(key);
     const uint2 ord = L.ord[it];
     int qmax = -1;
 #pragma unroll
@@ -855,7 +1058,7 @@ __device__ __forceinline__ void run_cluster(GroupLds& L, const ColourSet& cs, in
     float lb_err = thr;
     uint32_t lb_code = 0;
     int lb_it = 0;
-    float sa[3] = {0.0f, 0.0f, 0.0f}, sb[3] = {0.0f, 0.0f, 0.0f};  // best_start / best_end
+    uint32_t sa = 0, sb = 0;  // best_start / best_end
     float axx = px, axy = py, axz = pz;
     bool done = !act;
 
@@ -876,22 +1079,16 @@ __device__ __forceinline__ void run_cluster(GroupLds& L, const ColourSet& cs, in
                 lb_err = be;
                 lb_code = bc;
                 lb_it = it;
-                split_endpoints<NC>(L, n, bc, fp, sa, sb);
+                split_endpoints<NC>(L, n, bc, sa, sb);
             }
-            if (lb_it != it) {
-                done = true;
-            } else {
-                axx = sb[0] - sa[0];
-                axy = sb[1] - sa[1];
-                axz = sb[2] - sa[2];
-            }
+            if (lb_it != it) done = true;
+            else ends_axis(sa, sb, axx, axy, axz);
         }
     }
 
     if (act && lb_err < thr) {
         uint32_t nlo, nhi;
-        write_colour(NC == 4, sa[0], sa[1], sa[2], sb[0], sb[1], sb[2], split_index<NC>(L, n, cs.remap, lb_code, lb_it),
-                     l, nlo, nhi);
+        write_packed(NC == 4, sa, sb, split_index<NC>(L, n, cs.remap, lb_code, lb_it), l, nlo, nhi);
         lo = nlo;
         hi = nhi;
         best_err = lb_err;

@@ -45,11 +45,12 @@ __device__ __forceinline__ void run_chunk(const BatchTex& T, uint32_t first, uin
 // Persistent kernel: every wave takes chunks {texture, first block, count},
 // the first by its wave index and the rest from `counter`, until the queue
 // is exhausted.  A chunk's texture fixes the format and algorithm for the
-// whole wave, so the dispatch is wave-uniform.
+// whole wave, so the dispatch is wave-uniform.  At most 168 registers (three
+// waves per SIMD, the default 12 workgroups of a CU), without spills.
 template <int WAVES>
-__global__ __launch_bounds__(64 * WAVES) void k_batch(const BatchTex* __restrict__ tex,
-                                                     const uint4* __restrict__ chunks, uint32_t nchunks,
-                                                     uint32_t* __restrict__ counter)
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(3))) void k_batch(
+    const BatchTex* __restrict__ tex, const uint4* __restrict__ chunks, uint32_t nchunks,
+    uint32_t* __restrict__ counter)
 {
     __shared__ GroupLds lds[4 * WAVES];
     const int tid = (int)threadIdx.x, wave = tid >> 6, lane = tid & 63;

@@ -251,44 +251,47 @@ __global__ __launch_bounds__(256) void k_pipe_bin(const uint32_t* __restrict__ k
     }
 }
 
-// The record fields a finished block's output needs, read with the rest of
-// the record when the group takes it (not behind a load at emit time).
-struct RecOut {
-    uint32_t tex, block, alpha0, alpha1;
-};
+// A searched block's state that the split loops do not read, in GroupLds::keep
+// (the loops hold most of the 128 registers of a lane): its output fields,
+// read with the rest of the record when the group takes it (not behind a load
+// at emit time), its record slot, and three words that hold the principal axis
+// until the first ordering is built, then the best split's endpoints and key.
+enum { kKeepTex = 0, kKeepBlock = 1, kKeepAlpha = 2, kKeepRec = 4, kKeepAxis = 5, kKeepEnds = 5, kKeepKey = 7 };
 
 // Result of a finished block: the output block, or (NC = 3 for an opaque BC1
 // block) the 3-colour result kept in the record for the 4-colour pass.
 template <int NC>
-__device__ __forceinline__ void emit_block(const BatchTex* __restrict__ tex, const BatchTex& tex0, ClusterRec& R,
-                                           const RecOut& ro, uint32_t info, const GroupLds& L, int l, int n,
-                                           int remap, float lb_err, float thr, uint32_t lb_code, int lb_it,
-                                           const float (&sa)[3], const float (&sb)[3])
+__device__ __forceinline__ void emit_block(const BatchTex* __restrict__ tex, const BatchTex& tex0,
+                                           ClusterRec* __restrict__ recs, uint32_t info, const GroupLds& L, int l,
+                                           int n, int remap, float lb_err, float thr, int lb_it)
 {
     const uint32_t fmt = (info >> 12) & 15u;
     uint32_t lo = 0, hi = 0;
     const bool won = lb_err < thr;
+    ClusterRec& R = recs[L.keep[kKeepRec]];
     if (won) {
-        write_colour(NC == 4, sa[0], sa[1], sa[2], sb[0], sb[1], sb[2], split_index<NC>(L, n, remap, lb_code, lb_it),
-                     l, lo, hi);
+        write_packed(NC == 4, L.keep[kKeepEnds], L.keep[kKeepEnds + 1],
+                     split_index<NC>(L, n, remap, L.keep[kKeepKey], lb_it), l, lo, hi);
     } else if (NC == 4 && fmt == BC1) {
         lo = R.fit3[0];
         hi = R.fit3[1];
     }
     if (l == 0) {
-        const BatchTex& T = tex_at(tex, tex0, ro.tex);
+        uint8_t* const out = tex_at(tex, tex0, L.keep[kKeepTex]).out;
+        const size_t block = L.keep[kKeepBlock];
         if (NC == 3) {
             if ((info >> 8) & 1u) {
-                *reinterpret_cast<uint2*>(T.out + (size_t)ro.block * 8u) = make_uint2(lo, hi);
+                *reinterpret_cast<uint2*>(out + block * 8u) = make_uint2(lo, hi);
             } else {
                 R.fit3_err = won ? lb_err : thr;
                 R.fit3[0] = lo;
                 R.fit3[1] = hi;
             }
         } else if (fmt == BC1) {
-            *reinterpret_cast<uint2*>(T.out + (size_t)ro.block * 8u) = make_uint2(lo, hi);
+            *reinterpret_cast<uint2*>(out + block * 8u) = make_uint2(lo, hi);
         } else {
-            *reinterpret_cast<uint4*>(T.out + (size_t)ro.block * 16u) = make_uint4(ro.alpha0, ro.alpha1, lo, hi);
+            *reinterpret_cast<uint4*>(out + block * 16u) =
+                make_uint4(L.keep[kKeepAlpha], L.keep[kKeepAlpha + 1], lo, hi);
         }
     }
 }
@@ -389,12 +392,9 @@ __global__ __launch_bounds__(64 * kSearchWaves) __attribute__((amdgpu_waves_per_
     __syncthreads();
 
     bool idle = false, need = true, ready = false;
-    uint32_t r = 0, info = 0, lb_code = 0;
-    RecOut ro{0u, 0u, 0u, 0u};
-    int n = 0, iters = 1, it = 0, lb_it = 0, remap = -1;
+    uint32_t info = 0;
+    int it = 0, lb_it = 0, remap = -1;
     float thr = FLT_MAX, lb_err = FLT_MAX;
-    float sa[3] = {0.0f, 0.0f, 0.0f}, sb[3] = {0.0f, 0.0f, 0.0f};
-    float axx = 0.0f, axy = 0.0f, axz = 0.0f;
     FitParams fp{0.0f, 0.0f, 0.0f, 0u};
     for (;;) {
         // ---- ordering phase
@@ -413,26 +413,23 @@ __global__ __launch_bounds__(64 * kSearchWaves) __attribute__((amdgpu_waves_per_
                     if (p >= total) {
                         idle = true;
                     } else {
-                        r = list[p];
+                        const uint32_t r = list[p];
                         const ClusterRec& R = recs[r];
                         L.pts[l] = R.pts[l];
                         info = R.info;
-                        ro = RecOut{R.tex, R.block, R.alpha[0], R.alpha[1]};
-                        n = (int)(info & 31u);
-                        iters = (int)((info >> 16) & 15u);
                         const uint32_t byte = (R.remap[l >> 2] >> (8 * (l & 3))) & 255u;
                         remap = byte == 255u ? -1 : (int)byte;
                         fp = FitParams{R.w[0], R.w[1], R.w[2], 0u};
-                        axx = R.axis[0];
-                        axy = R.axis[1];
-                        axz = R.axis[2];
                         thr = NC == 4 ? R.fit3_err : FLT_MAX;
                         lb_err = thr;
-                        lb_code = 0;
                         lb_it = 0;
                         it = 0;
-                        sa[0] = sa[1] = sa[2] = 0.0f;
-                        sb[0] = sb[1] = sb[2] = 0.0f;
+                        if (l == 0) {
+                            uint4* const keep = reinterpret_cast<uint4*>(L.keep);
+                            keep[0] = make_uint4(R.tex, R.block, R.alpha[0], R.alpha[1]);
+                            keep[1] = make_uint4(r, __float_as_uint(R.axis[0]), __float_as_uint(R.axis[1]),
+                                                 __float_as_uint(R.axis[2]));
+                        }
                         need = false;
                     }
                 }
@@ -440,12 +437,16 @@ __global__ __launch_bounds__(64 * kSearchWaves) __attribute__((amdgpu_waves_per_
             }
             const bool todo = !idle && !ready;
             if (!wave_any(todo)) break;
+            const int n = (int)(info & 31u);
+            float axx = __uint_as_float(L.keep[kKeepAxis]), axy = __uint_as_float(L.keep[kKeepAxis + 1]),
+                  axz = __uint_as_float(L.keep[kKeepAxis + 2]);
+            if (it > 0) ends_axis(L.keep[kKeepEnds], L.keep[kKeepEnds + 1], axx, axy, axz);
             const bool unique = ordering_step(L, l, n, todo, it, axx, axy, axz);
             ready = ready || unique;
             const bool repeated = todo && !unique;
             if (wave_any(repeated)) {
                 if (repeated) {
-                    emit_block<NC>(tex, tex0, recs[r], ro, info, L, l, n, remap, lb_err, thr, lb_code, lb_it, sa, sb);
+                    emit_block<NC>(tex, tex0, recs, info, L, l, n, remap, lb_err, thr, lb_it);
                     need = true;
                 }
             }
@@ -454,28 +455,30 @@ __global__ __launch_bounds__(64 * kSearchWaves) __attribute__((amdgpu_waves_per_
         // ---- search phase
         float be;
         uint32_t bc;
+        const int n = (int)(info & 31u);
         search_step<NC>(L, l, n, ready, fp, be, bc);
         bool fin = false;
         if (ready) {
             ready = false;
-            if (be < lb_err) {
+            const bool better = be < lb_err;
+            uint32_t sa = 0, sb = 0;  // best_start = best_end = 0 until a split beats the threshold
+            if (better) {
                 lb_err = be;
-                lb_code = bc;
                 lb_it = it;
-                split_endpoints<NC>(L, n, bc, fp, sa, sb);
+                split_endpoints<NC>(L, n, bc, sa, sb);
             }
-            if (lb_it != it || it + 1 >= iters) {
-                fin = true;
-            } else {
-                axx = sb[0] - sa[0];
-                axy = sb[1] - sa[1];
-                axz = sb[2] - sa[2];
-                ++it;
+            if ((better || it == 0) && l == 0) {
+                L.keep[kKeepEnds] = sa;
+                L.keep[kKeepEnds + 1] = sb;
+                L.keep[kKeepKey] = bc;
             }
+            fin = lb_it != it || it + 1 >= (int)((info >> 16) & 15u);
+            if (!fin) ++it;
         }
+        group_sync();
         if (wave_any(fin)) {
             if (fin) {
-                emit_block<NC>(tex, tex0, recs[r], ro, info, L, l, n, remap, lb_err, thr, lb_code, lb_it, sa, sb);
+                emit_block<NC>(tex, tex0, recs, info, L, l, n, remap, lb_err, thr, lb_it);
                 need = true;
             }
         }
@@ -526,14 +529,12 @@ __global__ __launch_bounds__(64 * kSearchWaves) __attribute__((amdgpu_waves_per_
         ColourSet cs{0, -1, false};
         FitParams fp{0.0f, 0.0f, 0.0f, 0u};
         float axx = 0.0f, axy = 0.0f, axz = 0.0f;
-        uint32_t tex_idx = 0, block = 0, fmt = BC1, alo = 0, ahi = 0;
+        uint32_t fmt = BC1;
         if (has) {
             const ClusterRec& R = recs[list[p]];
             L.pts[l] = R.pts[l];
             const uint32_t info = R.info;
             fmt = (info >> 12) & 15u;
-            alo = R.alpha[0];
-            ahi = R.alpha[1];
             cs.n = (int)(info & 31u);
             cs.transparent = ((info >> 8) & 1u) != 0u;
             const uint32_t byte = (R.remap[l >> 2] >> (8 * (l & 3))) & 255u;
@@ -542,8 +543,7 @@ __global__ __launch_bounds__(64 * kSearchWaves) __attribute__((amdgpu_waves_per_
             axx = R.axis[0];
             axy = R.axis[1];
             axz = R.axis[2];
-            tex_idx = R.tex;
-            block = R.block;
+            if (l == 0) *reinterpret_cast<uint4*>(L.keep) = make_uint4(R.tex, R.block, R.alpha[0], R.alpha[1]);
         }
         group_sync();
         float best = FLT_MAX;
@@ -552,11 +552,12 @@ __global__ __launch_bounds__(64 * kSearchWaves) __attribute__((amdgpu_waves_per_
         run_cluster<4, 1>(L, cs, l, has && !(fmt == BC1 && cs.transparent), axx, axy, axz, fp, best, lo, hi,
                           has && fmt == BC1);
         if (has && l == 0) {
-            const BatchTex& T = tex_at(tex, tex0, tex_idx);
+            const uint4 keep = *reinterpret_cast<const uint4*>(L.keep);  // texture, block, alpha half
+            uint8_t* const out = tex_at(tex, tex0, keep.x).out;
             if (fmt == BC1)
-                *reinterpret_cast<uint2*>(T.out + (size_t)block * 8u) = make_uint2(lo, hi);
+                *reinterpret_cast<uint2*>(out + (size_t)keep.y * 8u) = make_uint2(lo, hi);
             else
-                *reinterpret_cast<uint4*>(T.out + (size_t)block * 16u) = make_uint4(alo, ahi, lo, hi);
+                *reinterpret_cast<uint4*>(out + (size_t)keep.y * 16u) = make_uint4(keep.z, keep.w, lo, hi);
         }
     }
 }

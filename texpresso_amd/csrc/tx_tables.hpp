@@ -15,17 +15,20 @@
 // 2. ClusterFit candidate lists (the split loops of
 //    lib/src/colourfit/cluster.rs:182-236 and 309-380).  compress4 searches
 //    the splits (i, j, k) with 0 <= i < n, i <= j <= n, max(j,1) <= k <= n;
-//    compress3 the splits (i, j) with 0 <= i < n, max(i,1) <= j <= n.  A
-//    split belongs to the search for n distinct colours iff
-//    max(i+1, last index) <= n, so listing the n = 16 splits sorted by that
-//    bound (stable in loop order) makes the list for every n a prefix of
-//    length len[n].  Each entry packs the prefix-table offsets the split
-//    reads and its rank in the reference's loop order, which breaks error
-//    ties exactly like the reference's "first strict minimum wins":
-//      bits  0..7   soff(i, j)  (compress3: part1 offset; compress4: part1)
-//      bits  8..15  soff(j, k)  (compress4 only: part2 offset)
-//      bits 16..19  i           (part0 = S[0][i] lives at offset i)
-//      bits 20..29  loop-order rank
+//    compress3 the splits (i, j) with 0 <= i < n, max(i,1) <= j <= n.
+//    A split's key, i << 26 | j << 21 | k << 16 (k = 0 for compress3), orders
+//    splits as the reference's loops visit them, so the smallest (error, key)
+//    is the reference's first strict minimum.
+//
+//    For one j the splits form a rectangle of i and k values.  The list for n
+//    cuts it into tiles of 2 x 2 splits (i, i+1) x (k, k+1), which share what
+//    depends on (i, j) or on (j, k) alone, and single splits for the odd row
+//    and column.  Both lists are in key order (of a tile's first split).  An
+//    entry holds the byte offsets of the prefix-table rows it reads in 16-bit
+//    halves:
+//      tile:   {soff(i,j) | soff(i+1,j) << 16, soff(j,k) | soff(j,k+1) << 16, key | 16 i}
+//      single: {soff(i,j) | soff(j,k) << 16, key | 16 i}
+//    (part0 = S[0][i] lives at entry i, and S[0][i+1] right after it).
 //    The prefix table S[a][b], a <= b <= 16, is stored compactly: every
 //    empty range S[a][a] (all zero) shares offset 0, row 0 (S[0][b], b >= 1)
 //    sits at offsets 1..16 so that part0 = S[0][i] is at offset i, and rows
@@ -42,22 +45,80 @@ constexpr int soff(int a, int b)
 constexpr int kSEntries = 137;  // soff(15, 16) + 1
 constexpr int kCand4 = 967;       // compress4 splits for 16 colours
 constexpr int kCand3 = 151;       // compress3 splits for 16 colours
-// Stored lengths: the candidate loop reads up to 48 entries past its last
-// 32-candidate trip, so the lists are padded (code 0 = prefix entries S[0],
-// unit entries zero) and every read is in bounds without a guard.
-constexpr int kCand4Stored = 1024;
-constexpr int kCand3Stored = 192;
+
+constexpr uint32_t split_key(int i, int j, int k)
+{
+    return ((uint32_t)i << 26) | ((uint32_t)j << 21) | ((uint32_t)k << 16);
+}
+constexpr int key_i(uint32_t key) { return (int)(key >> 26); }
+constexpr int key_j(uint32_t key) { return (int)((key >> 21) & 31u); }
+constexpr int key_k(uint32_t key) { return (int)((key >> 16) & 31u); }
+constexpr uint32_t kKeyNextI = 1u << 26;  // from (i, j, k) to (i + 1, j, k)
+constexpr uint32_t kKeyNextK = 1u << 16;  // from (i, j, k) to (i, j, k + 1)
 
 struct SingleLut {
     uint8_t v[4][256][6];  // [5_3, 6_3, 5_4, 6_4][value][start0,end0,err0,start1,end1,err1]
 };
 
+struct SplitTile {
+    uint32_t o1, o2, key;
+};
+struct SplitOne {
+    uint32_t o, key;
+};
+struct SplitList {
+    uint16_t start, len;  // entries [start, start + len)
+};
+struct SplitLists {
+    SplitList tiles, ones;
+};
+
+// Rows (i) and columns (k) of the rectangle of splits with this j.
+constexpr int rect_rows(int n, int j) { return (j < n - 1 ? j : n - 1) + 1; }
+constexpr int rect_col0(int j) { return j > 1 ? j : 1; }
+constexpr int rect_cols(int n, int j) { return n - rect_col0(j) + 1; }
+
+// Tiles of the n-colour list: as many as fill whole trips of a group's 16
+// lanes (the rest of the rectangle stays single splits), and none below
+// kTileMinColours, where the tiles' own loop costs what they save (per lane:
+// 10 colours 3 tiles and 6 single splits, 9 colours 2 and 6 against 14).
+constexpr int kTileMinColours = 10;
+
+constexpr int tiles_for(int n)
+{
+    int c = 0;
+    if (n >= kTileMinColours)
+        for (int j = 0; j <= n; ++j) c += (rect_rows(n, j) / 2) * (rect_cols(n, j) / 2);
+    return c & ~15;
+}
+constexpr int splits4_for(int n)
+{
+    int c = 0;
+    for (int j = 0; n > 0 && j <= n; ++j) c += rect_rows(n, j) * rect_cols(n, j);
+    return c;
+}
+constexpr int splits3_for(int n)
+{
+    int c = 0;
+    for (int i = 0; i < n; ++i) c += n - rect_col0(i) + 1;
+    return c;
+}
+constexpr int ones_for(int n) { return splits4_for(n) - 4 * tiles_for(n); }
+template <class F>
+constexpr int sum_to_16(F f)
+{
+    int c = 0;
+    for (int n = 0; n <= 16; ++n) c += f(n);
+    return c;
+}
+constexpr int kTiles = sum_to_16(tiles_for), kOnes4 = sum_to_16(ones_for), kOnes3 = sum_to_16(splits3_for);
+constexpr int kTiles16 = tiles_for(16), kOnes16 = ones_for(16);
+
 struct CandTables {
-    uint32_t t4[kCand4Stored];
-    uint32_t t3[kCand3Stored];
-    uint16_t len4[17];
-    uint16_t len3[17];
-    uint8_t off_b[kSEntries + 3];  // b of the entry at each offset (0 for the shared zero)
+    SplitTile tile[kTiles];
+    SplitOne one4[kOnes4];
+    SplitOne one3[kOnes3];
+    SplitLists lists4[17], lists3[17];  // by colour count
 };
 
 constexpr void build_lut_one(int bits, int colours, uint8_t (&out)[256][6])
@@ -122,57 +183,91 @@ constexpr SingleLut make_single_lut()
     return L;
 }
 
+// The tiles of the n-colour list, numbered in key order of their first splits:
+// `of` is the number of the tile that split (i, j, k) lies in, kTiles if none.
+struct TileMap {
+    uint16_t no[8][17][9] = {};
+    int n = 0;
+
+    constexpr explicit TileMap(int colours) : n(colours)
+    {
+        int c = 0;
+        for (int i = 0; i < n; i += 2)
+            for (int j = i; j <= n; ++j)
+                for (int k = rect_col0(j); k <= n; k += 2) {
+                    const bool whole = i + 1 < rect_rows(n, j) && k + 1 <= n;
+                    no[i / 2][j][(k - rect_col0(j)) / 2] = (uint16_t)(whole && c < tiles_for(n) ? c++ : kTiles);
+                }
+    }
+    constexpr int of(int i, int j, int k) const { return no[i / 2][j][(k - rect_col0(j)) / 2]; }
+};
+
 constexpr CandTables make_cand_tables()
 {
     CandTables T{};
-    // compress4: enumerate in loop order, then bucket by the bound m
-    {
-        uint32_t lex[kCand4] = {};
-        int bound[kCand4] = {};
-        int c = 0;
-        for (int i = 0; i < 16; ++i)
-            for (int j = i; j <= 16; ++j)
-                for (int k = (j > 1 ? j : 1); k <= 16; ++k) {
-                    lex[c] = (uint32_t)soff(i, j) | ((uint32_t)soff(j, k) << 8) | ((uint32_t)i << 16) |
-                             ((uint32_t)c << 20);
-                    bound[c] = (i + 1 > k) ? i + 1 : k;
-                    ++c;
+    int nt = 0, n4 = 0, n3 = 0;
+    for (int n = 0; n <= 16; ++n) {
+        const TileMap map(n);
+        T.lists4[n].tiles.start = (uint16_t)nt;
+        T.lists4[n].ones.start = (uint16_t)n4;
+        T.lists3[n].ones.start = (uint16_t)n3;
+        for (int i = 0; i < n; ++i)
+            for (int j = i; j <= n; ++j) {
+                const uint32_t io = 16u * (uint32_t)i, o1 = 16u * (uint32_t)soff(i, j);
+                for (int k = rect_col0(j); k <= n; ++k) {
+                    const uint32_t o2 = 16u * (uint32_t)soff(j, k);
+                    const bool tiled = map.of(i, j, k) < kTiles;
+                    if (tiled && i % 2 == 0 && (k - rect_col0(j)) % 2 == 0)
+                        T.tile[nt++] = SplitTile{o1 | (16u * (uint32_t)soff(i + 1, j)) << 16,
+                                                 o2 | (16u * (uint32_t)soff(j, k + 1)) << 16, split_key(i, j, k) | io};
+                    else if (!tiled)
+                        T.one4[n4++] = SplitOne{o1 | o2 << 16, split_key(i, j, k) | io};
                 }
-        int pos = 0;
-        for (int m = 0; m <= 16; ++m) {
-            for (int e = 0; e < kCand4; ++e)
-                if (bound[e] == m) T.t4[pos++] = lex[e];
-            T.len4[m] = (uint16_t)pos;
-        }
-    }
-    {
-        uint32_t lex[kCand3] = {};
-        int bound[kCand3] = {};
-        int c = 0;
-        for (int i = 0; i < 16; ++i)
-            for (int j = (i > 1 ? i : 1); j <= 16; ++j) {
-                lex[c] = (uint32_t)soff(i, j) | ((uint32_t)i << 16) | ((uint32_t)c << 20);
-                bound[c] = (i + 1 > j) ? i + 1 : j;
-                ++c;
+                if (j >= 1) T.one3[n3++] = SplitOne{o1, split_key(i, j, 0) | io};
             }
-        int pos = 0;
-        for (int m = 0; m <= 16; ++m) {
-            for (int e = 0; e < kCand3; ++e)
-                if (bound[e] == m) T.t3[pos++] = lex[e];
-            T.len3[m] = (uint16_t)pos;
-        }
+        T.lists4[n].tiles.len = (uint16_t)(nt - T.lists4[n].tiles.start);
+        T.lists4[n].ones.len = (uint16_t)(n4 - T.lists4[n].ones.start);
+        T.lists3[n].ones.len = (uint16_t)(n3 - T.lists3[n].ones.start);
     }
-    for (int a = 0; a <= 16; ++a)
-        for (int b = a + 1; b <= 16; ++b) T.off_b[soff(a, b)] = (uint8_t)b;
     return T;
 }
 
-// j (or k) of a packed candidate from the offset of S[i][j] (S[j][k]): an
-// empty range (offset 0) ends where it starts.
-constexpr int split_end(const CandTables& T, uint32_t off, int start)
+// Whether the lists of n colours hold every split exactly once, in key order.
+constexpr bool lists_cover(const CandTables& T, int n)
 {
-    return off == 0 ? start : (int)T.off_b[off];
+    bool seen[16][17][17] = {};
+    int count = 0;
+    bool ok = true;
+    uint32_t last = 0;
+    auto see = [&](uint32_t key, int di, int dk) {
+        bool& s = seen[key_i(key) + di][key_j(key)][key_k(key) + dk];
+        ok = ok && !s && key_i(key) + di <= key_j(key) && key_j(key) <= key_k(key) && key_k(key) + dk <= n;
+        s = true;
+        ++count;
+    };
+    for (int e = 0; e < T.lists4[n].tiles.len; ++e) {
+        const uint32_t key = T.tile[T.lists4[n].tiles.start + e].key;
+        for (int p = 0; p < 4; ++p) see(key, p / 2, p % 2);
+        ok = ok && key >= last;
+        last = key;
+    }
+    last = 0;
+    for (int e = 0; e < T.lists4[n].ones.len; ++e) {
+        const uint32_t key = T.one4[T.lists4[n].ones.start + e].key;
+        see(key, 0, 0);
+        ok = ok && key > last;
+        last = key;
+    }
+    return ok && count == splits4_for(n);
 }
+constexpr bool all_lists_cover()
+{
+    const CandTables T = make_cand_tables();
+    bool ok = true;
+    for (int n = 0; n <= 16; ++n) ok = ok && lists_cover(T, n);
+    return ok;
+}
+static_assert(all_lists_cover(), "each list holds its splits once, in key order");
 
 // 3. Unit-weight split constants.  When a block has 16 distinct colours and
 //    every point weight is exactly 1 (no duplicates, no alpha weighting),
@@ -182,16 +277,18 @@ constexpr int split_end(const CandTables& T, uint32_t off, int start)
 //    cluster.rs:193-202 / 325-335 are then the same numbers for every such
 //    block.  They are evaluated here with the kernel's own expressions
 //    (constant evaluation is IEEE binary32 with round-to-nearest-even and no
-//    contraction, like the device code), one entry per candidate in the
-//    order of CandTables, so the device reads bit-identical values instead
-//    of recomputing them.
+//    contraction, like the device code), one entry per split of the
+//    16-colour lists of CandTables in their order (tiles: one array per
+//    split of the tile, row (i, k), (i, k+1), (i+1, k), (i+1, k+1)), so the
+//    device reads bit-identical values instead of recomputing them.
 struct UnitSplit {
     float a2, b2, ab, factor;
 };
 
 struct UnitTables {
-    UnitSplit u4[kCand4Stored];
-    UnitSplit u3[kCand3Stored];
+    UnitSplit tile[4][kTiles16];
+    UnitSplit one4[kOnes16];
+    UnitSplit one3[kCand3];
 };
 
 constexpr UnitSplit unit_split4(int i, int j, int k)
@@ -214,28 +311,27 @@ constexpr UnitSplit unit_split3(int i, int j)
     return UnitSplit{a2, b2, ab, 1.0f / ((a2 * b2) - ab * ab)};
 }
 
-// (i, j, k) of a packed candidate: i from bits 16..19, j and k from the
-// prefix-table offsets soff(i, j) and soff(j, k).
-
 constexpr UnitTables make_unit_tables()
 {
     const CandTables C = make_cand_tables();
     UnitTables U{};
-    for (int e = 0; e < kCand4; ++e) {
-        const uint32_t code = C.t4[e];
-        const int i = (int)((code >> 16) & 15u);
-        const int j = split_end(C, code & 255u, i);
-        const int k = split_end(C, (code >> 8) & 255u, j);
-        U.u4[e] = unit_split4(i, j, k);
+    for (int e = 0; e < kTiles16; ++e) {
+        const uint32_t key = C.tile[C.lists4[16].tiles.start + e].key;
+        for (int p = 0; p < 4; ++p) U.tile[p][e] = unit_split4(key_i(key) + p / 2, key_j(key), key_k(key) + p % 2);
+    }
+    for (int e = 0; e < kOnes16; ++e) {
+        const uint32_t key = C.one4[C.lists4[16].ones.start + e].key;
+        U.one4[e] = unit_split4(key_i(key), key_j(key), key_k(key));
     }
     for (int e = 0; e < kCand3; ++e) {
-        const uint32_t code = C.t3[e];
-        const int i = (int)((code >> 16) & 15u);
-        U.u3[e] = unit_split3(i, split_end(C, code & 255u, i));
+        const uint32_t key = C.one3[C.lists3[16].ones.start + e].key;
+        U.one3[e] = unit_split3(key_i(key), key_j(key));
     }
     return U;
 }
 
+static_assert(splits4_for(16) == kCand4 && splits3_for(16) == kCand3 && kTiles16 == 192 && kOnes16 == 199,
+              "split counts of 16 colours");
 static_assert(soff(0, 16) == 16 && soff(1, 2) == 17 && soff(15, 16) == kSEntries - 1, "compact prefix table");
 
 }  // namespace txt
