@@ -387,6 +387,17 @@ __device__ __forceinline__ void single_fit(const LDS& L, const ColourSet& cs, in
     }
 }
 
+// 1.0f / x, correctly rounded, for |x| in [2^-126, 2^126), zeros, infinities
+// and NaN (compared with the division for every binary32 x on the device: it
+// differs only for subnormal x and where 1/x is subnormal): the hardware's
+// reciprocal, one Newton step, and the fix-up of the special cases -- 4
+// instructions, where the division takes 11 to cover every quotient.
+__device__ __forceinline__ float recip(float x)
+{
+    const float r = __builtin_amdgcn_rcpf(x);
+    return __builtin_amdgcn_div_fixupf(__builtin_fmaf(r, __builtin_fmaf(-x, r, 1.0f), r), x, 1.0f);
+}
+
 // A constant kept in a vector register.  As an operand of a VOP3 form (which
 // takes no literal) the compiler would put it in a scalar register, and a
 // scalar operand halves the issue rate of FP32 instructions (v_fma_f32 with
@@ -610,7 +621,9 @@ __device__ __forceinline__ SplitTerms split_terms4(const SplitRow& r, const Spli
         t.u.a2 = c.m.w + r.f.w;
         t.u.b2 = r.m.w + __builtin_fmaf(4.0f, c.m.w, p3w);
         t.u.ab = (2.0f / 9.0f) * (r.p1.w + c.p.w);
-        t.u.factor = 1.0f / ((t.u.a2 * t.u.b2) - t.u.ab * t.u.ab);
+        // point weights lie in [1/16, 4], so the products are 0 or at least
+        // 2^-20 and their difference 0 or at least 2^-44: recip() is exact
+        t.u.factor = recip((t.u.a2 * t.u.b2) - t.u.ab * t.u.ab);
     }
     return t;
 }
@@ -641,7 +654,7 @@ __device__ __forceinline__ SplitTerms split_terms3(const float4& p0, const float
         t.u.a2 = hw + p0.w;
         t.u.b2 = hw + p2w;
         t.u.ab = hw;
-        t.u.factor = 1.0f / ((t.u.a2 * t.u.b2) - t.u.ab * t.u.ab);
+        t.u.factor = recip((t.u.a2 * t.u.b2) - t.u.ab * t.u.ab);  // as for 4 colours
     }
     return t;
 }
