@@ -92,7 +92,7 @@ hipError_t reset_counters(uint32_t* d_counter, hipStream_t s);
 // images grid-stride.
 constexpr uint64_t kGroupsPerRow = 1ull << 16;
 constexpr uint64_t kMaxGroups2d = kGroupsPerRow * 65535ull;
-constexpr uint64_t kMaxDecodeTilesX = 1ull << 16;   // 64 x 4 pixel tiles per grid row
+constexpr uint64_t kMaxDecodeTilesX = 1ull << 16;  // 256-block tiles of the decoder per grid row
 constexpr uint64_t kMaxDecodeTilesY = 1ull << 14;
 
 inline uint32_t capped_grid(uint64_t groups, uint64_t cap) { return (uint32_t)(groups < cap ? groups : cap); }
