@@ -110,8 +110,10 @@ hipError_t launch_decode(int format, const uint8_t* data, uint32_t w, uint32_t h
 // 256 + 17 + 4096 floats; the three per-value outputs hold n entries each.
 hipError_t launch_elementary(const float* d_in, uint32_t n, float* d_tables, float* d_snap31, float* d_snap63,
                              int32_t* d_round255, hipStream_t s);
-// One mip step of the RGBA8 image src (w x h, 4-byte aligned) into dst
-// (max(1, w/2) x max(1, h/2)): 2x2 box, edge clamp, (sum + 2) >> 2.
-hipError_t launch_mip_down(const uint8_t* src, uint32_t w, uint32_t h, uint8_t* dst, hipStream_t s);
+// Levels 1..nout (1 <= nout <= kMipLevelsPerLaunch) of the RGBA8 image src
+// (w x h, 4-byte aligned) back to back into dst: 2x2 box of the level above,
+// edge clamp, (sum + 2) >> 2; level k is max(1, w >> k) x max(1, h >> k).
+constexpr uint32_t kMipLevelsPerLaunch = 6;
+hipError_t launch_mip_levels(const uint8_t* src, uint32_t w, uint32_t h, uint32_t nout, uint8_t* dst, hipStream_t s);
 
 }  // namespace txk

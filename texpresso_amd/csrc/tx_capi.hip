@@ -369,19 +369,22 @@ static int check_mips(size_t width, size_t height, uint32_t levels, size_t chain
     return TX_OK;
 }
 
-// Levels 1..levels-1 into d_chain, each from the previous one.
+// Levels 1..levels-1 into d_chain, kMipLevelsPerLaunch at a time.
 static hipError_t mips_on(const uint8_t* d_rgba, size_t width, size_t height, uint32_t levels, uint8_t* d_chain,
                           hipStream_t s)
 {
     const uint8_t* src = d_rgba;
-    size_t off = 0;
-    for (uint32_t k = 1; k < levels; ++k) {
-        uint8_t* dst = d_chain + off;
-        const hipError_t e = txk::launch_mip_down(src, (uint32_t)mip_side(width, k - 1),
-                                                  (uint32_t)mip_side(height, k - 1), dst, s);
+    uint8_t* dst = d_chain;
+    for (uint32_t k = 0; k + 1 < levels;) {
+        const uint32_t n = std::min(levels - 1 - k, txk::kMipLevelsPerLaunch);
+        const hipError_t e =
+            txk::launch_mip_levels(src, (uint32_t)mip_side(width, k), (uint32_t)mip_side(height, k), n, dst, s);
         if (e != hipSuccess) return e;
-        src = dst;
-        off += 4 * mip_side(width, k) * mip_side(height, k);
+        for (uint32_t m = 0; m < n; ++m) {  // dst ends up past the last of these levels, src on it
+            ++k;
+            src = dst;
+            dst += 4 * mip_side(width, k) * mip_side(height, k);
+        }
     }
     return hipSuccess;
 }
