@@ -148,6 +148,22 @@ __device__ __forceinline__ void grp_argmin(float& e, uint32_t& c)
     argmin_step<1>(e, c);
 }
 
+// The same over the T groups of a team, each with its own result on all of
+// its lanes.
+template <int T>
+__device__ __forceinline__ void team_argmin(float& e, uint32_t& c)
+{
+#pragma unroll
+    for (int d = 16; d < 16 * T; d *= 2) {
+        const int from = 4 * (int)(__lane_id() ^ (uint32_t)d);
+        const float e2 = __int_as_float(__builtin_amdgcn_ds_bpermute(from, __float_as_int(e)));
+        const uint32_t c2 = (uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)c);
+        const bool take = (e2 < e) | ((e2 == e) & (c2 < c));
+        e = take ? e2 : e;
+        c = take ? c2 : c;
+    }
+}
+
 __device__ __forceinline__ bool wave_any(bool p) { return __ballot(p) != 0; }
 
 // math.rs:100-102: roundf(a).max(0).min(limit) as i32, NaN -> 0
@@ -854,14 +870,15 @@ struct BestSplit {
 };
 
 // The single splits of a list (all of a 3-colour search, the odd rows and
-// columns of a 4-colour one).  Trip q covers entries 32q .. 32q + 31: lane l
-// evaluates entry 32q + l (A) and 32q + 16 + l (B), each while 32q is below
-// its limit, so a lane meets its entries in key order.  Loop control and the
+// columns of a 4-colour one).  T groups share the list: with t = 16 (g mod T) +
+// l the lane's place among their lanes, trip q covers entries 32Tq .. 32Tq +
+// 32T - 1 and the lane evaluates entry 32Tq + t (A) and 32Tq + 16T + t (B),
+// each while 32Tq is below its limit, so a lane meets its entries in key order.  Loop control and the
 // trip's offsets are scalar: the list is read through a buffer resource with
 // the lane's offset in a vector register and the trip's in a scalar one.
 // Entries are read two half-trips ahead and prefix sums one half-trip ahead.
-template <int NC, bool UNIT>
-__device__ __forceinline__ void search_ones(const GroupLds& L, int l, const txt::SplitList& list, uint32_t wlen,
+template <int NC, bool UNIT, int T>
+__device__ __forceinline__ void search_ones(const GroupLds& L, uint32_t t, const txt::SplitList& list, uint32_t wlen,
                                             const float4& xs, const FitParams& fp, const SnapGrids& sg,
                                             BestSplit& best)
 {
@@ -870,31 +887,31 @@ __device__ __forceinline__ void search_ones(const GroupLds& L, int l, const txt:
     const __amdgpu_buffer_rsrc_t ru = NC == 4 ? table_rsrc(c_unit.one4, sizeof c_unit.one4)
                                               : table_rsrc(c_unit.one3, sizeof c_unit.one3);
     const uint32_t mylen = list.len;
-    const uint32_t vo = 8u * ((uint32_t)list.start + (uint32_t)l), uo = 16u * (uint32_t)l;
+    const uint32_t vo = 8u * ((uint32_t)list.start + t), uo = 16u * t;
     auto one_at = [&](uint32_t so) {
         const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(rt, vo, so, 0);
         return txt::SplitOne{v[0], v[1]};
     };
-    const uint32_t limA = mylen > (uint32_t)l ? mylen - (uint32_t)l : 0u;
-    const uint32_t limB = mylen > (uint32_t)l + 16u ? mylen - (uint32_t)l - 16u : 0u;
+    const uint32_t limA = mylen > t ? mylen - t : 0u;
+    const uint32_t limB = mylen > t + 16u * T ? mylen - t - 16u * T : 0u;
     BestSplit mine;
     txt::SplitOne cA = one_at(0);
-    txt::SplitOne cB = one_at(128);
+    txt::SplitOne cB = one_at(128 * T);
     SplitSums sA = load_split<NC>(L, cA);
     txt::UnitSplit uA{};
     if (UNIT) uA = unit_at(ru, uo, 0);
-    for (uint32_t base = 0; base < wlen; base += 32) {
+    for (uint32_t base = 0; base < wlen; base += 32 * T) {
         const uint32_t so = 8u * base, su = 16u * base;
-        const txt::SplitOne cA2 = one_at(so + 256);
+        const txt::SplitOne cA2 = one_at(so + 256 * T);
         const SplitSums sB = load_split<NC>(L, cB);
         txt::UnitSplit uB{};
-        if (UNIT) uB = unit_at(ru, uo, su + 256);
+        if (UNIT) uB = unit_at(ru, uo, su + 256 * T);
         if (base < limA) {
             mine.see(split_error(split_terms<NC, UNIT>(sA, xs, uA), fp, sg), cA.key);
         }
-        const txt::SplitOne cB2 = one_at(so + 384);
+        const txt::SplitOne cB2 = one_at(so + 384 * T);
         sA = load_split<NC>(L, cA2);
-        if (UNIT) uA = unit_at(ru, uo, su + 512);
+        if (UNIT) uA = unit_at(ru, uo, su + 512 * T);
         if (base < limB) {
             mine.see(split_error(split_terms<NC, UNIT>(sB, xs, uB), fp, sg), cB.key);
         }
@@ -904,7 +921,8 @@ __device__ __forceinline__ void search_ones(const GroupLds& L, int l, const txt:
     best.merge(mine.e, mine.c);
 }
 
-// The 2 x 2 tiles of a 4-colour list, one tile per lane and trip.  The loop is
+// The 2 x 2 tiles of a 4-colour list, one tile per lane and trip (`t` and T as
+// for search_ones).  The loop is
 // bound by VALU issue; a tile computes what depends on (j, k) alone and on
 // (i, j) alone once for two splits each, decodes one list entry for four and
 // needs no tie compare (each row is met in key order), which takes a split
@@ -913,36 +931,36 @@ __device__ __forceinline__ void search_ones(const GroupLds& L, int l, const txt:
 // them the loop waits out four table loads a tile and gains nothing), 2048^2
 // BC3 IterativeClusterFit went from 1011 to 937 us.  Other weights need 26
 // more registers, so there the sums are read at the tile's start.
-template <bool UNIT>
-__device__ __forceinline__ void search_tiles(const GroupLds& L, int l, const txt::SplitList& list, uint32_t wlen,
+template <bool UNIT, int T>
+__device__ __forceinline__ void search_tiles(const GroupLds& L, uint32_t t, const txt::SplitList& list, uint32_t wlen,
                                              const float4& xs, const FitParams& fp, const SnapGrids& sg,
                                              BestSplit& best)
 {
     const __amdgpu_buffer_rsrc_t rt = table_rsrc(c_cand.tile, sizeof c_cand.tile);
     const __amdgpu_buffer_rsrc_t ru = table_rsrc(c_unit.tile, sizeof c_unit.tile);
     constexpr uint32_t kPos = sizeof c_unit.tile[0];  // bytes from one split of the tiles to the next
-    const uint32_t lim = list.len > l ? (uint32_t)list.len - (uint32_t)l : 0u;
-    const uint32_t vo = 12u * ((uint32_t)list.start + (uint32_t)l), uo = 16u * (uint32_t)l;
+    const uint32_t lim = list.len > t ? (uint32_t)list.len - t : 0u;
+    const uint32_t vo = 12u * ((uint32_t)list.start + t), uo = 16u * t;
     auto tile_at = [&](uint32_t so) { return __builtin_amdgcn_raw_buffer_load_b96(rt, vo, so, 0); };
     auto unit = [&](uint32_t so) { return UNIT ? unit_at(ru, uo, so) : txt::UnitSplit{}; };
     auto part0 = [&](uint32_t key, int r) { return sum_at(L.S + r, key & 0xFFFFu); };
     BestSplit rows[2];  // rows i and i + 1 of the tiles, each met in key order
-    u32x3 t = tile_at(0), t2 = tile_at(192);
+    u32x3 code = tile_at(0), code2 = tile_at(192 * T);
     float4 p0, p1, c0, c1;  // the first row's and the columns' sums
     auto load_sums = [&]() {
-        p0 = part0(t[2], 0);
-        p1 = sum_at(L.S, t[0] & 0xFFFFu);
-        c0 = sum_at(L.S, t[1] & 0xFFFFu);
-        c1 = sum_at(L.S, t[1] >> 16);
+        p0 = part0(code[2], 0);
+        p1 = sum_at(L.S, code[0] & 0xFFFFu);
+        c0 = sum_at(L.S, code[1] & 0xFFFFu);
+        c1 = sum_at(L.S, code[1] >> 16);
     };
     if (UNIT) load_sums();
     txt::UnitSplit u0 = unit(0);
-    for (uint32_t base = 0; base < wlen; base += 16) {
+    for (uint32_t base = 0; base < wlen; base += 16 * T) {
         const uint32_t su = 16u * base;
         const bool live = base < lim;
-        const uint32_t key = t[2];
+        const uint32_t key = code[2];
         if (!UNIT) load_sums();
-        const float4 q0 = part0(t[2], 1), q1 = sum_at(L.S, t[0] >> 16);
+        const float4 q0 = part0(code[2], 1), q1 = sum_at(L.S, code[0] >> 16);
         txt::UnitSplit u1 = unit(su + kPos);
         const SplitCol col0 = split_col(c0, xs), col1 = split_col(c1, xs);
         __builtin_amdgcn_sched_barrier(0);
@@ -954,14 +972,14 @@ __device__ __forceinline__ void search_tiles(const GroupLds& L, int l, const txt
             if (live) rows[0].see(split_error(split_terms4<UNIT>(row, col1, u1), fp, sg), key + txt::kKeyNextK);
             u1 = unit(su + 3 * kPos);
         }
-        t = t2;
-        t2 = tile_at(12u * base + 384u);
+        code = code2;
+        code2 = tile_at(12u * base + 384u * T);
         if (UNIT) load_sums();
         __builtin_amdgcn_sched_barrier(0);
         {
             const SplitRow row = split_row(q0, q1);
             if (live) rows[1].see(split_error(split_terms4<UNIT>(row, col0, u0), fp, sg), key);
-            u0 = unit(su + 256);
+            u0 = unit(su + 256 * T);
             __builtin_amdgcn_sched_barrier(0);
             if (live) rows[1].see(split_error(split_terms4<UNIT>(row, col1, u1), fp, sg), key + txt::kKeyNextK);
         }
@@ -972,11 +990,12 @@ __device__ __forceinline__ void search_tiles(const GroupLds& L, int l, const txt
 
 // The split search over the current prefix table: every group with `run`
 // set evaluates its splits and returns the first strict minimum (error, key)
-// on all of its lanes.  Executed by the whole wave.  When every searching
+// on all of its lanes.  With T > 1 the wave's T neighbouring groups hold the
+// same block and share its lists.  Executed by the whole wave.  When every searching
 // group holds 16 points of weight exactly 1, the weight terms come from the
 // unit-weight table (same values, fewer operations).
-template <int NC, bool UNIT>
-__device__ __forceinline__ void search_loop(const GroupLds& L, int l, int n, bool run, const float4& xs,
+template <int NC, bool UNIT, int T>
+__device__ __forceinline__ void search_loop(const GroupLds& L, uint32_t t, int n, bool run, const float4& xs,
                                             const FitParams& fp, float& be, uint32_t& bc)
 {
     // the tile and single lists of n colours, read together
@@ -987,23 +1006,25 @@ __device__ __forceinline__ void search_loop(const GroupLds& L, int l, int n, boo
     };
     const SnapGrids sg = snap_grids();
     BestSplit best;
-    if (NC == 4) search_tiles<UNIT>(L, l, lists.tiles, longest(lists.tiles.len), xs, fp, sg, best);
-    search_ones<NC, UNIT>(L, l, lists.ones, longest(lists.ones.len), xs, fp, sg, best);
+    if (NC == 4) search_tiles<UNIT, T>(L, t, lists.tiles, longest(lists.tiles.len), xs, fp, sg, best);
+    search_ones<NC, UNIT, T>(L, t, lists.ones, longest(lists.ones.len), xs, fp, sg, best);
     be = best.e;
     bc = best.c;
 }
 
-template <int NC>
+template <int NC, int T = 1>
 __device__ __forceinline__ void search_step(const GroupLds& L, int l, int n, bool run, const FitParams& fp,
                                             float& be, uint32_t& bc)
 {
     const float4 xs = L.S[n];  // xsum_wsum = S[0][n]
     const bool unit = n == 16 && grp_min(L.pts[l].w == 1.0f ? 1u : 0u) == 1u;
+    const uint32_t t = T == 1 ? (uint32_t)l : __lane_id() & (16u * T - 1u);
     if (!wave_any(run && !unit))
-        search_loop<NC, true>(L, l, n, run, xs, fp, be, bc);
+        search_loop<NC, true, T>(L, t, n, run, xs, fp, be, bc);
     else
-        search_loop<NC, false>(L, l, n, run, xs, fp, be, bc);
+        search_loop<NC, false, T>(L, t, n, run, xs, fp, be, bc);
     grp_argmin(be, bc);
+    if (T > 1) team_argmin<T>(be, bc);
 }
 
 // txt::soff without branches (row a >= 1 of the table starts at entry
@@ -1060,7 +1081,8 @@ __device__ __forceinline__ uint32_t split_index(const GroupLds& L, int n, int re
 // only): the group's LDS already holds this axis's ordering and prefix
 // table -- compress3 of ClusterFit built them, and its search, endpoints and
 // index assembly only read them -- so compress4 does not build them again.
-template <int NC, int ITERS>
+// T > 1: teams of T groups on the same block (search_step).
+template <int NC, int ITERS, int T = 1>
 __device__ __forceinline__ void run_cluster(GroupLds& L, const ColourSet& cs, int l, bool act, float px, float py,
                                             float pz, const FitParams& fp, float& best_err, uint32_t& lo,
                                             uint32_t& hi, bool table_ready = false)
@@ -1085,7 +1107,7 @@ __device__ __forceinline__ void run_cluster(GroupLds& L, const ColourSet& cs, in
         }
         float be;
         uint32_t bc;
-        search_step<NC>(L, l, n, !done, fp, be, bc);
+        search_step<NC, T>(L, l, n, !done, fp, be, bc);
         // iteration control, cluster.rs:222-249
         if (!done) {
             if (be < lb_err) {
@@ -1416,8 +1438,9 @@ __device__ __forceinline__ int encode_front(uint32_t px, bool valid, const FitPa
 // of the wave must call this (LDS hand-offs inside); groups without a block
 // pass valid = false and discard the result.  Returns the block words in
 // out[0..3] (8-byte formats use out[0..1]).  The four groups of a wave run
-// their ClusterFit searches in lockstep.
-template <int FMT, int ALG>
+// their ClusterFit searches in lockstep; with T > 1, T neighbouring groups
+// pass the same block and share its split searches.
+template <int FMT, int ALG, int T = 1>
 __device__ __forceinline__ void encode_block(uint32_t px, bool valid, const FitParams& fp, GroupLds& L, int g, int l,
                                              uint32_t (&out)[4])
 {
@@ -1435,9 +1458,9 @@ __device__ __forceinline__ void encode_block(uint32_t px, bool valid, const FitP
         if (wave_any(act)) {
             float best_err = FLT_MAX;
             uint32_t clo = 0, chi = 0;
-            if (FMT == BC1) run_cluster<3, ITERS>(L, cs, l, act, vx, vy, vz, fp, best_err, clo, chi);
-            run_cluster<4, ITERS>(L, cs, l, act && !(FMT == BC1 && cs.transparent), vx, vy, vz, fp, best_err, clo,
-                                  chi, FMT == BC1 && act);
+            if (FMT == BC1) run_cluster<3, ITERS, T>(L, cs, l, act, vx, vy, vz, fp, best_err, clo, chi);
+            run_cluster<4, ITERS, T>(L, cs, l, act && !(FMT == BC1 && cs.transparent), vx, vy, vz, fp, best_err, clo,
+                                     chi, FMT == BC1 && act);
             if (act) set_colour<FMT>(out, clo, chi);
         }
     }

@@ -26,8 +26,9 @@ __device__ __forceinline__ void store_block(uint8_t* out, uint64_t b, const uint
 // below 2^32 since y < 2^16 and x <= 2^16).
 __device__ __forceinline__ uint32_t group_index() { return blockIdx.y * gridDim.x + blockIdx.x; }
 
-// Plain per-texture launch: one wave per four consecutive output blocks.
-template <int FMT, int ALG>
+// Plain per-texture launch: one wave per 4 / T consecutive output blocks, each
+// held by T 16-lane groups that share its split searches.
+template <int FMT, int ALG, int T>
 __global__ __launch_bounds__(64) void k_encode(const uint8_t* __restrict__ rgba, uint32_t width, uint32_t height,
                                                uint32_t blocks_wide, uint64_t nblocks, uint8_t* __restrict__ out,
                                                FitParams fp)
@@ -36,15 +37,15 @@ __global__ __launch_bounds__(64) void k_encode(const uint8_t* __restrict__ rgba,
     const int tid = (int)threadIdx.x, g = tid >> 4, l = tid & 15;
     // the last row of a 2-D grid may hold groups past the texture: all their
     // blocks are not live, as in a part-filled last wave
-    const uint64_t b = (uint64_t)group_index() * 4u + (uint64_t)g;
+    const uint64_t b = (uint64_t)group_index() * (4u / T) + (uint64_t)(g / T);
     const bool live = b < nblocks;
     const uint32_t bx = live ? (uint32_t)(b % blocks_wide) : 0u;
     const uint32_t by = live ? (uint32_t)(b / blocks_wide) : 0u;
     bool valid;
     const uint32_t px = fetch_pixel(rgba, width, height, bx, by, live, l, valid);
     uint32_t w[4];
-    encode_block<FMT, ALG>(px, valid, fp, lds[g], g, l, w);
-    if (live && l == 0) store_block<FMT>(out, b, w);
+    encode_block<FMT, ALG, T>(px, valid, fp, lds[g], g, l, w);
+    if (live && l == 0 && g % T == 0) store_block<FMT>(out, b, w);
 }
 
 // BC4 / BC5 per-texture launch: one block per lane (alpha codebooks are
@@ -97,22 +98,23 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
 }
 
 // Explicit block list (Format::compress_block_masked over many blocks): block
-// b's 16 pixels are the 64 bytes at blocks + 64*b, its mask is masks[b].
-template <int FMT, int ALG>
+// b's 16 pixels are the 64 bytes at blocks + 64*b, its mask is masks[b].  T as
+// in k_encode.
+template <int FMT, int ALG, int T>
 __global__ __launch_bounds__(64) void k_encode_blocks(const uint8_t* __restrict__ blocks,
                                                       const uint32_t* __restrict__ masks, uint64_t nblocks,
                                                       uint8_t* __restrict__ out, FitParams fp)
 {
     __shared__ GroupLds lds[4];
     const int tid = (int)threadIdx.x, g = tid >> 4, l = tid & 15;
-    const uint64_t b = (uint64_t)group_index() * 4u + (uint64_t)g;
+    const uint64_t b = (uint64_t)group_index() * (4u / T) + (uint64_t)(g / T);
     const bool live = b < nblocks;
     const uint32_t mask = live ? masks[b] : 0u;
     const bool valid = live && ((mask >> l) & 1u);
     const uint32_t px = valid ? reinterpret_cast<const uint32_t*>(blocks + 64 * b)[l] : 0u;
     uint32_t w[4];
-    encode_block<FMT, ALG>(px, valid, fp, lds[g], g, l, w);
-    if (live && l == 0) store_block<FMT>(out, b, w);
+    encode_block<FMT, ALG, T>(px, valid, fp, lds[g], g, l, w);
+    if (live && l == 0 && g % T == 0) store_block<FMT>(out, b, w);
 }
 
 // ------------------------------------------------------------------ decode
@@ -346,15 +348,44 @@ __global__ __launch_bounds__(64) void k_elementary(const float* __restrict__ in,
 
 namespace {
 
+// Groups per block of the direct kernels.  A split search on 16 lanes takes a
+// wave 17 us (30-100 us for IterativeClusterFit) however few blocks there are;
+// on 32 or 64 lanes it takes half or a quarter, but a wave then holds 2 or 1
+// blocks and repeats what comes before the search.  Measured us for teams of 1
+// / 2 / 4 groups (BC1 ClusterFit): 27.5 / 18.5 / 14.4 at 256 blocks, 28.2 /
+// 23.4 / 20.8 at 2304, 27.9 / 23.4 / 24.8 at 3136, 33.8 / 29.0 / 35.2 at 5184,
+// 34.2 / 33.9 / 40.3 at 6400.  BC1 and BC3 IterativeClusterFit, several
+// searches a block: 120 / 68 / 48 and 99 / 61 / 39 at 256 blocks, 174 / 137 /
+// 130 and 174 / 134 / 116 at 9216, 164 / 140 / 150 and 178 / 147 / 136 at
+// 12544, 190 / 170 / 190 and 197 / 169 / 168 at 16384.
+int team_groups(int algorithm, uint64_t nblocks)
+{
+    if (algorithm == 0) return 1;  // RangeFit: no search
+    const bool iterative = algorithm == 2;
+    if (nblocks <= (iterative ? 10240u : 2560u)) return 4;
+    return nblocks <= (iterative ? 32768u : 6144u) ? 2 : 1;
+}
+
+template <int FMT, int ALG, int T>
+hipError_t launch_encode_n(const txk::EncodeArgs& a, hipStream_t s)
+{
+    if (a.nblocks > 4 * txk::kMaxGroups2d) return hipErrorInvalidValue;
+    const uint64_t groups = (a.nblocks * T + 3) / 4;
+    if (groups == 0) return hipSuccess;
+    hipLaunchKernelGGL((txd::k_encode<FMT, ALG, T>), txk::grid_2d(groups), dim3(64), 0, s, a.rgba, a.width, a.height,
+                       a.blocks_wide, a.nblocks, a.out, txd::FitParams{a.wr, a.wg, a.wb, a.weigh_alpha});
+    return hipGetLastError();
+}
+
 template <int FMT, int ALG>
 hipError_t launch_encode_t(const txk::EncodeArgs& a, hipStream_t s)
 {
-    const uint64_t groups = (a.nblocks + 3) / 4;
-    if (groups == 0) return hipSuccess;
-    if (groups > txk::kMaxGroups2d) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((txd::k_encode<FMT, ALG>), txk::grid_2d(groups), dim3(64), 0, s, a.rgba, a.width, a.height,
-                       a.blocks_wide, a.nblocks, a.out, txd::FitParams{a.wr, a.wg, a.wb, a.weigh_alpha});
-    return hipGetLastError();
+    if constexpr (ALG != 0) {
+        const int t = team_groups(ALG, a.nblocks);
+        if (t == 4) return launch_encode_n<FMT, ALG, 4>(a, s);
+        if (t == 2) return launch_encode_n<FMT, ALG, 2>(a, s);
+    }
+    return launch_encode_n<FMT, ALG, 1>(a, s);
 }
 
 template <int FMT>
@@ -386,15 +417,26 @@ hipError_t launch_encode_f(const txk::EncodeArgs& a, hipStream_t s)
     }
 }
 
+template <int FMT, int ALG, int T>
+hipError_t launch_blocks_n(const txk::BlockListArgs& a, hipStream_t s)
+{
+    if (a.nblocks > 4 * txk::kMaxGroups2d) return hipErrorInvalidValue;
+    const uint64_t groups = (a.nblocks * T + 3) / 4;
+    if (groups == 0) return hipSuccess;
+    hipLaunchKernelGGL((txd::k_encode_blocks<FMT, ALG, T>), txk::grid_2d(groups), dim3(64), 0, s, a.blocks, a.masks,
+                       a.nblocks, a.out, txd::FitParams{a.wr, a.wg, a.wb, a.weigh_alpha});
+    return hipGetLastError();
+}
+
 template <int FMT, int ALG>
 hipError_t launch_blocks_t(const txk::BlockListArgs& a, hipStream_t s)
 {
-    const uint64_t groups = (a.nblocks + 3) / 4;
-    if (groups == 0) return hipSuccess;
-    if (groups > txk::kMaxGroups2d) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((txd::k_encode_blocks<FMT, ALG>), txk::grid_2d(groups), dim3(64), 0, s, a.blocks, a.masks,
-                       a.nblocks, a.out, txd::FitParams{a.wr, a.wg, a.wb, a.weigh_alpha});
-    return hipGetLastError();
+    if constexpr (ALG != 0) {
+        const int t = team_groups(ALG, a.nblocks);
+        if (t == 4) return launch_blocks_n<FMT, ALG, 4>(a, s);
+        if (t == 2) return launch_blocks_n<FMT, ALG, 2>(a, s);
+    }
+    return launch_blocks_n<FMT, ALG, 1>(a, s);
 }
 
 template <int FMT>
