@@ -26,6 +26,7 @@
 #include <float.h>
 #include <stdint.h>
 
+#include "bcn_kernels.hpp"
 #include "tx_tables.hpp"
 
 #pragma clang fp contract(off)
@@ -1358,6 +1359,15 @@ __device__ __forceinline__ void encode_alpha_only(uint32_t px, bool valid, int l
     out[0] = out[1] = out[2] = out[3] = 0;
     bc3_alpha((int)(px & 255u), valid, l, out[0], out[1]);
     if (FMT == BC5) bc3_alpha((int)((px >> 8) & 255u), valid, l, out[2], out[3]);
+}
+
+// The chain level that workgroup (or chunk) `at` belongs to: lane k compares
+// it with the level's first.  Uniform over the wave.
+__device__ __forceinline__ uint32_t chain_level(const txk::ChainTable& chain, uint32_t at)
+{
+    const uint32_t lane = threadIdx.x & 63u;
+    const bool past = lane < chain.count && at >= chain.first[lane];
+    return (uint32_t)__builtin_amdgcn_readfirstlane((int)(__popcll(__ballot(past)) - 1));
 }
 
 // The colour half of a BC1/BC2/BC3 block: words 0-1 for BC1, 2-3 otherwise.

@@ -26,75 +26,137 @@ __device__ __forceinline__ void store_block(uint8_t* out, uint64_t b, const uint
 // below 2^32 since y < 2^16 and x <= 2^16).
 __device__ __forceinline__ uint32_t group_index() { return blockIdx.y * gridDim.x + blockIdx.x; }
 
-// Plain per-texture launch: one wave per 4 / T consecutive output blocks, each
-// held by T 16-lane groups that share its split searches.
-template <int FMT, int ALG, int T>
-__global__ __launch_bounds__(64) void k_encode(const uint8_t* __restrict__ rgba, uint32_t width, uint32_t height,
-                                               uint32_t blocks_wide, uint64_t nblocks, uint8_t* __restrict__ out,
-                                               FitParams fp)
+// One image as the one-pass encoders see it: a texture, or a level of a chain.
+struct Image {
+    const uint8_t* rgba;
+    uint32_t width, height, blocks_wide;
+    uint64_t nblocks;
+    uint8_t* out;
+};
+
+// Level of workgroup `group` and that workgroup's number within the level.
+template <int FMT>
+__device__ __forceinline__ Image chain_image(const txk::ChainTable& chain, uint8_t* out, uint32_t& group)
 {
-    __shared__ GroupLds lds[4];
+    const uint32_t k = chain_level(chain, group);
+    const txk::ChainTable::Level& v = chain.level[k];
+    group -= chain.first[k];
+    constexpr size_t bs = FMT == BC1 || FMT == BC4 ? 8u : 16u;
+    return Image{v.rgba, v.width, v.height, v.blocks_wide, v.nblocks, out + v.block0 * bs};
+}
+
+// One wave per 4 / T consecutive output blocks, each held by T 16-lane groups
+// that share its split searches.
+template <int FMT, int ALG, int T>
+__device__ __forceinline__ void encode_groups(const Image& im, uint32_t group, const FitParams& fp, GroupLds* lds)
+{
     const int tid = (int)threadIdx.x, g = tid >> 4, l = tid & 15;
     // the last row of a 2-D grid may hold groups past the texture: all their
     // blocks are not live, as in a part-filled last wave
-    const uint64_t b = (uint64_t)group_index() * (4u / T) + (uint64_t)(g / T);
-    const bool live = b < nblocks;
-    const uint32_t bx = live ? (uint32_t)(b % blocks_wide) : 0u;
-    const uint32_t by = live ? (uint32_t)(b / blocks_wide) : 0u;
+    const uint64_t b = (uint64_t)group * (4u / T) + (uint64_t)(g / T);
+    const bool live = b < im.nblocks;
+    const uint32_t bx = live ? (uint32_t)(b % im.blocks_wide) : 0u;
+    const uint32_t by = live ? (uint32_t)(b / im.blocks_wide) : 0u;
     bool valid;
-    const uint32_t px = fetch_pixel(rgba, width, height, bx, by, live, l, valid);
+    const uint32_t px = fetch_pixel(im.rgba, im.width, im.height, bx, by, live, l, valid);
     uint32_t w[4];
     encode_block<FMT, ALG, T>(px, valid, fp, lds[g], g, l, w);
-    if (live && l == 0 && g % T == 0) store_block<FMT>(out, b, w);
+    if (live && l == 0 && g % T == 0) store_block<FMT>(im.out, b, w);
 }
 
-// BC4 / BC5 per-texture launch: one block per lane (alpha codebooks are
-// integer work on 16 values; a lane's 16 dword loads keep many bytes in
-// flight, and neighbouring lanes read neighbouring 16-byte row segments).
-template <int FMT>
-__global__ __launch_bounds__(256) void k_encode_alpha(const uint8_t* __restrict__ rgba, uint32_t width,
-                                                      uint32_t height, uint32_t blocks_wide, uint64_t nblocks,
-                                                      uint8_t* __restrict__ out)
+// Plain per-texture launch, and the same over the levels of a chain.
+template <int FMT, int ALG, int T>
+__global__ __launch_bounds__(64) void k_encode(Image im, FitParams fp)
 {
-    const uint64_t b = (uint64_t)group_index() * blockDim.x + threadIdx.x;
-    if (b >= nblocks) return;
+    __shared__ GroupLds lds[4];
+    encode_groups<FMT, ALG, T>(im, group_index(), fp, lds);
+}
+
+template <int FMT, int ALG, int T>
+__global__ __launch_bounds__(64) void k_encode_chain(txk::ChainTable chain, uint8_t* __restrict__ out, FitParams fp)
+{
+    __shared__ GroupLds lds[4];
+    uint32_t group = group_index();
+    const Image im = chain_image<FMT>(chain, out, group);
+    encode_groups<FMT, ALG, T>(im, group, fp, lds);
+}
+
+// BC4 / BC5: one block per lane (alpha codebooks are integer work on 16
+// values; a lane's 16 dword loads keep many bytes in flight, and neighbouring
+// lanes read neighbouring 16-byte row segments).
+template <int FMT>
+__device__ __forceinline__ void encode_alpha_lanes(const Image& im, uint32_t group)
+{
+    const uint64_t b = (uint64_t)group * blockDim.x + threadIdx.x;
+    if (b >= im.nblocks) return;
     uint32_t px[16];
-    const uint32_t valid = fetch_block_lane(rgba, width, height, (uint32_t)(b % blocks_wide),
-                                            (uint32_t)(b / blocks_wide), px);
+    const uint32_t valid = fetch_block_lane(im.rgba, im.width, im.height, (uint32_t)(b % im.blocks_wide),
+                                            (uint32_t)(b / im.blocks_wide), px);
     uint32_t w[4];
     encode_alpha_lane<FMT>(px, valid, w);
-    store_block<FMT>(out, b, w);
+    store_block<FMT>(im.out, b, w);
 }
 
-// RangeFit per-texture launch (BC1/BC2/BC3): one block per lane, the front of
-// the pipeline's classify pass (alpha, colour set, principal axis, then the
-// single-colour or range fit) without its record path.  A RangeFit block is a
-// few hundred serial operations; on a 16-lane group every fold would run on
-// all 16 lanes.  Single-wave workgroups (the per-wave LDS copies of the
-// block pixels and weights), one per 64-block span of the texture.
 template <int FMT>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_encode_range_lane(
-    const uint8_t* __restrict__ rgba, uint32_t width, uint32_t height, uint32_t blocks_wide, uint64_t nblocks,
-    uint8_t* __restrict__ out, FitParams fp)
+__global__ __launch_bounds__(256) void k_encode_alpha(Image im)
 {
-    __shared__ LaneTables LT;
-    __shared__ LaneBlockLds LB;
+    encode_alpha_lanes<FMT>(im, group_index());
+}
+
+template <int FMT>
+__global__ __launch_bounds__(256) void k_encode_alpha_chain(txk::ChainTable chain, uint8_t* __restrict__ out)
+{
+    uint32_t group = group_index();
+    const Image im = chain_image<FMT>(chain, out, group);
+    encode_alpha_lanes<FMT>(im, group);
+}
+
+// RangeFit (BC1/BC2/BC3): one block per lane, the front of the pipeline's
+// classify pass (alpha, colour set, principal axis, then the single-colour or
+// range fit) without its record path.  A RangeFit block is a few hundred
+// serial operations; on a 16-lane group every fold would run on all 16 lanes.
+// Single-wave workgroups (the per-wave LDS copies of the block pixels and
+// weights), one per 64-block span of the image.
+template <int FMT>
+__device__ __forceinline__ void encode_range_lanes(const Image& im, uint32_t group, const FitParams& fp,
+                                                   LaneTables& LT, LaneBlockLds& LB)
+{
     const int lane = (int)threadIdx.x;
-    const uint64_t base = (uint64_t)group_index() * 64u;
-    if (base >= nblocks) return;
+    const uint64_t base = (uint64_t)group * 64u;
+    if (base >= im.nblocks) return;
     fill_lane_tables(LT, lane);
     group_sync();
     const uint64_t b = base + (uint64_t)lane;
-    if (b < nblocks) {
+    if (b < im.nblocks) {
         uint32_t px[16];
-        const uint32_t valid = fetch_block_lane(rgba, width, height, (uint32_t)(b % blocks_wide),
-                                                (uint32_t)(b / blocks_wide), px);
+        const uint32_t valid = fetch_block_lane(im.rgba, im.width, im.height, (uint32_t)(b % im.blocks_wide),
+                                                (uint32_t)(b / im.blocks_wide), px);
         uint32_t w[4];
         LaneSet S;
         float vx, vy, vz;
         encode_front_lane<FMT, RANGE_FIT>(px, valid, fp, LT, LB, lane, w, S, vx, vy, vz);
-        store_block<FMT>(out, b, w);
+        store_block<FMT>(im.out, b, w);
     }
+}
+
+template <int FMT>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_encode_range_lane(Image im,
+                                                                                                  FitParams fp)
+{
+    __shared__ LaneTables LT;
+    __shared__ LaneBlockLds LB;
+    encode_range_lanes<FMT>(im, group_index(), fp, LT, LB);
+}
+
+template <int FMT>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_encode_range_chain(
+    txk::ChainTable chain, uint8_t* __restrict__ out, FitParams fp)
+{
+    __shared__ LaneTables LT;
+    __shared__ LaneBlockLds LB;
+    uint32_t group = group_index();
+    const Image im = chain_image<FMT>(chain, out, group);
+    encode_range_lanes<FMT>(im, group, fp, LT, LB);
 }
 
 // Explicit block list (Format::compress_block_masked over many blocks): block
@@ -366,36 +428,60 @@ int team_groups(int algorithm, uint64_t nblocks)
     return nblocks <= (iterative ? 32768u : 6144u) ? 2 : 1;
 }
 
-template <int FMT, int ALG, int T>
-hipError_t launch_encode_n(const txk::EncodeArgs& a, hipStream_t s)
+txd::Image image_of(const txk::EncodeArgs& a)
 {
-    if (a.nblocks > 4 * txk::kMaxGroups2d) return hipErrorInvalidValue;
-    const uint64_t groups = (a.nblocks * T + 3) / 4;
-    if (groups == 0) return hipSuccess;
-    hipLaunchKernelGGL((txd::k_encode<FMT, ALG, T>), txk::grid_2d(groups), dim3(64), 0, s, a.rgba, a.width, a.height,
-                       a.blocks_wide, a.nblocks, a.out, txd::FitParams{a.wr, a.wg, a.wb, a.weigh_alpha});
+    return txd::Image{a.rgba, a.width, a.height, a.blocks_wide, a.nblocks, a.out};
+}
+txd::FitParams fit_of(const txk::EncodeArgs& a) { return txd::FitParams{a.wr, a.wg, a.wb, a.weigh_alpha}; }
+
+// Workgroups of `per_group` blocks for a texture, or for the levels of a chain
+// (which it numbers); 0 when there is nothing to launch or the grid's limit is
+// exceeded (`e` says which).
+uint64_t groups_for(const txk::EncodeArgs& a, txk::ChainTable* chain, uint32_t per_group, hipError_t& e)
+{
+    const uint64_t groups = chain ? chain->number(per_group) : (a.nblocks + per_group - 1) / per_group;
+    e = groups > txk::kMaxGroups2d ? hipErrorInvalidValue : hipSuccess;
+    return e == hipSuccess ? groups : 0;
+}
+
+// Every launcher takes the chain by pointer, null for a single texture.
+template <int FMT, int ALG, int T>
+hipError_t launch_encode_n(const txk::EncodeArgs& a, txk::ChainTable* chain, hipStream_t s)
+{
+    hipError_t e;
+    const uint64_t groups = groups_for(a, chain, 4 / T, e);
+    if (groups == 0) return e;
+    if (chain)
+        hipLaunchKernelGGL((txd::k_encode_chain<FMT, ALG, T>), txk::grid_2d(groups), dim3(64), 0, s, *chain, a.out,
+                           fit_of(a));
+    else
+        hipLaunchKernelGGL((txd::k_encode<FMT, ALG, T>), txk::grid_2d(groups), dim3(64), 0, s, image_of(a), fit_of(a));
     return hipGetLastError();
 }
 
 template <int FMT, int ALG>
-hipError_t launch_encode_t(const txk::EncodeArgs& a, hipStream_t s)
+hipError_t launch_encode_t(const txk::EncodeArgs& a, txk::ChainTable* chain, hipStream_t s)
 {
     if constexpr (ALG != 0) {
         const int t = team_groups(ALG, a.nblocks);
-        if (t == 4) return launch_encode_n<FMT, ALG, 4>(a, s);
-        if (t == 2) return launch_encode_n<FMT, ALG, 2>(a, s);
+        if (t == 4) return launch_encode_n<FMT, ALG, 4>(a, chain, s);
+        if (t == 2) return launch_encode_n<FMT, ALG, 2>(a, chain, s);
     }
-    return launch_encode_n<FMT, ALG, 1>(a, s);
+    return launch_encode_n<FMT, ALG, 1>(a, chain, s);
 }
 
 template <int FMT>
-hipError_t launch_encode_range(const txk::EncodeArgs& a, hipStream_t s)
+hipError_t launch_encode_range(const txk::EncodeArgs& a, txk::ChainTable* chain, hipStream_t s)
 {
-    const uint64_t waves = (a.nblocks + 63) / 64;
-    if (waves == 0) return hipSuccess;
-    if (waves > txk::kMaxGroups2d) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((txd::k_encode_range_lane<FMT>), txk::grid_2d(waves), dim3(64), 0, s, a.rgba, a.width, a.height,
-                       a.blocks_wide, a.nblocks, a.out, txd::FitParams{a.wr, a.wg, a.wb, a.weigh_alpha});
+    hipError_t e;
+    const uint64_t waves = groups_for(a, chain, 64, e);
+    if (waves == 0) return e;
+    if (chain)
+        hipLaunchKernelGGL((txd::k_encode_range_chain<FMT>), txk::grid_2d(waves), dim3(64), 0, s, *chain, a.out,
+                           fit_of(a));
+    else
+        hipLaunchKernelGGL((txd::k_encode_range_lane<FMT>), txk::grid_2d(waves), dim3(64), 0, s, image_of(a),
+                           fit_of(a));
     return hipGetLastError();
 }
 
@@ -408,12 +494,39 @@ hipError_t launch_encode_range(const txk::EncodeArgs& a, hipStream_t s)
 constexpr uint64_t kRangeLaneMinBlocks = 12288;
 
 template <int FMT>
-hipError_t launch_encode_f(const txk::EncodeArgs& a, hipStream_t s)
+hipError_t launch_encode_f(const txk::EncodeArgs& a, txk::ChainTable* chain, hipStream_t s)
 {
     switch (a.algorithm) {
-    case 0: return a.nblocks >= kRangeLaneMinBlocks ? launch_encode_range<FMT>(a, s) : launch_encode_t<FMT, 0>(a, s);
-    case 1: return launch_encode_t<FMT, 1>(a, s);
-    default: return launch_encode_t<FMT, 2>(a, s);
+    case 0:
+        return a.nblocks >= kRangeLaneMinBlocks ? launch_encode_range<FMT>(a, chain, s)
+                                                : launch_encode_t<FMT, 0>(a, chain, s);
+    case 1: return launch_encode_t<FMT, 1>(a, chain, s);
+    default: return launch_encode_t<FMT, 2>(a, chain, s);
+    }
+}
+
+template <int FMT>
+hipError_t launch_encode_alpha(const txk::EncodeArgs& a, txk::ChainTable* chain, hipStream_t s)
+{
+    hipError_t e;
+    const uint64_t groups = groups_for(a, chain, 256, e);
+    if (groups == 0) return e;
+    if (chain)
+        hipLaunchKernelGGL((txd::k_encode_alpha_chain<FMT>), txk::grid_2d(groups), dim3(256), 0, s, *chain, a.out);
+    else
+        hipLaunchKernelGGL((txd::k_encode_alpha<FMT>), txk::grid_2d(groups), dim3(256), 0, s, image_of(a));
+    return hipGetLastError();
+}
+
+hipError_t launch_encode_any(const txk::EncodeArgs& a, txk::ChainTable* chain, hipStream_t s)
+{
+    switch (a.format) {
+    case 0: return launch_encode_f<0>(a, chain, s);
+    case 1: return launch_encode_f<1>(a, chain, s);
+    case 2: return launch_encode_f<2>(a, chain, s);
+    case 3: return launch_encode_alpha<3>(a, chain, s);
+    case 4: return launch_encode_alpha<4>(a, chain, s);
+    default: return hipErrorInvalidValue;
     }
 }
 
@@ -467,27 +580,12 @@ hipError_t launch_decode_t(const uint8_t* data, uint32_t w, uint32_t h, uint8_t*
 
 namespace txk {
 
-template <int FMT>
-hipError_t launch_encode_alpha(const EncodeArgs& a, hipStream_t s)
-{
-    const uint64_t groups = (a.nblocks + 255) / 256;
-    if (groups == 0) return hipSuccess;
-    if (groups > kMaxGroups2d) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((txd::k_encode_alpha<FMT>), grid_2d(groups), dim3(256), 0, s, a.rgba, a.width, a.height,
-                       a.blocks_wide, a.nblocks, a.out);
-    return hipGetLastError();
-}
+hipError_t launch_encode(const EncodeArgs& a, hipStream_t s) { return launch_encode_any(a, nullptr, s); }
 
-hipError_t launch_encode(const EncodeArgs& a, hipStream_t s)
+hipError_t launch_encode_chain(const EncodeArgs& a, const ChainTable& levels, hipStream_t s)
 {
-    switch (a.format) {
-    case 0: return launch_encode_f<0>(a, s);
-    case 1: return launch_encode_f<1>(a, s);
-    case 2: return launch_encode_f<2>(a, s);
-    case 3: return launch_encode_alpha<3>(a, s);
-    case 4: return launch_encode_alpha<4>(a, s);
-    default: return hipErrorInvalidValue;
-    }
+    ChainTable chain = levels;
+    return launch_encode_any(a, &chain, s);
 }
 
 hipError_t launch_encode_blocks(const BlockListArgs& a, hipStream_t s)

@@ -28,6 +28,31 @@ struct BlockListArgs {
     uint32_t weigh_alpha;
 };
 
+// The levels of a mip chain encoded by one launch; their blocks lie back to
+// back in the output, level after level.
+constexpr uint32_t kMaxChainLevels = 32;
+struct ChainTable {
+    struct Level {
+        const uint8_t* rgba;  // device, 4-byte aligned
+        uint32_t width, height, blocks_wide, nblocks;
+        uint32_t block0;  // blocks of the levels before it
+    };
+    uint32_t count;
+    uint32_t first[kMaxChainLevels];  // first workgroup (or chunk) of each level, set by the launcher
+    Level level[kMaxChainLevels];
+
+    // Numbers the levels' workgroups of `per_group` blocks; returns how many.
+    uint64_t number(uint32_t per_group)
+    {
+        uint64_t n = 0;
+        for (uint32_t k = 0; k < count; ++k) {
+            first[k] = (uint32_t)n;
+            n += ((uint64_t)level[k].nblocks + per_group - 1) / per_group;
+        }
+        return n;
+    }
+};
+
 // One texture of a persistent batch launch, as the device reads it.
 struct BatchTex {
     const uint8_t* rgba;
@@ -104,6 +129,9 @@ inline dim3 grid_2d(uint64_t groups)
 }
 
 hipError_t launch_encode(const EncodeArgs& a, hipStream_t s);
+// The same kernels over every level of a chain in one launch: `a` holds the
+// format, algorithm, weights, output and the total block count (below 2^32).
+hipError_t launch_encode_chain(const EncodeArgs& a, const ChainTable& levels, hipStream_t s);
 hipError_t launch_encode_blocks(const BlockListArgs& a, hipStream_t s);
 hipError_t launch_decode(int format, const uint8_t* data, uint32_t w, uint32_t h, uint8_t* out, hipStream_t s);
 // The elementary-operation check (tx_util_elementary): d_tables holds

@@ -194,9 +194,9 @@ static bool takes_pipeline(const txk::EncodeArgs& a)
     return cluster && a.nblocks >= pipeline_threshold(a.format, a.algorithm) && a.nblocks <= 0xFFFFFFFFull;
 }
 
-// Launch shape of the binned pipeline for one texture on a device with
-// `cus` compute units.
-static txp::PipeLaunch pipe_launch_for(const txk::EncodeArgs& a, uint32_t cus)
+// Launch shape of the binned pipeline for one texture, or for the levels of
+// `chain` (a.nblocks blocks in all), on a device with `cus` compute units.
+static txp::PipeLaunch pipe_launch_for(const txk::EncodeArgs& a, const txk::ChainTable* chain, uint32_t cus)
 {
     txp::PipeLaunch p{};
     p.d_tex = nullptr;
@@ -223,7 +223,8 @@ static txp::PipeLaunch pipe_launch_for(const txk::EncodeArgs& a, uint32_t cus)
     uint64_t cb = (a.nblocks + simds - 1) / simds;
     cb = std::min<uint64_t>(64, std::max<uint64_t>(16, (cb + 15) & ~(uint64_t)15));
     p.chunk_blocks = (uint32_t)cb;
-    p.nchunks = (uint32_t)((a.nblocks + cb - 1) / cb);
+    if (chain) p.chain = *chain;
+    p.nchunks = (uint32_t)(chain ? p.chain.number(p.chunk_blocks) : (a.nblocks + cb - 1) / cb);
     p.nslots = a.nblocks;
     p.d_chunks = nullptr;
     p.classify_grid = (uint32_t)std::min<uint64_t>(cwaves, p.nchunks);
@@ -236,18 +237,20 @@ static txp::PipeLaunch pipe_launch_for(const txk::EncodeArgs& a, uint32_t cus)
 // binned pipeline (classify, bin, independent per-block searches),
 // everything else through the direct kernel.  Both produce the same bytes.
 // With `marks` (5 events) the pipeline records them between its kernels;
-// `used_pipeline` says which path ran.
+// `used_pipeline` says which path ran.  With `chain`, the levels of a chain
+// instead of one texture (a.nblocks counts the blocks of them all).
 static hipError_t encode_on(txc::DeviceContext* ctx, const txk::EncodeArgs& a, hipStream_t s,
-                            hipEvent_t* marks = nullptr, bool* used_pipeline = nullptr)
+                            const txk::ChainTable* chain = nullptr, hipEvent_t* marks = nullptr,
+                            bool* used_pipeline = nullptr)
 {
     if (used_pipeline) *used_pipeline = false;
-    if (!takes_pipeline(a)) return txk::launch_encode(a, s);
+    if (!takes_pipeline(a)) return chain ? txk::launch_encode_chain(a, *chain, s) : txk::launch_encode(a, s);
     if (used_pipeline) *used_pipeline = true;
     std::lock_guard<std::mutex> lock(ctx->pipe_mu);
     txp::PipeBufs bufs;
     if (!ctx->pipe_scratch(a.nblocks, &bufs)) return hipErrorOutOfMemory;
     if (!ctx->pipe_before(s)) return hipErrorUnknown;
-    const hipError_t e = txp::launch_pipeline(pipe_launch_for(a, (uint32_t)ctx->cus), bufs, s, marks);
+    const hipError_t e = txp::launch_pipeline(pipe_launch_for(a, chain, (uint32_t)ctx->cus), bufs, s, marks);
     if (!ctx->pipe_after(s)) return hipErrorUnknown;
     return e;
 }
@@ -316,7 +319,7 @@ int tx_compress_device_noalloc(int format, const uint8_t* d_rgba, size_t width, 
     if (a.nblocks > TX_NOALLOC_MAX_PIPELINE_BLOCKS) return TX_ERR_TOO_LARGE;
     txp::PipeBufs bufs;
     bufs.carve(dev->ptr, TX_NOALLOC_MAX_PIPELINE_BLOCKS);
-    return txp::launch_pipeline(pipe_launch_for(a, dev->cus), bufs, s) == hipSuccess ? TX_OK : TX_ERR_HIP;
+    return txp::launch_pipeline(pipe_launch_for(a, nullptr, dev->cus), bufs, s) == hipSuccess ? TX_OK : TX_ERR_HIP;
 }
 
 // ------------------------------------------------------------ mip chains
@@ -389,12 +392,21 @@ static hipError_t mips_on(const uint8_t* d_rgba, size_t width, size_t height, ui
     return hipSuccess;
 }
 
+// Levels of more blocks than this are encoded by launches of their own and the
+// rest of the chain by one: a level takes one block's latency however small it
+// is (13-70 us, eleven levels in series for a 1024^2 chain), while a large
+// level fills the GPU by itself and would only enlarge the record buffers.
+constexpr uint64_t kChainLevelMaxBlocks = 1u << 20;
+
 // Every level of the chain (level 0 = d_rgba, then d_chain) compressed back
 // to back into d_output, level 0 first.
 static hipError_t compress_chain_on(txc::DeviceContext* ctx, int format, const tx_params* params,
                                     const uint8_t* d_rgba, size_t width, size_t height, uint32_t levels,
                                     const uint8_t* d_chain, uint8_t* d_output, hipStream_t s)
 {
+    txk::ChainTable chain{};  // the levels that go together
+    uint64_t chain_blocks = 0;
+    uint8_t* chain_out = d_output;
     const uint8_t* src = d_rgba;
     size_t in_off = 0, out_off = 0;
     for (uint32_t k = 0; k < levels; ++k) {
@@ -404,11 +416,23 @@ static hipError_t compress_chain_on(txc::DeviceContext* ctx, int format, const t
             src = d_chain + in_off;
             in_off += 4 * w * h;
         }
-        const hipError_t e = encode_on(ctx, encode_args(format, params, src, w, h, d_output + out_off, n), s);
-        if (e != hipSuccess) return e;
+        const txk::EncodeArgs a = encode_args(format, params, src, w, h, d_output + out_off, n);
+        if (a.nblocks > kChainLevelMaxBlocks || levels == 1) {
+            const hipError_t e = encode_on(ctx, a, s);
+            if (e != hipSuccess) return e;
+        } else {
+            if (chain.count == 0) chain_out = a.out;
+            if (chain.count == txk::kMaxChainLevels) return hipErrorInvalidValue;
+            chain.level[chain.count++] = txk::ChainTable::Level{
+                src, (uint32_t)w, (uint32_t)h, a.blocks_wide, (uint32_t)a.nblocks, (uint32_t)chain_blocks};
+            chain_blocks += a.nblocks;
+        }
         out_off += n;
     }
-    return hipSuccess;
+    if (chain.count == 0) return hipSuccess;
+    txk::EncodeArgs a = encode_args(format, params, chain.level[0].rgba, chain.level[0].width, chain.level[0].height,
+                                    chain_out, chain_blocks * tx_block_size(format));
+    return encode_on(ctx, a, s, chain.count > 1 ? &chain : nullptr);
 }
 
 int tx_generate_mips_device(const uint8_t* d_rgba, size_t width, size_t height, uint32_t levels, uint8_t* d_chain,
@@ -697,7 +721,7 @@ int tx_util_time_phases(int format, const uint8_t* d_rgba, size_t width, size_t 
     const txk::EncodeArgs a = encode_args(format, params, d_rgba, width, height, d_output, out_len);
     for (int it = 0; it < iters && rc == TX_OK; ++it) {
         bool pipe = false;
-        if (encode_on(ctx, a, ctx->stream, ev, &pipe) != hipSuccess) rc = TX_ERR_HIP;
+        if (encode_on(ctx, a, ctx->stream, nullptr, ev, &pipe) != hipSuccess) rc = TX_ERR_HIP;
         *used_pipeline = pipe ? 1 : 0;
         if (rc != TX_OK || !pipe) break;
         if (hipEventSynchronize(ev[4]) != hipSuccess) rc = TX_ERR_HIP;

@@ -119,10 +119,17 @@ __device__ __forceinline__ uint32_t write_record_lane(ClusterRec* __restrict__ r
 
 // Blocks [first, first + count) of one texture, one per lane, 64 at a time.
 // Single-colour and range-fit blocks are finished here; ClusterFit blocks
-// become records in slots [slot0, slot0 + count), counted in ctl->part.
-template <int FMT, int ALG>
-__device__ __forceinline__ void classify_chunk(const BatchTex& T, uint32_t tex_idx, uint32_t first, uint32_t count,
-                                               uint32_t slot0, const LaneTables& LT, LaneBlockLds& LB, int lane,
+// become records in slots [slot0, slot0 + count), counted in ctl->part.  Block
+// b of the pixel grid (a texture, or a level of a chain) is block b + block0 of
+// the output.
+struct PixelGrid {
+    const uint8_t* rgba;
+    uint32_t width, height, blocks_wide;
+};
+
+template <int FMT, int ALG, class Grid>
+__device__ __forceinline__ void classify_chunk(const Grid& G, const BatchTex& T, uint32_t tex_idx, uint32_t first, uint32_t count,
+                                               uint32_t slot0, uint32_t block0, const LaneTables& LT, LaneBlockLds& LB, int lane,
                                                ClusterRec* recs, uint32_t* keys, PipeCtl* ctl)
 {
     const FitParams fp{T.wr, T.wg, T.wb, T.weigh_alpha};
@@ -132,19 +139,19 @@ __device__ __forceinline__ void classify_chunk(const BatchTex& T, uint32_t tex_i
         if (k < count) {
             const uint32_t b = first + k;
             uint32_t px[16];
-            const uint32_t valid = fetch_block_lane(T.rgba, T.width, T.height, b % T.blocks_wide,
-                                                    b / T.blocks_wide, px);
+            const uint32_t valid = fetch_block_lane(G.rgba, G.width, G.height, b % G.blocks_wide,
+                                                    b / G.blocks_wide, px);
             uint32_t w[4];
             LaneSet S;
             float vx, vy, vz;
             const int kind = encode_front_lane<FMT, ALG>(px, valid, fp, LT, LB, lane, w, S, vx, vy, vz,
                                                          recs[slot0 + k].pts);
             if (kind == KIND_CLUSTER) {
-                key = write_record_lane<FMT, ALG>(recs, slot0 + k, S, w, vx, vy, vz, fp, tex_idx, b);
+                key = write_record_lane<FMT, ALG>(recs, slot0 + k, S, w, vx, vy, vz, fp, tex_idx, block0 + b);
             } else if (FMT == BC1) {
-                *reinterpret_cast<uint2*>(T.out + (size_t)b * 8u) = make_uint2(w[0], w[1]);
+                *reinterpret_cast<uint2*>(T.out + ((size_t)block0 + b) * 8u) = make_uint2(w[0], w[1]);
             } else {
-                *reinterpret_cast<uint4*>(T.out + (size_t)b * 16u) = make_uint4(w[0], w[1], w[2], w[3]);
+                *reinterpret_cast<uint4*>(T.out + ((size_t)block0 + b) * 16u) = make_uint4(w[0], w[1], w[2], w[3]);
             }
             keys[slot0 + k] = key;
         }
@@ -152,14 +159,13 @@ __device__ __forceinline__ void classify_chunk(const BatchTex& T, uint32_t tex_i
     }
 }
 
-// Classify over the heavy chunks (BC1/BC2/BC3 textures), each workgroup
-// taking chunks blockIdx.x, blockIdx.x + gridDim.x, ...  Chunk c covers
-// blocks [first, first + count) of one texture and record slots
+// Classify over the heavy chunks (BC1/BC2/BC3 textures) of a batch, each
+// workgroup taking chunks blockIdx.x, blockIdx.x + gridDim.x, ...  Chunk c
+// covers blocks [first, first + count) of one texture and record slots
 // [slot0, slot0 + count).
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_pipe_classify(const BatchTex* __restrict__ tex, BatchTex tex0,
-                                                      const uint4* __restrict__ chunks, uint32_t nchunks,
-                                                      uint32_t chunk_blocks, ClusterRec* __restrict__ recs,
-                                                      uint32_t* __restrict__ keys, PipeCtl* __restrict__ ctl)
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_pipe_classify(
+    const BatchTex* __restrict__ tex, const uint4* __restrict__ chunks, uint32_t nchunks,
+    ClusterRec* __restrict__ recs, uint32_t* __restrict__ keys, PipeCtl* __restrict__ ctl)
 {
     __shared__ LaneTables LT;
     __shared__ LaneBlockLds LB;
@@ -169,25 +175,49 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
     // chunks hold similar work, so a plain grid-stride loop balances them
     // (a shared work counter would serialise thousands of atomics at launch)
     for (uint32_t c = blockIdx.x; c < nchunks; c += gridDim.x) {
-        uint4 ch;
-        if (chunks) {
-            ch = chunks[c];
-        } else {
-            const uint32_t f = c * chunk_blocks;
-            ch = make_uint4(0u, f, min(chunk_blocks, tex0.nblocks - f), f);
-        }
-        const BatchTex& T = tex_at(tex, tex0, ch.x);
+        const uint4 ch = chunks[c];
+        const BatchTex& T = tex[ch.x];
         switch (T.variant) {
-        case 0: classify_chunk<BC1, RANGE_FIT>(T, ch.x, ch.y, ch.z, ch.w, LT, LB, lane, recs, keys, ctl); break;
-        case 1: classify_chunk<BC1, CLUSTER_FIT>(T, ch.x, ch.y, ch.z, ch.w, LT, LB, lane, recs, keys, ctl); break;
-        case 2: classify_chunk<BC1, ITERATIVE_CLUSTER_FIT>(T, ch.x, ch.y, ch.z, ch.w, LT, LB, lane, recs, keys, ctl); break;
-        case 3: classify_chunk<BC2, RANGE_FIT>(T, ch.x, ch.y, ch.z, ch.w, LT, LB, lane, recs, keys, ctl); break;
-        case 4: classify_chunk<BC2, CLUSTER_FIT>(T, ch.x, ch.y, ch.z, ch.w, LT, LB, lane, recs, keys, ctl); break;
-        case 5: classify_chunk<BC2, ITERATIVE_CLUSTER_FIT>(T, ch.x, ch.y, ch.z, ch.w, LT, LB, lane, recs, keys, ctl); break;
-        case 6: classify_chunk<BC3, RANGE_FIT>(T, ch.x, ch.y, ch.z, ch.w, LT, LB, lane, recs, keys, ctl); break;
-        case 7: classify_chunk<BC3, CLUSTER_FIT>(T, ch.x, ch.y, ch.z, ch.w, LT, LB, lane, recs, keys, ctl); break;
-        default: classify_chunk<BC3, ITERATIVE_CLUSTER_FIT>(T, ch.x, ch.y, ch.z, ch.w, LT, LB, lane, recs, keys, ctl); break;
+        case 0: classify_chunk<BC1, RANGE_FIT>(T, T, ch.x, ch.y, ch.z, ch.w, 0u, LT, LB, lane, recs, keys, ctl); break;
+        case 1: classify_chunk<BC1, CLUSTER_FIT>(T, T, ch.x, ch.y, ch.z, ch.w, 0u, LT, LB, lane, recs, keys, ctl); break;
+        case 2: classify_chunk<BC1, ITERATIVE_CLUSTER_FIT>(T, T, ch.x, ch.y, ch.z, ch.w, 0u, LT, LB, lane, recs, keys, ctl); break;
+        case 3: classify_chunk<BC2, RANGE_FIT>(T, T, ch.x, ch.y, ch.z, ch.w, 0u, LT, LB, lane, recs, keys, ctl); break;
+        case 4: classify_chunk<BC2, CLUSTER_FIT>(T, T, ch.x, ch.y, ch.z, ch.w, 0u, LT, LB, lane, recs, keys, ctl); break;
+        case 5: classify_chunk<BC2, ITERATIVE_CLUSTER_FIT>(T, T, ch.x, ch.y, ch.z, ch.w, 0u, LT, LB, lane, recs, keys, ctl); break;
+        case 6: classify_chunk<BC3, RANGE_FIT>(T, T, ch.x, ch.y, ch.z, ch.w, 0u, LT, LB, lane, recs, keys, ctl); break;
+        case 7: classify_chunk<BC3, CLUSTER_FIT>(T, T, ch.x, ch.y, ch.z, ch.w, 0u, LT, LB, lane, recs, keys, ctl); break;
+        default: classify_chunk<BC3, ITERATIVE_CLUSTER_FIT>(T, T, ch.x, ch.y, ch.z, ch.w, 0u, LT, LB, lane, recs, keys, ctl); break;
         }
+    }
+}
+
+// The same for one texture, or the levels of a chain: chunks of chunk_blocks
+// blocks, none of them over two levels; slots and output blocks count through
+// the chain.  A kernel of its own per format and algorithm: the batch kernel
+// holds nine variants.
+template <int FMT, int ALG>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_pipe_classify_one(
+    BatchTex tex0, txk::ChainTable chain, uint32_t nchunks, uint32_t chunk_blocks, ClusterRec* __restrict__ recs,
+    uint32_t* __restrict__ keys, PipeCtl* __restrict__ ctl)
+{
+    __shared__ LaneTables LT;
+    __shared__ LaneBlockLds LB;
+    const int lane = (int)threadIdx.x;
+    fill_lane_tables(LT, lane);
+    group_sync();
+    for (uint32_t c = blockIdx.x; c < nchunks; c += gridDim.x) {
+        PixelGrid G{tex0.rgba, tex0.width, tex0.height, tex0.blocks_wide};
+        uint32_t f = c * chunk_blocks, n = tex0.nblocks, block0 = 0;
+        if (chain.count) {
+            const uint32_t k = chain_level(chain, c);
+            const txk::ChainTable::Level& v = chain.level[k];
+            f = (c - chain.first[k]) * chunk_blocks;
+            n = v.nblocks;
+            block0 = v.block0;
+            G = PixelGrid{v.rgba, v.width, v.height, v.blocks_wide};
+        }
+        classify_chunk<FMT, ALG>(G, tex0, 0u, f, min(chunk_blocks, n - f), block0 + f, block0, LT, LB, lane, recs,
+                                 keys, ctl);
     }
 }
 
@@ -566,6 +596,35 @@ __global__ __launch_bounds__(64 * kSearchWaves) __attribute__((amdgpu_waves_per_
 
 namespace txp {
 
+namespace {
+
+template <int FMT, int ALG>
+void launch_classify_one(const PipeLaunch& p, const PipeBufs& b, hipStream_t s)
+{
+    hipLaunchKernelGGL((txd::k_pipe_classify_one<FMT, ALG>), dim3(p.classify_grid), dim3(64), 0, s, p.tex0, p.chain,
+                       p.nchunks, p.chunk_blocks, b.recs, b.keys, b.ctl);
+}
+
+hipError_t launch_classify(const PipeLaunch& p, const PipeBufs& b, hipStream_t s)
+{
+    if (p.d_tex) {
+        hipLaunchKernelGGL(txd::k_pipe_classify, dim3(p.classify_grid), dim3(64), 0, s, p.d_tex, p.d_chunks,
+                           p.nchunks, b.recs, b.keys, b.ctl);
+        return hipSuccess;
+    }
+    switch (p.tex0.variant) {
+    case 1: launch_classify_one<0, 1>(p, b, s); return hipSuccess;
+    case 2: launch_classify_one<0, 2>(p, b, s); return hipSuccess;
+    case 4: launch_classify_one<1, 1>(p, b, s); return hipSuccess;
+    case 5: launch_classify_one<1, 2>(p, b, s); return hipSuccess;
+    case 7: launch_classify_one<2, 1>(p, b, s); return hipSuccess;
+    case 8: launch_classify_one<2, 2>(p, b, s); return hipSuccess;
+    default: return hipErrorInvalidValue;
+    }
+}
+
+}  // namespace
+
 hipError_t launch_pipeline(const PipeLaunch& p, const PipeBufs& b, hipStream_t s, hipEvent_t* marks)
 {
     if (p.nslots > b.capacity || p.nslots > 0xFFFFFFFFull) return hipErrorInvalidValue;
@@ -577,8 +636,7 @@ hipError_t launch_pipeline(const PipeLaunch& p, const PipeBufs& b, hipStream_t s
         return hipGetLastError();
     }
     if (mark(0) != hipSuccess) return hipErrorUnknown;
-    hipLaunchKernelGGL(txd::k_pipe_classify, dim3(p.classify_grid), dim3(64), 0, s, p.d_tex, p.tex0, p.d_chunks,
-                       p.nchunks, p.chunk_blocks, b.recs, b.keys, b.ctl);
+    if (launch_classify(p, b, s) != hipSuccess) return hipErrorInvalidValue;
     if (mark(1) != hipSuccess) return hipErrorUnknown;
     const uint32_t bin_grid = (uint32_t)((p.nslots + kBinSeg - 1) / kBinSeg);
     const uint32_t search_wgs = (p.search_grid + kSearchWaves - 1) / kSearchWaves;

@@ -101,10 +101,12 @@ constexpr uint32_t kSearchWavesPerCu = 16;
 constexpr uint32_t kSearchWaves = 4;  // waves per search workgroup (sharing one run of list positions)
 
 struct PipeLaunch {
-    const txk::BatchTex* d_tex;  // texture descriptors (null: only `tex0`)
-    txk::BatchTex tex0;          // the texture when d_tex is null
+    const txk::BatchTex* d_tex;  // texture descriptors, with d_chunks (null: only `tex0`)
+    txk::BatchTex tex0;          // the texture when d_tex is null (ClusterFit or IterativeClusterFit)
     const uint4* d_chunks;       // heavy chunks (texture, first block, count, first record slot);
-                                 // null: implicit chunks of tex0
+                                 // null with d_tex: implicit chunks of tex0
+    txk::ChainTable chain;       // count > 0: the levels of a chain, tex0 holding what they share and the
+                                 // output; implicit chunks, already numbered
     uint32_t nchunks;            // heavy chunks
     uint32_t chunk_blocks;       // implicit chunk size
     uint64_t nslots;             // record slots the chunks cover (<= capacity)
