@@ -415,6 +415,22 @@ __device__ __forceinline__ float recip(float x)
     return __builtin_amdgcn_div_fixupf(__builtin_fmaf(r, __builtin_fmaf(-x, r, 1.0f), r), x, 1.0f);
 }
 
+// u / 255.0f of a byte value: with 1/255 as a binary32 pair, the fused sum is
+// the correctly rounded quotient for all 256 values (the device is checked
+// against the division), two instructions for a division's eleven.
+__device__ __forceinline__ float unit8(uint32_t u)
+{
+    constexpr float hi = 1.0f / 255.0f, lo = (float)(1.0 / 255.0 - (double)(1.0f / 255.0f));
+    const float f = (float)u;
+    return __builtin_fmaf(f, hi, f * lo);
+}
+__device__ __forceinline__ void rgb_point(uint32_t px, float& x, float& y, float& z)
+{
+    x = unit8(px & 255u);
+    y = unit8((px >> 8) & 255u);
+    z = unit8((px >> 16) & 255u);
+}
+
 // A constant kept in a vector register.  As an operand of a VOP3 form (which
 // takes no literal) the compiler would put it in a scalar register, and a
 // scalar operand halves the issue rate of FP32 instructions (v_fma_f32 with
@@ -557,6 +573,17 @@ __device__ __forceinline__ void range_fit(const LDS& L, const ColourSet& cs, int
 __device__ __forceinline__ float4 sum_at(const float4* S, uint32_t bytes)
 {
     return *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(S) + bytes);
+}
+
+// range.rs:44-192 of a block without points (every pixel excluded), the only
+// range fits among the cluster fits: both endpoints snap to zero; the 3-colour
+// pass (BC1) takes the block with every index 3, the 4-colour pass has equal
+// endpoints and so every index 0.
+template <int FMT>
+__device__ __forceinline__ void empty_fit(uint32_t& lo, uint32_t& hi)
+{
+    lo = 0u;
+    hi = FMT == BC1 ? 0xFFFFFFFFu : 0u;
 }
 
 // The three prefix sums a split reads: part0 = S[0][i], part1, part2.
@@ -1424,8 +1451,9 @@ __device__ __forceinline__ int encode_front(uint32_t px, bool valid, const FitPa
     if (is_new) {
         // weights sum exactly (multiples of 1/256 below 16), then sqrtf
         const float w = fp.weigh_alpha ? (float)asum / 256.0f : (float)__popc(same);
-        L.pts[cs.remap] = make_float4((float)(rgb & 255u) / 255.0f, (float)((rgb >> 8) & 255u) / 255.0f,
-                                      (float)((rgb >> 16) & 255u) / 255.0f, sqrtf(w));
+        float x, y, z;
+        rgb_point(rgb, x, y, z);
+        L.pts[cs.remap] = make_float4(x, y, z, sqrtf(w));
     }
     group_sync();
 
@@ -1438,7 +1466,11 @@ __device__ __forceinline__ int encode_front(uint32_t px, bool valid, const FitPa
     vy = 0.0f;
     vz = 0.0f;
     if (kind != KIND_SINGLE) principal_axis(L, cs.n, vx, vy, vz);
-    if (kind == KIND_RANGE) range_fit<FMT>(L, cs, l, fp, vx, vy, vz, lo, hi);
+    if (ALG == RANGE_FIT) {
+        if (kind == KIND_RANGE) range_fit<FMT>(L, cs, l, fp, vx, vy, vz, lo, hi);
+    } else if (kind == KIND_RANGE) {
+        empty_fit<FMT>(lo, hi);
+    }
     set_colour<FMT>(out, lo, hi);
     return kind;
 }

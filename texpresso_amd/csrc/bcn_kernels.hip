@@ -377,7 +377,7 @@ __global__ __launch_bounds__(256) void k_decode(const uint8_t* __restrict__ data
 
 // The exactly specified elementary operations of the encoder, evaluated by
 // the device functions the kernels use, for an exhaustive check against a
-// host IEEE binary32 evaluation: the u8/255 and sqrt(count) tables the
+// host IEEE binary32 evaluation: u8/255 (unit8), the sqrt(count) table the
 // one-block-per-lane front fills (fill_lane_tables), sqrtf(k / 256) of the
 // alpha-weighted point weights (k = 1..4096, the range of the summed
 // (alpha + 1) values), and for each input value the 5- and 6-bit grid snap
@@ -392,7 +392,7 @@ __global__ __launch_bounds__(64) void k_elementary(const float* __restrict__ in,
     if (blockIdx.x == 0) {
         fill_lane_tables(T, lane);
         group_sync();
-        for (int i = lane; i < 256; i += 64) tables[i] = T.u8f[i];
+        for (int i = lane; i < 256; i += 64) tables[i] = unit8((uint32_t)i);
         if (lane < 17) tables[256 + lane] = T.sqc[lane];
         for (int k = lane + 1; k <= 4096; k += 64) tables[256 + 17 + (k - 1)] = sqrtf((float)k / 256.0f);
     }

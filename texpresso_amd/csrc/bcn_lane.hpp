@@ -15,24 +15,20 @@
 
 namespace txd {
 
-// Exact values the front needs, filled once per workgroup with the same
-// expressions the group front evaluates: u8 / 255 for the colour channels and
-// sqrtf(count) for unweighted point weights.
+// sqrtf(count) of the unweighted point weights, filled once per workgroup.
 struct LaneTables {
-    float u8f[256];
     float sqc[17];
 };
 
 __device__ __forceinline__ void fill_lane_tables(LaneTables& T, int lane)
 {
-    for (int i = lane; i < 256; i += 64) T.u8f[i] = (float)i / 255.0f;
     if (lane < 17) T.sqc[lane] = sqrtf((float)lane);
 }
 
 // Per-wave LDS of the lane front: the pixels and point weights of every
 // lane's block, pixel-major with the lane fastest (each access by the wave is
-// 64 consecutive words, free of bank conflicts).  Loops over pixels read
-// them here by index instead of holding 16-wide arrays in registers.
+// 64 consecutive words, free of bank conflicts).  Rolled loops over pixels
+// read them here by index.
 struct LaneBlockLds {
     uint32_t px[16][64];
     float w[16][64];
@@ -52,17 +48,6 @@ struct LaneSet {
     __device__ uint32_t pix(int p) const { return L->px[p][lane]; }
     __device__ float wt(int p) const { return L->w[p][lane]; }  // sqrt(weight), 0 off the points
 };
-
-// Colour of a pixel as a point (x, y, z in [0, 1]), from the u8 / 255 table.
-// (An arithmetic form, c * (1/255) corrected by one fma step from the exact
-// residual, is correctly rounded for all 256 bytes but measured no faster:
-// its fma and conversion issue at half the rate of plain adds.)
-__device__ __forceinline__ void xyz(const LaneTables& T, uint32_t rgb, float& x, float& y, float& z)
-{
-    x = T.u8f[rgb & 255u];
-    y = T.u8f[(rgb >> 8) & 255u];
-    z = T.u8f[(rgb >> 16) & 255u];
-}
 
 // Pixel p's colour as a comparison key: its RGB when included, otherwise a
 // value no colour has (so it matches nothing).
@@ -247,19 +232,21 @@ __device__ __forceinline__ void colour_set_lane(const uint32_t (&px)[16], uint32
 }
 
 // math.rs:44-97 over the points of a lane's set (same folds as
-// principal_axis).  The folds run over all 16 pixels: a pixel that opens no
+// principal_axis).  The folds run over all 16 pixels, unrolled, with the
+// colours converted from the pixel registers (a rolled loop over LDS copies
+// waits out two LDS reads per step, most of its time): a pixel that opens no
 // point has w = 0, so its terms are +0 or -0 and adding them leaves the
 // (never negative-zero) accumulators unchanged.  With `pts`, the first fold
 // also stores each point as (x, y, z, weight) at its point index there (the
 // ClusterFit record of the block).
-__device__ __forceinline__ void principal_axis_lane(const LaneSet& S, const LaneTables& T, float& vx, float& vy,
+__device__ __forceinline__ void principal_axis_lane(const LaneSet& S, const uint32_t (&px)[16], float& vx, float& vy,
                                                     float& vz, float4* __restrict__ pts = nullptr)
 {
     float total = 0.0f, cx = 0.0f, cy = 0.0f, cz = 0.0f;
-#pragma unroll 4
+#pragma unroll
     for (int p = 0; p < 16; ++p) {
         float x, y, z;
-        xyz(T, S.pix(p), x, y, z);
+        rgb_point(px[p], x, y, z);
         const float w = S.wt(p);
         if (pts && ((S.first >> p) & 1u)) pts[__popc(S.first & ((1u << p) - 1u))] = make_float4(x, y, z, w);
         total = total + w;
@@ -273,10 +260,10 @@ __device__ __forceinline__ void principal_axis_lane(const LaneSet& S, const Lane
         cz = cz / total;
     }
     float c0 = 0.0f, c1 = 0.0f, c2 = 0.0f, c3 = 0.0f, c4 = 0.0f, c5 = 0.0f;
-#pragma unroll 4
+#pragma unroll
     for (int p = 0; p < 16; ++p) {
         float x, y, z;
-        xyz(T, S.pix(p), x, y, z);
+        rgb_point(px[p], x, y, z);
         const float w = S.wt(p);
         const float ax = x - cx, ay = y - cy, az = z - cz;
         const float bx = ax * w, by = ay * w, bz = az * w;
@@ -332,17 +319,17 @@ __device__ __forceinline__ uint32_t spread_index(uint32_t inc, uint32_t in)
 }
 
 // Colour of point 0 (the lowest pixel that opens a point).
-__device__ __forceinline__ void point0_lane(const LaneSet& S, const LaneTables& T, float& qx, float& qy, float& qz)
+__device__ __forceinline__ void point0_lane(const LaneSet& S, float& qx, float& qy, float& qz)
 {
-    xyz(T, S.pix(S.first ? __builtin_ctz(S.first) : 0), qx, qy, qz);
+    rgb_point(S.pix(S.first ? __builtin_ctz(S.first) : 0), qx, qy, qz);
 }
 
 // single.rs:100-164 (same steps as single_fit)
 template <int FMT>
-__device__ __forceinline__ void single_fit_lane(const LaneSet& S, const LaneTables& T, uint32_t& lo, uint32_t& hi)
+__device__ __forceinline__ void single_fit_lane(const LaneSet& S, uint32_t& lo, uint32_t& hi)
 {
     float qx, qy, qz;
-    point0_lane(S, T, qx, qy, qz);
+    point0_lane(S, qx, qy, qz);
     const int cr = f32_to_i32_clamped(qx * 255.0f, 255);
     const int cg = f32_to_i32_clamped(qy * 255.0f, 255);
     const int cb = f32_to_i32_clamped(qz * 255.0f, 255);
@@ -364,39 +351,39 @@ __device__ __forceinline__ void single_fit_lane(const LaneSet& S, const LaneTabl
 }
 
 // range.rs:44-192 (same steps as range_fit): the index of every included
-// pixel is that of its colour, which is its point's.
+// pixel is that of its colour, which is its point's.  The pixel loops are
+// unrolled over the pixel registers and free of branches, so that a pixel's
+// arithmetic runs beside its neighbours': a range fit is a few thousand
+// dependent operations per lane, and a launch of up to 65,536 blocks has one
+// wave per SIMD to hide them.
 template <int FMT>
-__device__ __forceinline__ void range_fit_lane(const LaneSet& S, const LaneTables& T, const FitParams& fp, float px,
-                                               float py, float pz, uint32_t& lo, uint32_t& hi)
+__device__ __forceinline__ void range_fit_lane(const LaneSet& S, const uint32_t (&pix)[16], const FitParams& fp,
+                                               float px, float py, float pz, uint32_t& lo, uint32_t& hi)
 {
+    // extremes of the projections over the points, in point order from point
+    // 0: a new minimum first, else a new maximum
     float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, e0 = 0.0f, e1 = 0.0f, e2 = 0.0f;
-    if (S.n > 0) {
-        float q0x, q0y, q0z;
-        point0_lane(S, T, q0x, q0y, q0z);
-        s0 = q0x; s1 = q0y; s2 = q0z;
-        e0 = s0; e1 = s1; e2 = s2;
-        float mn = q0x * px + q0y * py + q0z * pz;
-        float mx = mn;
-        const uint32_t rest = S.first & (S.first - 1u);  // points 1..n-1
-#pragma unroll 2
-        for (int p = 0; p < 16; ++p) {
-            if ((rest >> p) & 1u) {
-                float x, y, z;
-                xyz(T, S.pix(p), x, y, z);
-                const float d = x * px + y * py + z * pz;
-                if (d < mn) {
-                    s0 = x; s1 = y; s2 = z; mn = d;
-                } else if (d > mx) {
-                    e0 = x; e1 = y; e2 = z; mx = d;
-                }
-            }
-        }
+    float mn = 0.0f, mx = 0.0f;
+    bool any = false;
+#pragma unroll
+    for (int p = 0; p < 16; ++p) {
+        float x, y, z;
+        rgb_point(pix[p], x, y, z);
+        const float d = x * px + y * py + z * pz;
+        const bool pt = (S.first >> p) & 1u;
+        const bool lower = pt & (!any | (d < mn));
+        const bool upper = pt & (!any | (!lower & (d > mx)));
+        s0 = lower ? x : s0; s1 = lower ? y : s1; s2 = lower ? z : s2;
+        mn = lower ? d : mn;
+        e0 = upper ? x : e0; e1 = upper ? y : e1; e2 = upper ? z : e2;
+        mx = upper ? d : mx;
+        any = any | pt;
     }
     s0 = snap(s0, 31.0f, 1.0f / 31.0f); s1 = snap(s1, 63.0f, 1.0f / 63.0f); s2 = snap(s2, 31.0f, 1.0f / 31.0f);
     e0 = snap(e0, 31.0f, 1.0f / 31.0f); e1 = snap(e1, 63.0f, 1.0f / 63.0f); e2 = snap(e2, 31.0f, 1.0f / 31.0f);
 
-    // range.rs:104-141 for the 3-colour pass (BC1) and the 4-colour pass
-    // (unless BC1 with transparent pixels) in one loop over the pixels: the
+    // range.rs:104-141 for the 3-colour pass (BC1) and the 4-colour pass (not
+    // used for BC1 with transparent pixels) in one loop over the pixels: the
     // two codebooks share codes 0 and 1 (the snapped start and end), so each
     // pixel's distances to them are computed once and serve both passes.
     // Each pass keeps its own first strict minimum per pixel (codes in
@@ -416,10 +403,10 @@ __device__ __forceinline__ void range_fit_lane(const LaneSet& S, const LaneTable
     };
     float error3 = 0.0f, error4 = 0.0f;
     uint32_t idx3 = 0, idx4 = 0;
-#pragma unroll 2
+#pragma unroll
     for (int p = 0; p < 16; ++p) {
         float x, y, z;
-        xyz(T, S.pix(p), x, y, z);
+        rgb_point(pix[p], x, y, z);
         const float d0 = dist_to(x, y, z, s0, s1, s2);
         const float d1 = dist_to(x, y, z, e0, e1, e2);
         // codes 0 and 1: the first strict minimum starts from FLT_MAX
@@ -440,9 +427,9 @@ __device__ __forceinline__ void range_fit_lane(const LaneSet& S, const LaneTable
                 k = 2;
             }
             idx3 |= (in ? k : 3u) << (2 * p);
-            if (pt) error3 += dist;
+            error3 = pt ? error3 + dist : error3;
         }
-        if (do4) {
+        {
             float dist = m01;
             uint32_t k = k01;
             const float d2 = dist_to(x, y, z, f0, f1, f2);
@@ -456,7 +443,7 @@ __device__ __forceinline__ void range_fit_lane(const LaneSet& S, const LaneTable
                 k = 3;
             }
             idx4 |= (in ? k : 3u) << (2 * p);
-            if (pt) error4 += dist;
+            error4 = pt ? error4 + dist : error4;
         }
     }
     float best = FLT_MAX;
@@ -504,9 +491,16 @@ __device__ __forceinline__ int encode_front_lane(const uint32_t (&px)[16], uint3
     const int kind = S.n == 1 ? KIND_SINGLE : (ALG == RANGE_FIT || S.n == 0) ? KIND_RANGE : KIND_CLUSTER;
     uint32_t lo = 0, hi = 0;
     vx = vy = vz = 0.0f;
-    if (kind == KIND_SINGLE) single_fit_lane<FMT>(S, T, lo, hi);
-    if (kind != KIND_SINGLE) principal_axis_lane(S, T, vx, vy, vz, kind == KIND_CLUSTER ? cluster_pts : nullptr);
-    if (kind == KIND_RANGE) range_fit_lane<FMT>(S, T, fp, vx, vy, vz, lo, hi);
+    if (kind == KIND_SINGLE) single_fit_lane<FMT>(S, lo, hi);
+    if (ALG == RANGE_FIT) {
+        if (kind == KIND_RANGE) {
+            principal_axis_lane(S, px, vx, vy, vz);
+            range_fit_lane<FMT>(S, px, fp, vx, vy, vz, lo, hi);
+        }
+    } else {
+        if (kind == KIND_CLUSTER) principal_axis_lane(S, px, vx, vy, vz, cluster_pts);
+        if (kind == KIND_RANGE) empty_fit<FMT>(lo, hi);
+    }
     set_colour<FMT>(out, lo, hi);
     return kind;
 }
