@@ -1,8 +1,7 @@
 """compress_mips_device encodes the levels of a chain in one launch: every
 level must equal the same level compressed alone, for every format and
 algorithm, on the direct kernels and through the pipeline, for chains of one
-level, of sides of 1, of ragged levels, cut short, and where the lane kernels
-start."""
+level, of sides of 1, of ragged levels and cut short."""
 import numpy as np
 import pytest
 
@@ -43,14 +42,3 @@ def test_chain_equals_its_levels(gpu, oracle, fmt, alg, threshold):
             np.testing.assert_array_equal(got, np.concatenate(want), err_msg=str((w, h, levels)))
     finally:
         tx.set_pipeline_threshold(old)
-
-
-def test_range_fit_chain_on_the_lane_kernel(gpu, oracle):
-    # 12,288 blocks and more take one block per lane
-    w, h = 451, 440
-    img = texgen.with_alpha_field(texgen.rgb_texture(w, h, 3), 3)
-    p = tx.Params(tx.Algorithm.RangeFit)
-    got = chain_bytes(tx.Format.Bc3, img, tx.mip_levels(w, h), p)
-    op = oracle.params(0, p.weights, False)
-    want = [oracle.compress(2, lv, lv.shape[1], lv.shape[0], op, threads=8) for lv in texgen.mip_chain(img)]
-    np.testing.assert_array_equal(got, np.concatenate(want))

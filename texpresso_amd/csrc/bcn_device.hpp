@@ -358,9 +358,12 @@ __device__ __forceinline__ void principal_axis(const LDS& L, int n, float& vx, f
     }
 }
 
-// single.rs:58-98 for one codebook; returns the winning error
-__device__ __forceinline__ uint32_t single_endpoints(int tr, int tg, int cr, int cg, int cb, float (&s)[3],
-                                                     float (&e)[3], uint32_t& index)
+// single.rs:58-98 for one codebook; returns the winning error.  The table's
+// endpoints are levels of the 565 grid: the reference divides them by 31 / 63
+// and packs round(31 * (v / 31)) (63 * (v / 63)), which is v again for every
+// level, so they are packed as they are.
+__device__ __forceinline__ uint32_t single_endpoints(int tr, int tg, int cr, int cg, int cb, uint32_t& start,
+                                                     uint32_t& end, uint32_t& index)
 {
     uint32_t best = 0xFFFFFFFFu;
 #pragma unroll
@@ -371,8 +374,8 @@ __device__ __forceinline__ uint32_t single_endpoints(int tr, int tg, int cr, int
         const uint32_t er = r[2], eg = g[2], eb = b[2];
         const uint32_t err = er * er + eg * eg + eb * eb;
         if (err < best) {
-            s[0] = (float)r[0] / 31.0f; s[1] = (float)g[0] / 63.0f; s[2] = (float)b[0] / 31.0f;
-            e[0] = (float)r[1] / 31.0f; e[1] = (float)g[1] / 63.0f; e[2] = (float)b[1] / 31.0f;
+            start = ((uint32_t)r[0] << 11) | ((uint32_t)g[0] << 5) | (uint32_t)b[0];
+            end = ((uint32_t)r[1] << 11) | ((uint32_t)g[1] << 5) | (uint32_t)b[1];
             index = (uint32_t)(2 * k);
             best = err;
         }
@@ -389,18 +392,17 @@ __device__ __forceinline__ void single_fit(const LDS& L, const ColourSet& cs, in
     const int cg = f32_to_i32_clamped(q.y * 255.0f, 255);
     const int cb = f32_to_i32_clamped(q.z * 255.0f, 255);
     uint32_t best = 0xFFFFFFFFu;
-    float s[3], e[3];
-    uint32_t index = 0;
+    uint32_t s = 0, e = 0, index = 0;
     if (FMT == BC1) {
         const uint32_t err = single_endpoints(0, 1, cr, cg, cb, s, e, index);
         if (err < best) {
-            write_colour(false, s[0], s[1], s[2], e[0], e[1], e[2], cs.remap < 0 ? 3u : index, l, lo, hi);
+            write_packed(false, s, e, cs.remap < 0 ? 3u : index, l, lo, hi);
             best = err;
         }
     }
     if (FMT != BC1 || !cs.transparent) {
         const uint32_t err = single_endpoints(2, 3, cr, cg, cb, s, e, index);
-        if (err < best) write_colour(true, s[0], s[1], s[2], e[0], e[1], e[2], cs.remap < 0 ? 3u : index, l, lo, hi);
+        if (err < best) write_packed(true, s, e, cs.remap < 0 ? 3u : index, l, lo, hi);
     }
 }
 

@@ -113,10 +113,13 @@ __global__ __launch_bounds__(256) void k_encode_alpha_chain(txk::ChainTable chai
 
 // RangeFit (BC1/BC2/BC3): one block per lane, the front of the pipeline's
 // classify pass (alpha, colour set, principal axis, then the single-colour or
-// range fit) without its record path.  A RangeFit block is a few hundred
-// serial operations; on a 16-lane group every fold would run on all 16 lanes.
-// Single-wave workgroups (the per-wave LDS copies of the block pixels and
-// weights), one per 64-block span of the image.
+// range fit) without its record path.  A RangeFit block is a few thousand
+// mostly serial operations; on a 16-lane group every fold would run on all 16
+// lanes (measured, BC1: 10.0 us against 9.0 at 256 blocks, 12.0 / 9.1 at 4096,
+// 18.3 / 9.2 at 16384).  Single-wave workgroups (the wave's LDS copies of the
+// block pixels and weights): of four waves they were 3-5 % faster where the
+// blocks fill whole rounds of the GPU (2048^2 23.6 -> 22.8 us) and 3 % slower
+// between (344,000 blocks 31.1 -> 32.0 us).
 template <int FMT>
 __device__ __forceinline__ void encode_range_lanes(const Image& im, uint32_t group, const FitParams& fp,
                                                    LaneTables& LT, LaneBlockLds& LB)
@@ -422,7 +425,6 @@ namespace {
 // 12544, 190 / 170 / 190 and 197 / 169 / 168 at 16384.
 int team_groups(int algorithm, uint64_t nblocks)
 {
-    if (algorithm == 0) return 1;  // RangeFit: no search
     const bool iterative = algorithm == 2;
     if (nblocks <= (iterative ? 10240u : 2560u)) return 4;
     return nblocks <= (iterative ? 32768u : 6144u) ? 2 : 1;
@@ -462,44 +464,33 @@ hipError_t launch_encode_n(const txk::EncodeArgs& a, txk::ChainTable* chain, hip
 template <int FMT, int ALG>
 hipError_t launch_encode_t(const txk::EncodeArgs& a, txk::ChainTable* chain, hipStream_t s)
 {
-    if constexpr (ALG != 0) {
-        const int t = team_groups(ALG, a.nblocks);
-        if (t == 4) return launch_encode_n<FMT, ALG, 4>(a, chain, s);
-        if (t == 2) return launch_encode_n<FMT, ALG, 2>(a, chain, s);
+    switch (team_groups(ALG, a.nblocks)) {
+    case 4: return launch_encode_n<FMT, ALG, 4>(a, chain, s);
+    case 2: return launch_encode_n<FMT, ALG, 2>(a, chain, s);
+    default: return launch_encode_n<FMT, ALG, 1>(a, chain, s);
     }
-    return launch_encode_n<FMT, ALG, 1>(a, chain, s);
 }
 
 template <int FMT>
 hipError_t launch_encode_range(const txk::EncodeArgs& a, txk::ChainTable* chain, hipStream_t s)
 {
     hipError_t e;
-    const uint64_t waves = groups_for(a, chain, 64, e);
-    if (waves == 0) return e;
+    const uint64_t groups = groups_for(a, chain, 64, e);
+    if (groups == 0) return e;
     if (chain)
-        hipLaunchKernelGGL((txd::k_encode_range_chain<FMT>), txk::grid_2d(waves), dim3(64), 0, s, *chain, a.out,
+        hipLaunchKernelGGL((txd::k_encode_range_chain<FMT>), txk::grid_2d(groups), dim3(64), 0, s, *chain, a.out,
                            fit_of(a));
     else
-        hipLaunchKernelGGL((txd::k_encode_range_lane<FMT>), txk::grid_2d(waves), dim3(64), 0, s, image_of(a),
+        hipLaunchKernelGGL((txd::k_encode_range_lane<FMT>), txk::grid_2d(groups), dim3(64), 0, s, image_of(a),
                            fit_of(a));
     return hipGetLastError();
 }
-
-// RangeFit textures of at least this many blocks take the one-block-per-lane
-// kernel, smaller ones the 16-lane-group kernel: a lane-per-block wave costs
-// one block's serial latency (~17 us on MI355X however few blocks it has),
-// while the group kernel spreads a block over 16 lanes (measured per level
-// of a 4096^2 chain, BC1: 11.6 vs 17.1 us at 4096 blocks, 18.5 vs 16.8 us
-// at 16384, 166 vs 33 us at 262144).
-constexpr uint64_t kRangeLaneMinBlocks = 12288;
 
 template <int FMT>
 hipError_t launch_encode_f(const txk::EncodeArgs& a, txk::ChainTable* chain, hipStream_t s)
 {
     switch (a.algorithm) {
-    case 0:
-        return a.nblocks >= kRangeLaneMinBlocks ? launch_encode_range<FMT>(a, chain, s)
-                                                : launch_encode_t<FMT, 0>(a, chain, s);
+    case 0: return launch_encode_range<FMT>(a, chain, s);
     case 1: return launch_encode_t<FMT, 1>(a, chain, s);
     default: return launch_encode_t<FMT, 2>(a, chain, s);
     }

@@ -288,10 +288,9 @@ __device__ __forceinline__ void principal_axis_lane(const LaneSet& S, const uint
 
 // colourblock.rs:58-94 with all 16 indices on one lane (pixel p in bits
 // 2p..2p+1 of `idx`).
-__device__ __forceinline__ void write_colour_lane(bool four, float sx, float sy, float sz, float ex, float ey, float ez,
-                                                  uint32_t idx, uint32_t& lo, uint32_t& hi)
+__device__ __forceinline__ void write_packed_lane(bool four, uint32_t a, uint32_t b, uint32_t idx, uint32_t& lo,
+                                                  uint32_t& hi)
 {
-    uint32_t a = pack_565(sx, sy, sz), b = pack_565(ex, ey, ez);
     if (!four) {
         if (a > b) {  // write3: a <= b, swap palette slots 0 and 1
             const uint32_t t = a; a = b; b = t;
@@ -318,35 +317,27 @@ __device__ __forceinline__ uint32_t spread_index(uint32_t inc, uint32_t in)
     return ((in * 0x55555555u) & m2) | (0xFFFFFFFFu & ~m2);
 }
 
-// Colour of point 0 (the lowest pixel that opens a point).
-__device__ __forceinline__ void point0_lane(const LaneSet& S, float& qx, float& qy, float& qz)
-{
-    rgb_point(S.pix(S.first ? __builtin_ctz(S.first) : 0), qx, qy, qz);
-}
-
 // single.rs:100-164 (same steps as single_fit)
 template <int FMT>
 __device__ __forceinline__ void single_fit_lane(const LaneSet& S, uint32_t& lo, uint32_t& hi)
 {
-    float qx, qy, qz;
-    point0_lane(S, qx, qy, qz);
-    const int cr = f32_to_i32_clamped(qx * 255.0f, 255);
-    const int cg = f32_to_i32_clamped(qy * 255.0f, 255);
-    const int cb = f32_to_i32_clamped(qz * 255.0f, 255);
+    // point 0 is the lowest pixel that opens a point; round(255 * (u / 255)) is
+    // the byte u again
+    const uint32_t q = S.pix(__builtin_ctz(S.first));
+    const int cr = (int)(q & 255u), cg = (int)((q >> 8) & 255u), cb = (int)((q >> 16) & 255u);
     uint32_t best = 0xFFFFFFFFu;
-    float s[3], e[3];
-    uint32_t index = 0;
+    uint32_t s = 0, e = 0, index = 0;
     if (FMT == BC1) {
         const uint32_t err = single_endpoints(0, 1, cr, cg, cb, s, e, index);
         if (err < best) {
-            write_colour_lane(false, s[0], s[1], s[2], e[0], e[1], e[2], spread_index(S.inc, index), lo, hi);
+            write_packed_lane(false, s, e, spread_index(S.inc, index), lo, hi);
             best = err;
         }
     }
     if (FMT != BC1 || !S.transparent) {
         const uint32_t err = single_endpoints(2, 3, cr, cg, cb, s, e, index);
         if (err < best)
-            write_colour_lane(true, s[0], s[1], s[2], e[0], e[1], e[2], spread_index(S.inc, index), lo, hi);
+            write_packed_lane(true, s, e, spread_index(S.inc, index), lo, hi);
     }
 }
 
@@ -446,12 +437,13 @@ __device__ __forceinline__ void range_fit_lane(const LaneSet& S, const uint32_t 
             error4 = pt ? error4 + dist : error4;
         }
     }
+    const uint32_t a = pack_565(s0, s1, s2), b = pack_565(e0, e1, e2);
     float best = FLT_MAX;
     if (do3 && error3 < best) {
-        write_colour_lane(false, s0, s1, s2, e0, e1, e2, idx3, lo, hi);
+        write_packed_lane(false, a, b, idx3, lo, hi);
         best = error3;
     }
-    if (do4 && error4 < best) write_colour_lane(true, s0, s1, s2, e0, e1, e2, idx4, lo, hi);
+    if (do4 && error4 < best) write_packed_lane(true, a, b, idx4, lo, hi);
 }
 
 // BC2 alpha of one lane's block (alpha.rs:27-51, same steps as bc2_alpha).
@@ -481,12 +473,11 @@ __device__ __forceinline__ int encode_front_lane(const uint32_t (&px)[16], uint3
     out[0] = out[1] = out[2] = out[3] = 0;
     colour_set_lane<FMT>(px, valid, fp, T, L, lane, S);
     if (FMT == BC2) bc2_alpha_lane(px, valid, out[0], out[1]);
-    // BC3 alpha from the pixel copies in LDS, loops rolled (the unrolled
-    // 16 x 8 codebook search would need many more registers)
+    // BC3 alpha from the pixel registers; a block with masked pixels (the last
+    // row and column of an image) takes the rolled form over the LDS copies
     if (FMT == BC3) {
-        auto alpha = [&](int p) { return (int)(S.pix(p) >> 24); };
-        if (valid == 0xFFFFu) bc3_alpha_full<1>(alpha, out[0], out[1]);
-        else bc3_alpha_core<1>(alpha, valid, out[0], out[1]);
+        if (valid == 0xFFFFu) bc3_alpha_full<16>([&](int p) { return (int)(px[p] >> 24); }, out[0], out[1]);
+        else bc3_alpha_core<1>([&](int p) { return (int)(S.pix(p) >> 24); }, valid, out[0], out[1]);
     }
     const int kind = S.n == 1 ? KIND_SINGLE : (ALG == RANGE_FIT || S.n == 0) ? KIND_RANGE : KIND_CLUSTER;
     uint32_t lo = 0, hi = 0;
