@@ -41,7 +41,7 @@ struct LaneSet {
     int lane;
     uint32_t first;     // bit p: pixel p opens a point
     uint32_t inc;       // bit p: pixel p is in the set
-    uint32_t remap[4];  // one byte per pixel: point index, 255 = excluded
+    uint64_t lowest;    // nibble p: the lowest pixel of pixel p's colour
     int n;
     bool transparent;
 
@@ -115,8 +115,8 @@ __device__ __forceinline__ void sort16(uint32_t (&k)[16])
 // pixel first.  The run's first pixel opens the colour's point when it is in
 // the set (it is the lowest pixel of that colour); every pixel of the run has
 // it as its lowest same-colour pixel; the point's weight is sqrtf(run
-// length).  Same sets, remaps and weights as the pairwise compares of the
-// weighted form below.
+// length).  Same sets and weights as the pairwise compares of the weighted
+// form below.
 template <int FMT>
 __device__ __forceinline__ void colour_set_lane_sorted(const uint32_t (&px)[16], uint32_t inc, const LaneTables& T,
                                                        LaneBlockLds& L, int lane, LaneSet& S)
@@ -126,7 +126,7 @@ __device__ __forceinline__ void colour_set_lane_sorted(const uint32_t (&px)[16],
     for (int p = 0; p < 16; ++p) k[p] = (colour_key(px[p], inc, p) << 4) | (uint32_t)p;
     sort16(k);
     uint32_t first = 0, head = 0, cnt = 0;
-    uint64_t lowest = 0;  // nibble p: the lowest pixel of pixel p's colour
+    uint64_t lowest = 0;
 #pragma unroll
     for (int s = 0; s < 16; ++s) {
         const uint32_t i = k[s] & 15u;
@@ -142,28 +142,15 @@ __device__ __forceinline__ void colour_set_lane_sorted(const uint32_t (&px)[16],
         L.w[i][lane] = start && in ? T.sqc[1] : 0.0f;
         if (!start) L.w[head][lane] = T.sqc[cnt];
     }
-    uint64_t remap = 0;
-#pragma unroll
-    for (int p = 0; p < 16; ++p) {
-        const uint32_t f = (uint32_t)(lowest >> (4 * p)) & 15u;
-        const uint64_t r = ((inc >> p) & 1u) ? (uint64_t)__popc(first & ((1u << f) - 1u)) : 255u;
-        remap |= r << (8 * (p & 7));
-        if (p == 7) {
-            S.remap[0] = (uint32_t)remap;
-            S.remap[1] = (uint32_t)(remap >> 32);
-            remap = 0;
-        }
-    }
-    S.remap[2] = (uint32_t)remap;
-    S.remap[3] = (uint32_t)(remap >> 32);
+    S.lowest = lowest;
     S.first = first;
     S.n = __popc(first);
 }
 
 // colourset.rs:35-112 on one lane.  For each pixel p, same = the pixels with
-// p's colour (p included): p opens a point when none of them is lower; its
-// point index counts the points opened below its lowest same-colour pixel;
-// the point's weight is the pixel count, or the sum of (alpha + 1) / 256
+// p's colour (p included): p opens a point when none of them is lower (a
+// pixel's point index counts the points opened below its lowest same-colour
+// pixel); the point's weight is the pixel count, or the sum of (alpha + 1) / 256
 // over those pixels (exact in binary32), then sqrtf.  Unweighted points take
 // the sorted form above.
 template <int FMT>
@@ -188,7 +175,7 @@ __device__ __forceinline__ void colour_set_lane(const uint32_t (&px)[16], uint32
         return;
     }
     uint32_t first = 0;
-    uint64_t remap = 0;
+    uint64_t lowest = 0;
     uint32_t keys[16];
 #pragma unroll
     for (int m = 0; m < 16; ++m) keys[m] = colour_key(px[m], inc, m);
@@ -213,20 +200,12 @@ __device__ __forceinline__ void colour_set_lane(const uint32_t (&px)[16], uint32
         const bool in = (inc >> p) & 1u;
         const bool opens = in && (same & ((1u << p) - 1u)) == 0u;
         first |= (opens ? 1u : 0u) << p;
-        const uint32_t f = (uint32_t)__builtin_ctz(same);  // lowest pixel of p's colour
-        const uint64_t r = in ? (uint64_t)__popc(first & ((1u << f) - 1u)) : 255u;
-        remap |= r << (8 * (p & 7));
-        if (p == 7) {
-            S.remap[0] = (uint32_t)remap;
-            S.remap[1] = (uint32_t)(remap >> 32);
-            remap = 0;
-        }
+        lowest |= (uint64_t)__builtin_ctz(same) << (4 * p);
         float w = 0.0f;
         if (opens) w = fp.weigh_alpha ? sqrtf((float)asum / 256.0f) : T.sqc[__popc(same)];
         L.w[p][lane] = w;
     }
-    S.remap[2] = (uint32_t)remap;
-    S.remap[3] = (uint32_t)(remap >> 32);
+    S.lowest = lowest;
     S.first = first;
     S.n = __popc(first);
 }
@@ -236,11 +215,9 @@ __device__ __forceinline__ void colour_set_lane(const uint32_t (&px)[16], uint32
 // colours converted from the pixel registers (a rolled loop over LDS copies
 // waits out two LDS reads per step, most of its time): a pixel that opens no
 // point has w = 0, so its terms are +0 or -0 and adding them leaves the
-// (never negative-zero) accumulators unchanged.  With `pts`, the first fold
-// also stores each point as (x, y, z, weight) at its point index there (the
-// ClusterFit record of the block).
+// (never negative-zero) accumulators unchanged.
 __device__ __forceinline__ void principal_axis_lane(const LaneSet& S, const uint32_t (&px)[16], float& vx, float& vy,
-                                                    float& vz, float4* __restrict__ pts = nullptr)
+                                                    float& vz)
 {
     float total = 0.0f, cx = 0.0f, cy = 0.0f, cz = 0.0f;
 #pragma unroll
@@ -248,7 +225,6 @@ __device__ __forceinline__ void principal_axis_lane(const LaneSet& S, const uint
         float x, y, z;
         rgb_point(px[p], x, y, z);
         const float w = S.wt(p);
-        if (pts && ((S.first >> p) & 1u)) pts[__popc(S.first & ((1u << p) - 1u))] = make_float4(x, y, z, w);
         total = total + w;
         cx = cx + x * w;
         cy = cy + y * w;
@@ -467,8 +443,7 @@ __device__ __forceinline__ void bc2_alpha_lane(const uint32_t (&px)[16], uint32_
 template <int FMT, int ALG>
 __device__ __forceinline__ int encode_front_lane(const uint32_t (&px)[16], uint32_t valid, const FitParams& fp,
                                                  const LaneTables& T, LaneBlockLds& L, int lane, uint32_t (&out)[4],
-                                                 LaneSet& S, float& vx, float& vy, float& vz,
-                                                 float4* __restrict__ cluster_pts = nullptr)
+                                                 LaneSet& S, float& vx, float& vy, float& vz)
 {
     out[0] = out[1] = out[2] = out[3] = 0;
     colour_set_lane<FMT>(px, valid, fp, T, L, lane, S);
@@ -489,7 +464,7 @@ __device__ __forceinline__ int encode_front_lane(const uint32_t (&px)[16], uint3
             range_fit_lane<FMT>(S, px, fp, vx, vy, vz, lo, hi);
         }
     } else {
-        if (kind == KIND_CLUSTER) principal_axis_lane(S, px, vx, vy, vz, cluster_pts);
+        if (kind == KIND_CLUSTER) principal_axis_lane(S, px, vx, vy, vz);
         if (kind == KIND_RANGE) empty_fit<FMT>(lo, hi);
     }
     set_colour<FMT>(out, lo, hi);

@@ -86,24 +86,26 @@ __device__ __forceinline__ void count_keys(PipeCtl* __restrict__ ctl, uint32_t k
     }
 }
 
-// ClusterFit block on one lane: the rest of its record in slot r (the points
-// were written by the front's centroid fold), and its key.
+// ClusterFit block on one lane: its record in slot r, and its key.
 template <int FMT, int ALG>
 __device__ __forceinline__ uint32_t write_record_lane(ClusterRec* __restrict__ recs, uint32_t r,
                                                       const LaneSet& S, const uint32_t (&out)[4],
-                                                      float vx, float vy, float vz, const FitParams& fp,
-                                                      uint32_t tex_idx, uint32_t block)
+                                                      float vx, float vy, float vz, const FitParams& fp, uint32_t tex_idx, uint32_t block)
 {
-    ClusterRec& R = recs[r];  // points: written by the front's centroid fold
     const bool need4 = !(FMT == BC1 && S.transparent);
     const uint32_t info = (uint32_t)S.n | ((S.transparent ? 1u : 0u) << 8) | ((uint32_t)FMT << 12) |
                           ((ALG == ITERATIVE_CLUSTER_FIT ? 8u : 1u) << 16);
-    uint4* tail = reinterpret_cast<uint4*>(R.remap);
-    tail[0] = make_uint4(S.remap[0], S.remap[1], S.remap[2], S.remap[3]);
-    tail[1] = make_uint4(out[0], out[1], __float_as_uint(vx), __float_as_uint(vy));
-    tail[2] = make_uint4(__float_as_uint(vz), __float_as_uint(FLT_MAX), 0u, 0u);
-    tail[3] = make_uint4(__float_as_uint(fp.wr), __float_as_uint(fp.wg), __float_as_uint(fp.wb), tex_idx);
-    tail[4] = make_uint4(block, info, 0u, 0u);
+    uint4* const q = reinterpret_cast<uint4*>(recs + r);
+#pragma unroll
+    for (int p = 0; p < 16; p += 4) q[p / 4] = make_uint4(S.pix(p), S.pix(p + 1), S.pix(p + 2), S.pix(p + 3));
+#pragma unroll
+    for (int p = 0; p < 16; p += 4)
+        q[4 + p / 4] = make_uint4(__float_as_uint(S.wt(p)), __float_as_uint(S.wt(p + 1)), __float_as_uint(S.wt(p + 2)),
+                                  __float_as_uint(S.wt(p + 3)));
+    q[8] = make_uint4((uint32_t)S.lowest, (uint32_t)(S.lowest >> 32), S.first | (S.inc << 16), info);
+    q[9] = make_uint4(out[0], out[1], __float_as_uint(vx), __float_as_uint(vy));
+    q[10] = make_uint4(__float_as_uint(vz), __float_as_uint(FLT_MAX), __float_as_uint(fp.wr), __float_as_uint(fp.wg));
+    q[11] = make_uint4(__float_as_uint(fp.wb), tex_idx, block, 0u);
     // ClusterFit: list C (all of the block's searches in one pass);
     // IterativeClusterFit: the 3-colour search for BC1 (list A) and the
     // 4-colour one unless transparent (list B)
@@ -144,8 +146,7 @@ __device__ __forceinline__ void classify_chunk(const Grid& G, const BatchTex& T,
             uint32_t w[4];
             LaneSet S;
             float vx, vy, vz;
-            const int kind = encode_front_lane<FMT, ALG>(px, valid, fp, LT, LB, lane, w, S, vx, vy, vz,
-                                                         recs[slot0 + k].pts);
+            const int kind = encode_front_lane<FMT, ALG>(px, valid, fp, LT, LB, lane, w, S, vx, vy, vz);
             if (kind == KIND_CLUSTER) {
                 key = write_record_lane<FMT, ALG>(recs, slot0 + k, S, w, vx, vy, vz, fp, tex_idx, block0 + b);
             } else if (FMT == BC1) {
@@ -281,12 +282,27 @@ __global__ __launch_bounds__(256) void k_pipe_bin(const uint32_t* __restrict__ k
     }
 }
 
+// The block of record R into its group's LDS: lane l writes the point that
+// pixel l opens, if it does (colourset.rs:45-97 in pixel order).  Returns the
+// pixel's point index, -1 when it is excluded.
+__device__ __forceinline__ int load_points(const ClusterRec& R, GroupLds& L, int l)
+{
+    const uint32_t first = R.masks & 0xFFFFu, inc = R.masks >> 16;
+    if ((first >> l) & 1u) {
+        float x, y, z;
+        rgb_point(R.px[l], x, y, z);
+        L.pts[__popc(first & ((1u << l) - 1u))] = make_float4(x, y, z, R.wt[l]);
+    }
+    const uint32_t low = (R.lowest[l >> 3] >> (4 * (l & 7))) & 15u;
+    return (inc >> l) & 1u ? __popc(first & ((1u << low) - 1u)) : -1;
+}
+
 // A searched block's state that the split loops do not read, in GroupLds::keep
 // (the loops hold most of the 128 registers of a lane): its output fields,
 // read with the rest of the record when the group takes it (not behind a load
 // at emit time), its record slot, and three words that hold the principal axis
 // until the first ordering is built, then the best split's endpoints and key.
-enum { kKeepTex = 0, kKeepBlock = 1, kKeepAlpha = 2, kKeepRec = 4, kKeepAxis = 5, kKeepEnds = 5, kKeepKey = 7 };
+enum { kKeepTex = 0, kKeepBlock = 1, kKeepHalf = 2, kKeepRec = 4, kKeepAxis = 5, kKeepEnds = 5, kKeepKey = 7 };
 
 // Result of a finished block: the output block, or (NC = 3 for an opaque BC1
 // block) the 3-colour result kept in the record for the 4-colour pass.
@@ -298,13 +314,12 @@ __device__ __forceinline__ void emit_block(const BatchTex* __restrict__ tex, con
     const uint32_t fmt = (info >> 12) & 15u;
     uint32_t lo = 0, hi = 0;
     const bool won = lb_err < thr;
-    ClusterRec& R = recs[L.keep[kKeepRec]];
     if (won) {
         write_packed(NC == 4, L.keep[kKeepEnds], L.keep[kKeepEnds + 1],
                      split_index<NC>(L, n, remap, L.keep[kKeepKey], lb_it), l, lo, hi);
     } else if (NC == 4 && fmt == BC1) {
-        lo = R.fit3[0];
-        hi = R.fit3[1];
+        lo = L.keep[kKeepHalf];  // compress3's block
+        hi = L.keep[kKeepHalf + 1];
     }
     if (l == 0) {
         uint8_t* const out = tex_at(tex, tex0, L.keep[kKeepTex]).out;
@@ -313,15 +328,16 @@ __device__ __forceinline__ void emit_block(const BatchTex* __restrict__ tex, con
             if ((info >> 8) & 1u) {
                 *reinterpret_cast<uint2*>(out + block * 8u) = make_uint2(lo, hi);
             } else {
+                ClusterRec& R = recs[L.keep[kKeepRec]];
                 R.fit3_err = won ? lb_err : thr;
-                R.fit3[0] = lo;
-                R.fit3[1] = hi;
+                R.half[0] = lo;
+                R.half[1] = hi;
             }
         } else if (fmt == BC1) {
             *reinterpret_cast<uint2*>(out + block * 8u) = make_uint2(lo, hi);
         } else {
             *reinterpret_cast<uint4*>(out + block * 16u) =
-                make_uint4(L.keep[kKeepAlpha], L.keep[kKeepAlpha + 1], lo, hi);
+                make_uint4(L.keep[kKeepHalf], L.keep[kKeepHalf + 1], lo, hi);
         }
     }
 }
@@ -445,10 +461,8 @@ __global__ __launch_bounds__(64 * kSearchWaves) __attribute__((amdgpu_waves_per_
                     } else {
                         const uint32_t r = list[p];
                         const ClusterRec& R = recs[r];
-                        L.pts[l] = R.pts[l];
+                        remap = load_points(R, L, l);
                         info = R.info;
-                        const uint32_t byte = (R.remap[l >> 2] >> (8 * (l & 3))) & 255u;
-                        remap = byte == 255u ? -1 : (int)byte;
                         fp = FitParams{R.w[0], R.w[1], R.w[2], 0u};
                         thr = NC == 4 ? R.fit3_err : FLT_MAX;
                         lb_err = thr;
@@ -456,7 +470,7 @@ __global__ __launch_bounds__(64 * kSearchWaves) __attribute__((amdgpu_waves_per_
                         it = 0;
                         if (l == 0) {
                             uint4* const keep = reinterpret_cast<uint4*>(L.keep);
-                            keep[0] = make_uint4(R.tex, R.block, R.alpha[0], R.alpha[1]);
+                            keep[0] = make_uint4(R.tex, R.block, R.half[0], R.half[1]);
                             keep[1] = make_uint4(r, __float_as_uint(R.axis[0]), __float_as_uint(R.axis[1]),
                                                  __float_as_uint(R.axis[2]));
                         }
@@ -562,18 +576,16 @@ __global__ __launch_bounds__(64 * kSearchWaves) __attribute__((amdgpu_waves_per_
         uint32_t fmt = BC1;
         if (has) {
             const ClusterRec& R = recs[list[p]];
-            L.pts[l] = R.pts[l];
+            cs.remap = load_points(R, L, l);
             const uint32_t info = R.info;
             fmt = (info >> 12) & 15u;
             cs.n = (int)(info & 31u);
             cs.transparent = ((info >> 8) & 1u) != 0u;
-            const uint32_t byte = (R.remap[l >> 2] >> (8 * (l & 3))) & 255u;
-            cs.remap = byte == 255u ? -1 : (int)byte;
             fp = FitParams{R.w[0], R.w[1], R.w[2], 0u};
             axx = R.axis[0];
             axy = R.axis[1];
             axz = R.axis[2];
-            if (l == 0) *reinterpret_cast<uint4*>(L.keep) = make_uint4(R.tex, R.block, R.alpha[0], R.alpha[1]);
+            if (l == 0) *reinterpret_cast<uint4*>(L.keep) = make_uint4(R.tex, R.block, R.half[0], R.half[1]);
         }
         group_sync();
         float best = FLT_MAX;

@@ -26,27 +26,29 @@
 
 namespace txp {
 
-// One ClusterFit block between the passes (336 bytes).
-struct __align__(16) ClusterRec {
-    float4 pts[16];     // distinct colours: x, y, z, sqrt(weight)
-    uint32_t remap[4];  // one byte per pixel: point index, 255 = excluded
-    uint32_t alpha[2];  // alpha half of the block (BC2/BC3)
-    float axis[3];      // principal axis
-    float fit3_err;     // 3-colour result: ClusterFit::best_error after compress3
-    uint32_t fit3[2];   // 3-colour result: ClusterFit::best_compressed after compress3
-    float w[3];         // Params::weights
-    uint32_t tex;       // texture index
-    uint32_t block;     // block index within the texture
-    uint32_t info;      // n | transparent << 8 | format << 12 | iterations << 16
-    uint32_t pad[2];
+// One ClusterFit block between the passes: three 64-byte pieces, written whole
+// by the classify lane that owns the block.  The points stay in pixel order
+// as classify holds them; the search's lane l turns pixel l into its point.
+struct __align__(64) ClusterRec {
+    uint32_t px[16];     // the block's RGBA8 pixels
+    float wt[16];        // sqrt(weight) of the point a pixel opens, 0 for the others
+    uint32_t lowest[2];  // nibble p: the lowest pixel of pixel p's colour
+    uint32_t masks;      // pixels that open a point | pixels of the set << 16
+    uint32_t info;       // n | transparent << 8 | format << 12 | iterations << 16
+    uint32_t half[2];    // BC2/BC3: alpha half of the block; BC1: ClusterFit::best_compressed after compress3
+    float axis[3];       // principal axis
+    float fit3_err;      // ClusterFit::best_error after compress3
+    float w[3];          // Params::weights
+    uint32_t tex;        // texture index
+    uint32_t block;      // block index within the texture (or through the chain)
+    uint32_t pad;
 };
-static_assert(sizeof(ClusterRec) == 336, "record layout");
-// the classify pass stores the tail as five 16-byte words starting at remap
-static_assert(offsetof(ClusterRec, remap) == 256 && offsetof(ClusterRec, alpha) == 272 &&
-                  offsetof(ClusterRec, axis) == 280 && offsetof(ClusterRec, fit3_err) == 292 &&
-                  offsetof(ClusterRec, fit3) == 296 && offsetof(ClusterRec, w) == 304 &&
-                  offsetof(ClusterRec, tex) == 316 && offsetof(ClusterRec, block) == 320 &&
-                  offsetof(ClusterRec, info) == 324,
+static_assert(sizeof(ClusterRec) == 192, "record layout");
+// the classify pass stores the tail as four 16-byte words starting at lowest
+static_assert(offsetof(ClusterRec, lowest) == 128 && offsetof(ClusterRec, half) == 144 &&
+                  offsetof(ClusterRec, axis) == 152 && offsetof(ClusterRec, fit3_err) == 164 &&
+                  offsetof(ClusterRec, w) == 168 && offsetof(ClusterRec, tex) == 180 &&
+                  offsetof(ClusterRec, block) == 184,
               "record tail layout");
 
 // Counters of one pipeline run (cleared by the reset kernel).  Every update

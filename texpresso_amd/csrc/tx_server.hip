@@ -121,7 +121,7 @@ struct Launch {
 };
 
 // Largest number of BC1-BC3 blocks a launch sends through the binned
-// pipeline (records: 336 bytes each, so 1.4 GB per launch slot at most);
+// pipeline (records: 192 bytes each, so 0.8 GB per launch slot at most);
 // larger launches use the lockstep persistent kernel.
 constexpr uint64_t kServerPipeMaxBlocks = 4u << 20;
 
