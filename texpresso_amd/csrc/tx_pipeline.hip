@@ -21,7 +21,7 @@ void PipeBufs::carve(uint8_t* base, uint64_t cap)
     off += up(4 * cap);
     for (int k = 0; k < kLists; ++k) {
         list[k] = reinterpret_cast<uint32_t*>(base + off);
-        off += up(4 * cap);
+        off += up(4 * kListArrays * cap);
     }
     ctl = reinterpret_cast<PipeCtl*>(base + off);
     capacity = cap;
@@ -42,48 +42,18 @@ using txp::kListC;
 using txp::kSearchWaves;
 constexpr uint32_t key_bit(int list) { return 1u << (5 + list); }
 
-__global__ void k_pipe_reset(PipeCtl* ctl)
-{
-    uint32_t* w = reinterpret_cast<uint32_t*>(ctl);
-    for (uint32_t i = threadIdx.x; i < sizeof(PipeCtl) / 4; i += blockDim.x) w[i] = 0u;
-}
-
 __device__ __forceinline__ const BatchTex& tex_at(const BatchTex* tex, const BatchTex& tex0, uint32_t i)
 {
     return tex ? tex[i] : tex0;
 }
 
-// Calls f(g, m) once for every value g of `group` among the lanes with `in`
-// set, m = the ballot of those lanes.  Uniform over the wave.
-template <class F>
-__device__ __forceinline__ void for_each_group(bool in, uint32_t group, F&& f)
+// The counters of this run, cleared by the first workgroup of the classify
+// pass: the kernels that use them start when it has ended.
+__device__ __forceinline__ void clear_counters(PipeCtl* __restrict__ ctl, int lane)
 {
-    uint64_t rem = __ballot(in);
-    while (rem) {
-        const int src = (int)__builtin_ctzll(rem);
-        const uint32_t g = (uint32_t)__builtin_amdgcn_readlane((int)group, src);
-        const uint64_t m = __ballot(in && group == g);
-        rem &= ~m;
-        f(g, m);
-    }
-}
-
-// Counts a wave of keys (lane slot `slot`) into the count copies: one ballot
-// per (copy, colour count) present among the lanes of each list the texture
-// variant feeds, and one atomic add by its first lane.
-template <int FMT, int ALG>
-__device__ __forceinline__ void count_keys(PipeCtl* __restrict__ ctl, uint32_t key, uint32_t slot, int lane)
-{
-    const uint32_t group = ((slot / txp::kBinSeg) % txp::kHistCopies) << 5 | (key & 31u);
-#pragma unroll
-    for (int k = 0; k < kLists; ++k) {
-        if (ALG == RANGE_FIT) continue;
-        if (ALG == CLUSTER_FIT && k != kListC) continue;
-        if (ALG == ITERATIVE_CLUSTER_FIT && (k == kListC || (k == kListA && FMT != BC1))) continue;
-        for_each_group((key & key_bit(k)) != 0u, group, [&](uint32_t g, uint64_t m) {
-            if (lane == (int)__builtin_ctzll(m)) atomicAdd(&ctl->part[g >> 5][k][g & 31u], (uint32_t)__popcll(m));
-        });
-    }
+    constexpr int words = sizeof(PipeCtl) / 4;
+    static_assert(words <= 64, "one word per lane");
+    if (blockIdx.x == 0 && lane < words) reinterpret_cast<uint32_t*>(ctl)[lane] = 0u;
 }
 
 // ClusterFit block on one lane: its record in slot r, and its key.
@@ -121,7 +91,7 @@ __device__ __forceinline__ uint32_t write_record_lane(ClusterRec* __restrict__ r
 
 // Blocks [first, first + count) of one texture, one per lane, 64 at a time.
 // Single-colour and range-fit blocks are finished here; ClusterFit blocks
-// become records in slots [slot0, slot0 + count), counted in ctl->part.  Block
+// become records in slots [slot0, slot0 + count).  Block
 // b of the pixel grid (a texture, or a level of a chain) is block b + block0 of
 // the output.
 struct PixelGrid {
@@ -132,7 +102,7 @@ struct PixelGrid {
 template <int FMT, int ALG, class Grid>
 __device__ __forceinline__ void classify_chunk(const Grid& G, const BatchTex& T, uint32_t tex_idx, uint32_t first, uint32_t count,
                                                uint32_t slot0, uint32_t block0, const LaneTables& LT, LaneBlockLds& LB, int lane,
-                                               ClusterRec* recs, uint32_t* keys, PipeCtl* ctl)
+                                               ClusterRec* recs, uint32_t* keys)
 {
     const FitParams fp{T.wr, T.wg, T.wb, T.weigh_alpha};
     for (uint32_t off = 0; off < count; off += 64) {
@@ -156,7 +126,6 @@ __device__ __forceinline__ void classify_chunk(const Grid& G, const BatchTex& T,
             }
             keys[slot0 + k] = key;
         }
-        count_keys<FMT, ALG>(ctl, key, slot0 + k, lane);
     }
 }
 
@@ -171,6 +140,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
     __shared__ LaneTables LT;
     __shared__ LaneBlockLds LB;
     const int lane = (int)threadIdx.x;
+    clear_counters(ctl, lane);
     fill_lane_tables(LT, lane);
     group_sync();
     // chunks hold similar work, so a plain grid-stride loop balances them
@@ -179,15 +149,15 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
         const uint4 ch = chunks[c];
         const BatchTex& T = tex[ch.x];
         switch (T.variant) {
-        case 0: classify_chunk<BC1, RANGE_FIT>(T, T, ch.x, ch.y, ch.z, ch.w, 0u, LT, LB, lane, recs, keys, ctl); break;
-        case 1: classify_chunk<BC1, CLUSTER_FIT>(T, T, ch.x, ch.y, ch.z, ch.w, 0u, LT, LB, lane, recs, keys, ctl); break;
-        case 2: classify_chunk<BC1, ITERATIVE_CLUSTER_FIT>(T, T, ch.x, ch.y, ch.z, ch.w, 0u, LT, LB, lane, recs, keys, ctl); break;
-        case 3: classify_chunk<BC2, RANGE_FIT>(T, T, ch.x, ch.y, ch.z, ch.w, 0u, LT, LB, lane, recs, keys, ctl); break;
-        case 4: classify_chunk<BC2, CLUSTER_FIT>(T, T, ch.x, ch.y, ch.z, ch.w, 0u, LT, LB, lane, recs, keys, ctl); break;
-        case 5: classify_chunk<BC2, ITERATIVE_CLUSTER_FIT>(T, T, ch.x, ch.y, ch.z, ch.w, 0u, LT, LB, lane, recs, keys, ctl); break;
-        case 6: classify_chunk<BC3, RANGE_FIT>(T, T, ch.x, ch.y, ch.z, ch.w, 0u, LT, LB, lane, recs, keys, ctl); break;
-        case 7: classify_chunk<BC3, CLUSTER_FIT>(T, T, ch.x, ch.y, ch.z, ch.w, 0u, LT, LB, lane, recs, keys, ctl); break;
-        default: classify_chunk<BC3, ITERATIVE_CLUSTER_FIT>(T, T, ch.x, ch.y, ch.z, ch.w, 0u, LT, LB, lane, recs, keys, ctl); break;
+        case 0: classify_chunk<BC1, RANGE_FIT>(T, T, ch.x, ch.y, ch.z, ch.w, 0u, LT, LB, lane, recs, keys); break;
+        case 1: classify_chunk<BC1, CLUSTER_FIT>(T, T, ch.x, ch.y, ch.z, ch.w, 0u, LT, LB, lane, recs, keys); break;
+        case 2: classify_chunk<BC1, ITERATIVE_CLUSTER_FIT>(T, T, ch.x, ch.y, ch.z, ch.w, 0u, LT, LB, lane, recs, keys); break;
+        case 3: classify_chunk<BC2, RANGE_FIT>(T, T, ch.x, ch.y, ch.z, ch.w, 0u, LT, LB, lane, recs, keys); break;
+        case 4: classify_chunk<BC2, CLUSTER_FIT>(T, T, ch.x, ch.y, ch.z, ch.w, 0u, LT, LB, lane, recs, keys); break;
+        case 5: classify_chunk<BC2, ITERATIVE_CLUSTER_FIT>(T, T, ch.x, ch.y, ch.z, ch.w, 0u, LT, LB, lane, recs, keys); break;
+        case 6: classify_chunk<BC3, RANGE_FIT>(T, T, ch.x, ch.y, ch.z, ch.w, 0u, LT, LB, lane, recs, keys); break;
+        case 7: classify_chunk<BC3, CLUSTER_FIT>(T, T, ch.x, ch.y, ch.z, ch.w, 0u, LT, LB, lane, recs, keys); break;
+        default: classify_chunk<BC3, ITERATIVE_CLUSTER_FIT>(T, T, ch.x, ch.y, ch.z, ch.w, 0u, LT, LB, lane, recs, keys); break;
         }
     }
 }
@@ -204,6 +174,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
     __shared__ LaneTables LT;
     __shared__ LaneBlockLds LB;
     const int lane = (int)threadIdx.x;
+    clear_counters(ctl, lane);
     fill_lane_tables(LT, lane);
     group_sync();
     for (uint32_t c = blockIdx.x; c < nchunks; c += gridDim.x) {
@@ -218,69 +189,91 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
             G = PixelGrid{v.rgba, v.width, v.height, v.blocks_wide};
         }
         classify_chunk<FMT, ALG>(G, tex0, 0u, f, min(chunk_blocks, n - f), block0 + f, block0, LT, LB, lane, recs,
-                                 keys, ctl);
+                                 keys);
     }
 }
 
-// Counting sort of the records by colour count, 16 first, one workgroup
-// per slot segment s (kBinSeg slots).  Bin (list k, colour count v) starts
-// after bins v+1..16 of its list and holds the records of count copy 0, then
-// copy 1, ...; the workgroup sums the copies into the totals (workgroup 0
-// also stores them in ctl->hist for the search passes) and into the start
-// of its own copy c = s % kHistCopies, counts its keys per bin in LDS,
-// reserves one range per non-empty bin with one atomic add on copy c's
-// cursor, then places its records inside those ranges (order within a bin
-// is free: it only steers which records share a wave).
-__global__ __launch_bounds__(256) void k_pipe_bin(const uint32_t* __restrict__ keys, uint64_t nslots,
+// Where position p of a part lies in its list's arrays of nslots entries.
+__device__ __forceinline__ size_t part_at(uint32_t part, uint32_t p, uint32_t nslots)
+{
+    return (size_t)(part >> 1) * nslots + (part & 1u ? nslots - 1u - p : p);
+}
+
+// The records of one slot segment into the lists: a counting sort by colour
+// count, 16 first, in LDS, and a range of each part reserved with one atomic.
+// A part is thus sorted run by run, not as a whole; a whole sort took a
+// histogram in the classify pass, its reset and a sum over its copies here
+// (reset 4.5 us, bin 11, against 7 now).
+__global__ __launch_bounds__(256) void k_pipe_bin(const uint32_t* __restrict__ keys, uint32_t nslots,
                                                   PipeCtl* __restrict__ ctl, uint32_t* __restrict__ list_a,
                                                   uint32_t* __restrict__ list_b, uint32_t* __restrict__ list_c)
 {
-    constexpr uint32_t kCounts = kLists * 17;
-    __shared__ uint32_t cnt[kLists][17], base[kLists][17], tot[kLists][17], pre[kLists][17];
+    constexpr uint32_t kPer = txp::kBinSeg / 256, kParts = txp::kListParts;
+    __shared__ uint32_t cnt[kLists][17], off[kLists][17], base[kLists][kParts];
     uint32_t* const lists[kLists] = {list_a, list_b, list_c};
     const uint32_t t = threadIdx.x;
-    const uint32_t copy = blockIdx.x % txp::kHistCopies;
-    if (t < 17)
-        for (int k = 0; k < kLists; ++k) cnt[k][t] = tot[k][t] = pre[k][t] = 0u;
-    __syncthreads();
-    // totals and the start of this copy: 4 threads per count, each summing
-    // every 4th copy
-    if (t < 4 * kCounts) {
-        const uint32_t km = t % kCounts;
-        uint32_t sum = 0, below = 0;
-        for (uint32_t c = t / kCounts; c < txp::kHistCopies; c += 4) {
-            const uint32_t v = (&ctl->part[c][0][0])[km];
-            sum += v;
-            below += c < copy ? v : 0u;
-        }
-        if (sum) atomicAdd(&(&tot[0][0])[km], sum);
-        if (below) atomicAdd(&(&pre[0][0])[km], below);
+    if (t < kLists * 17) (&cnt[0][0])[t] = 0u;
+    uint32_t key[kPer], rank[kPer][kLists];
+#pragma unroll
+    for (uint32_t i = 0; i < kPer; ++i) {
+        const uint64_t r = (uint64_t)blockIdx.x * txp::kBinSeg + i * 256u + t;
+        key[i] = r < nslots ? keys[r] : 0u;
     }
-    const uint64_t s0 = (uint64_t)blockIdx.x * txp::kBinSeg;
-    const uint64_t s1 = s0 + txp::kBinSeg < nslots ? s0 + txp::kBinSeg : nslots;
-    for (uint64_t r = s0 + t; r < s1; r += blockDim.x) {
-        const uint32_t key = keys[r];
+    __syncthreads();
+#pragma unroll
+    for (uint32_t i = 0; i < kPer; ++i)
         for (int k = 0; k < kLists; ++k)
-            if (key & key_bit(k)) atomicAdd(&cnt[k][key & 31u], 1u);
+            if (key[i] & key_bit(k)) rank[i][k] = atomicAdd(&cnt[k][key[i] & 31u], 1u);
+    __syncthreads();
+    // the second wave reserves the ranges while the first sums, for each
+    // count, the larger ones of its part
+    if (t >= 64u && t < 64u + kLists * kParts) {
+        const uint32_t k = (t - 64u) / kParts, part = (t - 64u) % kParts;
+        uint32_t n = 0;
+#pragma unroll
+        for (uint32_t m = 0; m <= 16; ++m) n += txp::part_of(m) == part ? cnt[k][m] : 0u;
+        base[k][part] = n ? atomicAdd(&ctl->count[k][part], n) : 0u;
+    } else if (t < kLists * 17) {
+        const uint32_t k = t / 17u, n = t % 17u;
+        uint32_t sum = 0;
+#pragma unroll
+        for (uint32_t m = 1; m <= 16; ++m) sum += m > n && txp::part_of(m) == txp::part_of(n) ? cnt[k][m] : 0u;
+        off[k][n] = sum;
     }
     __syncthreads();
-    if (blockIdx.x == 0 && t < kCounts) (&ctl->hist[0][0])[t] = (&tot[0][0])[t];
-    if (t < 17) {
-        for (int k = 0; k < kLists; ++k) {
-            uint32_t o = pre[k][t];
-            for (int m = 16; m > (int)t; --m) o += tot[k][m];
-            base[k][t] = cnt[k][t] ? o + atomicAdd(&ctl->pos[copy][k][t], cnt[k][t]) : 0u;
-            cnt[k][t] = 0u;
-        }
-    }
-    __syncthreads();
-    for (uint64_t r = s0 + t; r < s1; r += blockDim.x) {
-        const uint32_t key = keys[r];
-        const uint32_t n = key & 31u;
+#pragma unroll
+    for (uint32_t i = 0; i < kPer; ++i) {
+        const uint32_t r = blockIdx.x * txp::kBinSeg + i * 256u + t, n = key[i] & 31u;
+        const uint32_t part = txp::part_of(n);
         for (int k = 0; k < kLists; ++k)
-            if (key & key_bit(k)) lists[k][base[k][n] + atomicAdd(&cnt[k][n], 1u)] = (uint32_t)r;
+            if (key[i] & key_bit(k)) lists[k][part_at(part, base[k][part] + off[k][n] + rank[i][k], nslots)] = r;
     }
 }
+
+// One list as a search reads it.
+struct RecList {
+    const uint32_t* __restrict__ slots;
+    uint32_t nslots, end[txp::kListParts];  // end: positions up to and with each part
+
+    __device__ RecList(const uint32_t* s, uint32_t n, const PipeCtl* __restrict__ ctl, int k) : slots(s), nslots(n)
+    {
+        uint32_t sum = 0;
+        for (uint32_t i = 0; i < txp::kListParts; ++i) end[i] = sum += ctl->count[k][i];
+    }
+    __device__ uint32_t total() const { return end[txp::kListParts - 1]; }
+    // Record slot at position p < total().
+    __device__ uint32_t at(uint32_t p) const
+    {
+        uint32_t part = 0, start = 0;
+#pragma unroll
+        for (uint32_t i = 0; i + 1 < txp::kListParts; ++i) {
+            const bool past = p >= end[i];
+            part = past ? i + 1 : part;
+            start = past ? end[i] : start;
+        }
+        return slots[part_at(part, p - start, nslots)];
+    }
+};
 
 // The block of record R into its group's LDS: lane l writes the point that
 // pixel l opens, if it does (colourset.rs:45-97 in pixel order).  Returns the
@@ -412,16 +405,18 @@ __device__ __forceinline__ void take_positions(uint64_t* run, uint32_t* refillin
 // are otherwise independent (no workgroup barrier after the set-up).
 template <int NC>
 __global__ __launch_bounds__(64 * kSearchWaves) __attribute__((amdgpu_waves_per_eu(4))) void k_pipe_search(
-    const BatchTex* __restrict__ tex, BatchTex tex0, ClusterRec* __restrict__ recs, const uint32_t* __restrict__ list,
-    const uint32_t* __restrict__ hist, uint32_t* __restrict__ cursor)
+    const BatchTex* __restrict__ tex, BatchTex tex0, ClusterRec* __restrict__ recs, const uint32_t* __restrict__ slots,
+    uint32_t nslots, PipeCtl* __restrict__ ctl)
 {
+    constexpr int kList = NC == 3 ? kListA : kListB;
+    const RecList list(slots, nslots, ctl, kList);
+    uint32_t* const cursor = &ctl->cursor[kList];
     __shared__ GroupLds lds[4 * kSearchWaves];
     __shared__ uint64_t run;
     __shared__ uint32_t refilling;
     const int lane = (int)(threadIdx.x & 63u), g = lane >> 4, l = lane & 15;
     GroupLds& L = lds[4 * (threadIdx.x >> 6) + g];
-    uint32_t total = 0;
-    for (int m = 0; m < 17; ++m) total += hist[m];
+    const uint32_t total = list.total();
     // refills of kRefill positions: at most one per group of the workgroup
     // and at most the records per wave, so a short list still spreads over
     // every workgroup; the first run of each workgroup is fixed by its index
@@ -459,7 +454,7 @@ __global__ __launch_bounds__(64 * kSearchWaves) __attribute__((amdgpu_waves_per_
                     if (p >= total) {
                         idle = true;
                     } else {
-                        const uint32_t r = list[p];
+                        const uint32_t r = list.at(p);
                         const ClusterRec& R = recs[r];
                         remap = load_points(R, L, l);
                         info = R.info;
@@ -542,15 +537,16 @@ __global__ __launch_bounds__(64 * kSearchWaves) __attribute__((amdgpu_waves_per_
 // idle wave could have run.
 __global__ __launch_bounds__(64 * kSearchWaves) __attribute__((amdgpu_waves_per_eu(4))) void k_pipe_cluster(
     const BatchTex* __restrict__ tex, BatchTex tex0, const ClusterRec* __restrict__ recs,
-    const uint32_t* __restrict__ list, const uint32_t* __restrict__ hist, uint32_t* __restrict__ cursor)
+    const uint32_t* __restrict__ slots, uint32_t nslots, PipeCtl* __restrict__ ctl)
 {
+    const RecList list(slots, nslots, ctl, kListC);
+    uint32_t* const cursor = &ctl->cursor[kListC];
     __shared__ GroupLds lds[4 * kSearchWaves];
     __shared__ uint64_t run;
     __shared__ uint32_t refilling;
     const int lane = (int)(threadIdx.x & 63u), g = lane >> 4, l = lane & 15;
     GroupLds& L = lds[4 * (threadIdx.x >> 6) + g];
-    uint32_t total = 0;
-    for (int m = 0; m < 17; ++m) total += hist[m];
+    const uint32_t total = list.total();
     // refills of up to four steps for one wave (16 positions), at most the
     // records per wave; the first run of each workgroup is fixed by its
     // index, refills come from the shared cursor, offset past those runs
@@ -575,7 +571,7 @@ __global__ __launch_bounds__(64 * kSearchWaves) __attribute__((amdgpu_waves_per_
         float axx = 0.0f, axy = 0.0f, axz = 0.0f;
         uint32_t fmt = BC1;
         if (has) {
-            const ClusterRec& R = recs[list[p]];
+            const ClusterRec& R = recs[list.at(p)];
             cs.remap = load_points(R, L, l);
             const uint32_t info = R.info;
             fmt = (info >> 12) & 15u;
@@ -641,7 +637,6 @@ hipError_t launch_pipeline(const PipeLaunch& p, const PipeBufs& b, hipStream_t s
 {
     if (p.nslots > b.capacity || p.nslots > 0xFFFFFFFFull) return hipErrorInvalidValue;
     auto mark = [&](int i) { return marks ? hipEventRecord(marks[i], s) : hipSuccess; };
-    hipLaunchKernelGGL(txd::k_pipe_reset, dim3(1), dim3(256), 0, s, b.ctl);
     if (p.nchunks == 0 || p.nslots == 0) {
         for (int i = 0; i < 5; ++i)
             if (mark(i) != hipSuccess) return hipErrorUnknown;
@@ -652,19 +647,19 @@ hipError_t launch_pipeline(const PipeLaunch& p, const PipeBufs& b, hipStream_t s
     if (mark(1) != hipSuccess) return hipErrorUnknown;
     const uint32_t bin_grid = (uint32_t)((p.nslots + kBinSeg - 1) / kBinSeg);
     const uint32_t search_wgs = (p.search_grid + kSearchWaves - 1) / kSearchWaves;
-    hipLaunchKernelGGL(txd::k_pipe_bin, dim3(bin_grid), dim3(256), 0, s, b.keys, p.nslots, b.ctl, b.list[kListA],
+    hipLaunchKernelGGL(txd::k_pipe_bin, dim3(bin_grid), dim3(256), 0, s, b.keys, (uint32_t)p.nslots, b.ctl, b.list[kListA],
                        b.list[kListB], b.list[kListC]);
     if (mark(2) != hipSuccess) return hipErrorUnknown;
     if (p.lists & (1u << kListC))
         hipLaunchKernelGGL(txd::k_pipe_cluster, dim3(search_wgs), dim3(64 * kSearchWaves), 0, s, p.d_tex, p.tex0, b.recs,
-                           b.list[kListC], b.ctl->hist[kListC], &b.ctl->cursor[kListC]);
+                           b.list[kListC], (uint32_t)p.nslots, b.ctl);
     if (p.lists & (1u << kListA))
         hipLaunchKernelGGL(txd::k_pipe_search<3>, dim3(search_wgs), dim3(64 * kSearchWaves), 0, s, p.d_tex, p.tex0, b.recs,
-                           b.list[kListA], b.ctl->hist[kListA], &b.ctl->cursor[kListA]);
+                           b.list[kListA], (uint32_t)p.nslots, b.ctl);
     if (mark(3) != hipSuccess) return hipErrorUnknown;
     if (p.lists & (1u << kListB))
         hipLaunchKernelGGL(txd::k_pipe_search<4>, dim3(search_wgs), dim3(64 * kSearchWaves), 0, s, p.d_tex, p.tex0, b.recs,
-                           b.list[kListB], b.ctl->hist[kListB], &b.ctl->cursor[kListB]);
+                           b.list[kListB], (uint32_t)p.nslots, b.ctl);
     if (mark(4) != hipSuccess) return hipErrorUnknown;
     return hipGetLastError();
 }

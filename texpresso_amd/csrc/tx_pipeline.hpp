@@ -1,11 +1,12 @@
 // tx_pipeline.hpp -- the binned ClusterFit pipeline (host-side interface).
 //
-//   reset -> classify -> bin -> search<3> (BC1) -> search<4>
+//   classify -> bin -> search<3> (BC1) -> search<4>
 //
 // classify: alpha, colour set and fit choice for every block, one block per
 //   lane; single-colour and range-fit blocks are finished here, ClusterFit
 //   blocks become a ClusterRec and are counted by distinct-colour count n.
-// bin: counting sort of the records by n (16 first) into one list per pass
+// bin: the records into one list per pass, many-coloured ones first and
+//   neighbours of one colour count
 //   (list A: BC1 IterativeClusterFit records for the 3-colour search; list
 //   B: records that need the 4-colour search -- BC1 IterativeClusterFit
 //   without transparency, BC2/BC3 IterativeClusterFit; list C: ClusterFit
@@ -51,42 +52,41 @@ static_assert(offsetof(ClusterRec, lowest) == 128 && offsetof(ClusterRec, half) 
                   offsetof(ClusterRec, block) == 184,
               "record tail layout");
 
-// Counters of one pipeline run (cleared by the reset kernel).  Every update
-// is aggregated (per workgroup or per batch of records) so that no counter
-// takes one global atomic per block.
 enum { kListA = 0, kListB = 1, kListC = 2, kLists = 3 };
 
-// The bin pass sorts kBinSeg consecutive record slots per workgroup.
+// The bin pass takes kBinSeg consecutive record slots per workgroup.
 constexpr uint32_t kBinSeg = 1024;
 
-// Bin counts and bin cursors are kept in kHistCopies copies: the records of
-// slot segment s (slots [s * kBinSeg, (s + 1) * kBinSeg)) are counted in copy
-// s % kHistCopies, and bin (list k, colour count v) is laid out copy after
-// copy.  Device-scope atomic adds on one word serialise; with a single copy,
-// thousands of classify workgroups finishing together, nearly all counting
-// 16-colour blocks, queued on the same word (2048x2048: ~27 us per list of
-// a ~70 us pass), and every bin workgroup on the same cursor.  With copies,
-// no word takes more than a few dozen adds.
-constexpr uint32_t kHistCopies = 64;
+// A list's records lie in six parts by colour count, handed out in order: 16
+// colours from the front of the list's first array up, 15 from its end down,
+// 14 and 13 likewise in the second array, 10-12 and the others in the third.
+// So groups of a wave, which draw from runs far apart in the list, nearly
+// always search equally long candidate lists, and the long records come
+// first.  (IterativeClusterFit search of a 2048^2 texture: 873 us with a list
+// sorted as a whole, 890 with six parts, 895 with four, 929 with two; the
+// whole sort cost 10 us more before the search.)
+constexpr uint32_t kListParts = 6, kListArrays = 3;
+constexpr uint32_t part_of(uint32_t n) { return n >= 13u ? 16u - n : n >= 10u ? 4u : 5u; }
 
+// Counters of one pipeline run, cleared by the classify pass (which does not
+// use them).
 struct PipeCtl {
-    uint32_t cursor[kLists];
-    uint32_t hist[kLists][17];                // records per colour count (totals, written by the bin pass)
-    uint32_t part[kHistCopies][kLists][17];   // records per colour count, copy by copy (classify pass)
-    uint32_t pos[kHistCopies][kLists][17];    // records placed per colour count, copy by copy (bin pass)
+    uint32_t count[kLists][kListParts];  // records in each part
+    uint32_t cursor[kLists];             // positions the search has handed out
 };
 
 struct PipeBufs {
     ClusterRec* recs = nullptr;          // capacity records; slot = the block's position among the chunks
     uint32_t* keys = nullptr;            // capacity: n | in list L << (5 + L); 0 = no record
-    uint32_t* list[kLists] = {nullptr};  // capacity each: record slots sorted by n, 16 first
+    uint32_t* list[kLists] = {nullptr};  // kListArrays arrays of `capacity` record slots each
     PipeCtl* ctl = nullptr;
     uint64_t capacity = 0;
 
     // bytes of device memory for `cap` records (one allocation, 256-aligned parts)
     static constexpr size_t bytes_for(uint64_t cap)
     {
-        return align256(sizeof(ClusterRec) * cap) + (1 + kLists) * align256(4 * cap) + align256(sizeof(PipeCtl));
+        return align256(sizeof(ClusterRec) * cap) + align256(4 * cap) + kLists * align256(4 * kListArrays * cap) +
+               align256(sizeof(PipeCtl));
     }
     static constexpr size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
     // carves the parts out of one allocation of bytes_for(cap) bytes
@@ -127,7 +127,7 @@ inline uint32_t lists_for(uint32_t format, uint32_t algorithm)
     return format == 0 ? (1u << kListA) | (1u << kListB) : 1u << kListB;
 }
 
-// Launches reset, classify, bin and the searches on `s`.  With `marks`
+// Launches classify, bin and the searches on `s`.  With `marks`
 // (5 events), marks[0] is recorded before classify, marks[1] after it,
 // marks[2] after bin, marks[3] after the ClusterFit pass and the 3-colour
 // search (recorded even when there are none) and marks[4] after the
