@@ -255,6 +255,66 @@ static hipError_t encode_on(txc::DeviceContext* ctx, const txk::EncodeArgs& a, h
     return e;
 }
 
+// Kernels read pinned input themselves up to this size.  The decoder and the
+// one-block-per-lane encoders read it once in long runs: no copy is faster at
+// every staged size (RangeFit 512^2 71 us against 83 with one, 64^2 24 / 27;
+// decoding 512^2 68 / 80, 64^2 16 / 21).  The 16-lane groups of the cluster
+// fits fetch 16 bytes at a time over the bus, which a copy beats from about 64
+// KiB on (BC1 ClusterFit 64^2 31 us against 32 with a copy, 128^2 41 / 40,
+// 256^2 64 / 59).
+constexpr size_t kDirectGroupBytes = 32u << 10;
+
+static size_t direct_in_bytes(int format, int algorithm)
+{
+    return format <= TX_BC3 && algorithm != TX_RANGE_FIT ? kDirectGroupBytes : txc::kStageBytes;
+}
+
+namespace {
+
+// Moves a host-staged call's input and output (txc::kStageBytes).  Used under
+// the context's lock, by one call at a time, which ends with finish().
+class HostCall {
+public:
+    HostCall(txc::DeviceContext* c, size_t in_total, size_t direct_in_max, size_t out_total) : ctx(c)
+    {
+        if (in_total <= txc::kStageBytes || out_total <= txc::kStageBytes) pin = ctx->staging();
+        stage_in = pin && in_total <= txc::kStageBytes;
+        direct_in = stage_in && in_total <= direct_in_max;
+        stage_out = pin && out_total <= txc::kStageBytes;
+    }
+    // n bytes of `src` where kernels on the context's stream can read them:
+    // d_buf, or the pinned memory itself at `at` of its input half (the parts
+    // of a call's input follow one another).  Null on an error.
+    const uint8_t* upload(uint8_t* d_buf, const void* src, size_t n, size_t at = 0)
+    {
+        if (n == 0) return d_buf;
+        if (stage_in) {
+            memcpy(pin + at, src, n);
+            if (direct_in) return pin + at;
+            src = pin + at;
+        }
+        return hipMemcpyAsync(d_buf, src, n, hipMemcpyHostToDevice, ctx->stream) == hipSuccess ? d_buf : nullptr;
+    }
+    // Where kernels write the output: d_buf, or the pinned memory.
+    uint8_t* output(uint8_t* d_buf) { return stage_out ? pin + txc::kStageBytes : d_buf; }
+    // Waits for the call's work and leaves its n bytes of output in dst.
+    int finish(void* dst, const uint8_t* d_buf, size_t n)
+    {
+        if (!stage_out && hipMemcpyAsync(dst, d_buf, n, hipMemcpyDeviceToHost, ctx->stream) != hipSuccess)
+            return TX_ERR_HIP;
+        if (hipStreamSynchronize(ctx->stream) != hipSuccess) return TX_ERR_HIP;
+        if (stage_out) memcpy(dst, pin + txc::kStageBytes, n);
+        return TX_OK;
+    }
+
+private:
+    txc::DeviceContext* ctx;
+    uint8_t* pin = nullptr;
+    bool stage_in = false, direct_in = false, stage_out = false;
+};
+
+}  // namespace
+
 int tx_compress(int format, const uint8_t* rgba, size_t rgba_len, size_t width, size_t height,
                 const tx_params* params, uint8_t* output, size_t out_len)
 {
@@ -270,16 +330,14 @@ int tx_compress(int format, const uint8_t* rgba, size_t rgba_len, size_t width, 
     const size_t in_cap = (in_bytes + 255) & ~(size_t)255;
     uint8_t* d = ctx->scratch(in_cap + out_len);
     if (!d) return TX_ERR_NOMEM;
-    uint8_t* d_in = d;
-    uint8_t* d_out = d + in_cap;
-    if (in_bytes && hipMemcpyAsync(d_in, rgba, in_bytes, hipMemcpyHostToDevice, ctx->stream) != hipSuccess)
-        return TX_ERR_HIP;
+    HostCall call(ctx, in_bytes, direct_in_bytes(format, params->algorithm), out_len);
+    const uint8_t* d_in = call.upload(d, rgba, in_bytes);
+    uint8_t* d_out = call.output(d + in_cap);
+    if (!d_in) return TX_ERR_HIP;
     if (encode_on(ctx, encode_args(format, params, d_in, width, height, d_out, out_len), ctx->stream) !=
         hipSuccess)
         return TX_ERR_HIP;
-    if (hipMemcpyAsync(output, d_out, out_len, hipMemcpyDeviceToHost, ctx->stream) != hipSuccess) return TX_ERR_HIP;
-    if (hipStreamSynchronize(ctx->stream) != hipSuccess) return TX_ERR_HIP;
-    return TX_OK;
+    return call.finish(output, d_out, out_len);
 }
 
 int tx_compress_device(int format, const uint8_t* d_rgba, size_t width, size_t height, const tx_params* params,
@@ -489,17 +547,16 @@ int tx_compress_mips(int format, const uint8_t* rgba, size_t rgba_len, size_t wi
     auto up = [](size_t x) { return (x + 255) & ~(size_t)255; };
     uint8_t* d = ctx->scratch(up(in_bytes) + up(chain_len) + need);
     if (!d) return TX_ERR_NOMEM;
-    uint8_t* d_in = d;
     uint8_t* d_chain = d + up(in_bytes);
-    uint8_t* d_out = d_chain + up(chain_len);
-    if (hipMemcpyAsync(d_in, rgba, in_bytes, hipMemcpyHostToDevice, ctx->stream) != hipSuccess) return TX_ERR_HIP;
+    HostCall call(ctx, in_bytes, direct_in_bytes(format, params->algorithm), need);
+    const uint8_t* d_in = call.upload(d, rgba, in_bytes);
+    uint8_t* d_out = call.output(d_chain + up(chain_len));
+    if (!d_in) return TX_ERR_HIP;
     if (mips_on(d_in, width, height, levels, d_chain, ctx->stream) != hipSuccess) return TX_ERR_HIP;
     if (compress_chain_on(ctx, format, params, d_in, width, height, levels, d_chain, d_out, ctx->stream) !=
         hipSuccess)
         return TX_ERR_HIP;
-    if (hipMemcpyAsync(output, d_out, need, hipMemcpyDeviceToHost, ctx->stream) != hipSuccess) return TX_ERR_HIP;
-    if (hipStreamSynchronize(ctx->stream) != hipSuccess) return TX_ERR_HIP;
-    return TX_OK;
+    return call.finish(output, d_out, need);
 }
 
 int tx_compress_block_masked(int format, const uint8_t rgba[64], uint32_t mask, const tx_params* params,
@@ -526,17 +583,16 @@ int tx_compress_blocks(int format, const uint8_t* blocks, const uint32_t* masks,
     const size_t pix = 64 * nblocks, msk = (4 * nblocks + 255) & ~(size_t)255;
     uint8_t* d = ctx->scratch(pix + msk + nblocks * bs);
     if (!d) return TX_ERR_NOMEM;
-    uint8_t* d_pix = d;
-    uint32_t* d_mask = reinterpret_cast<uint32_t*>(d + pix);
-    uint8_t* d_out = d + pix + msk;
-    if (hipMemcpyAsync(d_pix, blocks, pix, hipMemcpyHostToDevice, ctx->stream) != hipSuccess) return TX_ERR_HIP;
-    if (hipMemcpyAsync(d_mask, masks, 4 * nblocks, hipMemcpyHostToDevice, ctx->stream) != hipSuccess)
-        return TX_ERR_HIP;
+    HostCall call(ctx, pix + 4 * nblocks, kDirectGroupBytes, nblocks * bs);
+    const uint8_t* d_pix = call.upload(d, blocks, pix);
+    const uint8_t* d_mask = call.upload(d + pix, masks, 4 * nblocks, pix);
+    uint8_t* d_out = call.output(d + pix + msk);
+    if (!d_pix || !d_mask) return TX_ERR_HIP;
     txk::BlockListArgs a;
     a.format = format;
     a.algorithm = params->algorithm;
     a.blocks = d_pix;
-    a.masks = d_mask;
+    a.masks = reinterpret_cast<const uint32_t*>(d_mask);
     a.nblocks = nblocks;
     a.out = d_out;
     a.wr = params->weights[0];
@@ -544,10 +600,7 @@ int tx_compress_blocks(int format, const uint8_t* blocks, const uint32_t* masks,
     a.wb = params->weights[2];
     a.weigh_alpha = params->weigh_colour_by_alpha ? 1u : 0u;
     if (txk::launch_encode_blocks(a, ctx->stream) != hipSuccess) return TX_ERR_HIP;
-    if (hipMemcpyAsync(output, d_out, nblocks * bs, hipMemcpyDeviceToHost, ctx->stream) != hipSuccess)
-        return TX_ERR_HIP;
-    if (hipStreamSynchronize(ctx->stream) != hipSuccess) return TX_ERR_HIP;
-    return TX_OK;
+    return call.finish(output, d_out, nblocks * bs);
 }
 
 int tx_decompress(int format, const uint8_t* data, size_t data_len, size_t width, size_t height, uint8_t* output,
@@ -570,13 +623,13 @@ int tx_decompress(int format, const uint8_t* data, size_t data_len, size_t width
     const size_t in_cap = (need + 255) & ~(size_t)255;
     uint8_t* d = ctx->scratch(in_cap + px_bytes);
     if (!d) return TX_ERR_NOMEM;
-    if (hipMemcpyAsync(d, data, need, hipMemcpyHostToDevice, ctx->stream) != hipSuccess) return TX_ERR_HIP;
-    if (txk::launch_decode(format, d, (uint32_t)width, (uint32_t)height, d + in_cap, ctx->stream) != hipSuccess)
+    HostCall call(ctx, need, txc::kStageBytes, px_bytes);
+    const uint8_t* d_in = call.upload(d, data, need);
+    uint8_t* d_out = call.output(d + in_cap);
+    if (!d_in) return TX_ERR_HIP;
+    if (txk::launch_decode(format, d_in, (uint32_t)width, (uint32_t)height, d_out, ctx->stream) != hipSuccess)
         return TX_ERR_HIP;
-    if (hipMemcpyAsync(output, d + in_cap, px_bytes, hipMemcpyDeviceToHost, ctx->stream) != hipSuccess)
-        return TX_ERR_HIP;
-    if (hipStreamSynchronize(ctx->stream) != hipSuccess) return TX_ERR_HIP;
-    return TX_OK;
+    return call.finish(output, d_out, px_bytes);
 }
 
 int tx_decompress_device(int format, const uint8_t* d_data, size_t width, size_t height, uint8_t* d_output,

@@ -38,6 +38,16 @@ uint8_t* DeviceContext::scratch(size_t bytes)
     return pool;
 }
 
+uint8_t* DeviceContext::staging()
+{
+    if (!pinned && hipHostMalloc(reinterpret_cast<void**>(&pinned), 2 * kStageBytes,
+                                   hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
+        pinned = nullptr;
+        (void)hipGetLastError();
+    }
+    return pinned;
+}
+
 bool DeviceContext::pipe_scratch(uint64_t recs, txp::PipeBufs* out)
 {
     if (recs > pipe_recs || !pipe) {

@@ -10,6 +10,12 @@
 
 namespace txc {
 
+// A host-staged call's input or output of up to kStageBytes goes through the
+// context's pinned memory: the runtime stages a copy from pageable memory
+// itself and waits for it, while pinned memory is copied by an enqueued
+// command, or read and written by the kernels themselves without any copy.
+constexpr size_t kStageBytes = 1u << 20;
+
 struct DeviceContext {
     int device = -1;
     char arch[64] = {0};
@@ -18,6 +24,11 @@ struct DeviceContext {
     std::mutex mu;                 // guards the staging pool and host-staged calls
     uint8_t* pool = nullptr;
     size_t pool_cap = 0;
+
+    // Pinned host memory for small host-staged calls: kStageBytes for what goes
+    // to the device, then as much for what comes back.  Allocated at the first
+    // such call, held as long as the context; guarded by `mu`.
+    uint8_t* pinned = nullptr;
 
     // Binned-pipeline scratch, shared by every stream of the device.  Uses
     // are ordered through `pipe_done`: a use on a caller's stream waits for
@@ -34,6 +45,8 @@ struct DeviceContext {
 
     // Device staging memory of at least `bytes` (grown geometrically); call with mu held.
     uint8_t* scratch(size_t bytes);
+    // The pinned memory, null when it cannot be had; call with mu held.
+    uint8_t* staging();
     // Pipeline buffers for `recs` records; call with pipe_mu held.
     bool pipe_scratch(uint64_t recs, txp::PipeBufs* out);
     // Orders a use of the pipeline scratch on `s` after every earlier use
