@@ -64,46 +64,66 @@ struct BatchTex {
     uint32_t weigh_alpha;
 };
 
+// Blocks per chunk of an alpha-only (BC4/BC5) texture encoded one block per
+// lane: 8 steps of 64 blocks.
+constexpr uint32_t kLightChunkBlocks = 512;
+
+// Launch shape of the alpha-only kernel.  One block per lane: 4-wave
+// workgroups, up to 8 per CU, whose waves take pieces of `steps` steps (1, 2, 4
+// or 8) of a chunk: as large as leaves every wave one (a whole chunk takes a
+// wave 35 us, so a small batch is cut finer).  16 lanes per block: the LDS
+// encoder's workgroups over whole chunks.
+struct AlphaShape {
+    uint32_t grid, steps;
+    uint32_t pieces(uint32_t nlight) const { return steps ? nlight * (kLightChunkBlocks / 64u / steps) : nlight; }
+};
+inline AlphaShape alpha_shape(uint32_t cus, uint32_t nlight, uint32_t alpha_lanes, uint32_t groups_per_cu,
+                              uint32_t waves_per_group)
+{
+    AlphaShape a{0, 0};
+    if (alpha_lanes != 16) {
+        a.steps = kLightChunkBlocks / 64u;
+        while (a.steps > 1 && (uint64_t)a.pieces(nlight) < (uint64_t)cus * 32) a.steps /= 2;
+    }
+    const uint64_t want = alpha_lanes == 16 ? ((uint64_t)nlight + waves_per_group - 1) / waves_per_group
+                                            : ((uint64_t)a.pieces(nlight) + 3) / 4;
+    const uint64_t cap = alpha_lanes == 16 ? (uint64_t)cus * groups_per_cu : (uint64_t)cus * 8;
+    a.grid = (uint32_t)(want < 1 ? 1 : want < cap ? want : cap);
+    return a;
+}
+
 // Counter reset + persistent kernels over chunks {texture, first block,
 // block count, 0}: the first `nheavy` chunks (any format) go to the LDS
 // encoder (`grid` workgroups of `waves_per_group` = 1, 2 or 4 waves), the
-// next `nlight` (BC4/BC5 only) to the alpha-only launch (launch_alpha_chunks,
-// `grid_light` workgroups, `alpha_lanes` lanes per block), on `s_light` when
-// given (fork/join through the two events) or after the heavy kernel on `s`.
-// d_counter holds two counters.
+// next `nlight` (BC4/BC5 only) to the alpha-only launch (launch_alpha_chunks),
+// on `s_light` when given (fork/join through the two events) or after the
+// heavy kernel on `s`.  d_counter holds two counters.
 hipError_t launch_batch_raw(const BatchTex* d_tex, const uint4* d_chunks, uint32_t nheavy, uint32_t nlight,
-                            uint32_t* d_counter, uint32_t grid, uint32_t grid_light, uint32_t waves_per_group,
+                            uint32_t* d_counter, uint32_t grid, AlphaShape light, uint32_t waves_per_group,
                             uint32_t alpha_lanes, hipStream_t s, hipStream_t s_light, hipEvent_t fork,
                             hipEvent_t join);
-
-// Blocks per chunk of an alpha-only (BC4/BC5) texture encoded one block per
-// lane: the kernel runs 8 steps of 64 blocks per chunk.
-constexpr uint32_t kLightChunkBlocks = 512;
 
 // Persistent kernel over the BC4/BC5 chunks [first, first + nlight):
 // alpha_lanes = 1 runs one block per lane (k_batch_light, 4-wave
 // workgroups); 16 runs a 16-lane group per block (k_batch with
 // `waves_per_group` waves per workgroup).  `d_counter` is its work counter
-// (not reset here).
+// (not reset here; not used when alpha_needs_counter() says so).
 hipError_t launch_alpha_chunks(const BatchTex* d_tex, const uint4* d_chunks, uint32_t first, uint32_t nlight,
-                               uint32_t* d_counter, uint32_t grid, uint32_t alpha_lanes, uint32_t waves_per_group,
+                               uint32_t* d_counter, AlphaShape shape, uint32_t alpha_lanes, uint32_t waves_per_group,
                                hipStream_t s);
 
-// Workgroups of the alpha-only launch for `nlight` chunks on `cus` CUs.
-inline uint32_t alpha_grid(uint32_t cus, uint32_t nlight, uint32_t alpha_lanes, uint32_t groups_per_cu,
-                           uint32_t waves_per_group)
+// Whether the alpha-only kernel draws work from its counter: not when one
+// block per lane leaves each wave at most one piece.
+inline bool alpha_needs_counter(AlphaShape shape, uint32_t nlight, uint32_t alpha_lanes)
 {
-    const uint64_t want = alpha_lanes == 16 ? ((uint64_t)nlight + waves_per_group - 1) / waves_per_group
-                                            : ((uint64_t)nlight + 3) / 4;
-    const uint64_t cap = alpha_lanes == 16 ? (uint64_t)cus * groups_per_cu : (uint64_t)cus * 8;
-    return (uint32_t)(want < 1 ? 1 : want < cap ? want : cap);
+    return alpha_lanes == 16 || (uint64_t)shape.pieces(nlight) > (uint64_t)shape.grid * 4;
 }
 
-// Counter reset (d_counter[0..1]) + the alpha-only kernel over chunks
-// [first, first + nlight) on `s`.
+// Counter reset (d_counter[0..1], where it is needed) + the alpha-only kernel
+// over chunks [first, first + nlight) on `s`.
 hipError_t launch_batch_light(const BatchTex* d_tex, const uint4* d_chunks, uint32_t first, uint32_t nlight,
-                              uint32_t* d_counter, uint32_t grid_light, uint32_t alpha_lanes,
-                              uint32_t waves_per_group, hipStream_t s);
+                              uint32_t* d_counter, AlphaShape shape, uint32_t alpha_lanes, uint32_t waves_per_group,
+                              hipStream_t s);
 
 // Clears d_counter[0..1] on `s` (a kernel: replay-safe inside graphs).
 hipError_t reset_counters(uint32_t* d_counter, hipStream_t s);

@@ -114,19 +114,25 @@ __device__ __forceinline__ void run_chunk_light(const BatchTex& T, uint32_t firs
 
 // Persistent kernel for the alpha-only formats (BC4/BC5): no LDS and few
 // registers, so many waves stay resident to hide memory latency.  Takes
-// chunks [first, first + nchunks), the first by wave index and the rest
-// through its own counter.
+// pieces of `steps` steps of the chunks [first, first + nchunks), the first by
+// wave index and the rest through its own counter (null: there are none).
 __global__ __launch_bounds__(256) void k_batch_light(const BatchTex* __restrict__ tex,
                                                      const uint4* __restrict__ chunks, uint32_t first,
-                                                     uint32_t nchunks, uint32_t* __restrict__ counter)
+                                                     uint32_t npieces, uint32_t steps, uint32_t* __restrict__ counter)
 {
     const int lane = (int)threadIdx.x & 63;
     const uint32_t nwaves = gridDim.x * (blockDim.x >> 6);
-    for (uint32_t c = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); c < nchunks;) {
-        const uint4 ch = chunks[first + c];
-        const BatchTex& T = tex[ch.x];
-        if (T.variant == 9u) run_chunk_light<BC4>(T, ch.y, ch.z, lane);
-        else run_chunk_light<BC5>(T, ch.y, ch.z, lane);
+    const uint32_t per_chunk = txk::kLightChunkBlocks / 64u / steps, span = 64u * steps;
+    for (uint32_t c = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); c < npieces;) {
+        const uint4 ch = chunks[first + c / per_chunk];
+        const uint32_t off = (c % per_chunk) * span;
+        if (off < ch.z) {
+            const BatchTex& T = tex[ch.x];
+            const uint32_t n = min(span, ch.z - off);
+            if (T.variant == 9u) run_chunk_light<BC4>(T, ch.y + off, n, lane);
+            else run_chunk_light<BC5>(T, ch.y + off, n, lane);
+        }
+        if (!counter) break;
         uint32_t next = 0;
         if (lane == 0) next = atomicAdd(counter, 1u);
         c = __builtin_amdgcn_readfirstlane(next) + nwaves;
@@ -152,13 +158,15 @@ hipError_t reset_counters(uint32_t* d_counter, hipStream_t s)
 }
 
 hipError_t launch_alpha_chunks(const BatchTex* d_tex, const uint4* d_chunks, uint32_t first, uint32_t nlight,
-                               uint32_t* d_counter, uint32_t grid, uint32_t alpha_lanes, uint32_t waves_per_group,
+                               uint32_t* d_counter, AlphaShape shape, uint32_t alpha_lanes, uint32_t waves_per_group,
                                hipStream_t s)
 {
     if (nlight == 0) return hipSuccess;
+    const uint32_t grid = shape.grid;
     if (alpha_lanes != 16) {
-        hipLaunchKernelGGL(txd::k_batch_light, dim3(grid), dim3(256), 0, s, d_tex, d_chunks, first, nlight,
-                           d_counter);
+        hipLaunchKernelGGL(txd::k_batch_light, dim3(grid), dim3(256), 0, s, d_tex, d_chunks, first,
+                           shape.pieces(nlight), shape.steps,
+                           alpha_needs_counter(shape, nlight, alpha_lanes) ? d_counter : nullptr);
         return hipGetLastError();
     }
     // 16 lanes per block: the LDS encoder's persistent kernel over the
@@ -178,17 +186,17 @@ hipError_t launch_alpha_chunks(const BatchTex* d_tex, const uint4* d_chunks, uin
 }
 
 hipError_t launch_batch_light(const BatchTex* d_tex, const uint4* d_chunks, uint32_t first, uint32_t nlight,
-                              uint32_t* d_counter, uint32_t grid_light, uint32_t alpha_lanes,
+                              uint32_t* d_counter, AlphaShape shape, uint32_t alpha_lanes,
                               uint32_t waves_per_group, hipStream_t s)
 {
     if (nlight == 0) return hipSuccess;
-    hipLaunchKernelGGL(txd::k_reset_counter, dim3(1), dim3(1), 0, s, d_counter);
-    return launch_alpha_chunks(d_tex, d_chunks, first, nlight, d_counter, grid_light, alpha_lanes, waves_per_group,
-                               s);
+    if (alpha_needs_counter(shape, nlight, alpha_lanes))
+        hipLaunchKernelGGL(txd::k_reset_counter, dim3(1), dim3(1), 0, s, d_counter);
+    return launch_alpha_chunks(d_tex, d_chunks, first, nlight, d_counter, shape, alpha_lanes, waves_per_group, s);
 }
 
 hipError_t launch_batch_raw(const BatchTex* d_tex, const uint4* d_chunks, uint32_t nheavy, uint32_t nlight,
-                            uint32_t* d_counter, uint32_t grid, uint32_t grid_light, uint32_t waves_per_group,
+                            uint32_t* d_counter, uint32_t grid, AlphaShape light, uint32_t waves_per_group,
                             uint32_t alpha_lanes, hipStream_t s, hipStream_t s_light, hipEvent_t fork,
                             hipEvent_t join)
 {
@@ -199,7 +207,7 @@ hipError_t launch_batch_raw(const BatchTex* d_tex, const uint4* d_chunks, uint32
             return hipErrorUnknown;
         sl = s_light;
     }
-    if (nlight && launch_alpha_chunks(d_tex, d_chunks, nheavy, nlight, d_counter + 1, grid_light, alpha_lanes,
+    if (nlight && launch_alpha_chunks(d_tex, d_chunks, nheavy, nlight, d_counter + 1, light, alpha_lanes,
                                       waves_per_group, sl) != hipSuccess)
         return hipErrorUnknown;
     if (nheavy) {
@@ -233,7 +241,8 @@ struct tx_batch {
     uint32_t nheavy = 0;
     uint64_t nblocks = 0;
     tx_batch_tuning tuning{};
-    uint32_t grid = 0, grid_light = 0;
+    uint32_t grid = 0;
+    txk::AlphaShape light{0, 0};
     hipStream_t light_stream = nullptr;  // runs the alpha-only kernel beside the heavy one
     hipEvent_t fork = nullptr, join = nullptr;
     hipGraph_t graph = nullptr;
@@ -276,18 +285,19 @@ hipError_t launch_batch(tx_batch* b, hipStream_t s)
 {
     if (!b->tuning.pipeline || b->nheavy == 0)
         return txk::launch_batch_raw(b->d_tex, b->d_chunks, b->nheavy, b->nchunks - b->nheavy, b->d_counter,
-                                     b->grid, b->grid_light, b->tuning.waves_per_group, b->tuning.lanes_per_block,
+                                     b->grid, b->light, b->tuning.waves_per_group, b->tuning.lanes_per_block,
                                      s, b->light_stream, b->fork, b->join);
     // alpha-only chunks on the side stream, the binned pipeline on `s`
     const uint32_t nlight = b->nchunks - b->nheavy;
-    hipLaunchKernelGGL(txd::k_reset_counter, dim3(1), dim3(1), 0, s, b->d_counter);
+    if (nlight && txk::alpha_needs_counter(b->light, nlight, b->tuning.lanes_per_block))
+        hipLaunchKernelGGL(txd::k_reset_counter, dim3(1), dim3(1), 0, s, b->d_counter);
     hipStream_t sl = s;
     if (nlight && b->light_stream) {
         if (hipEventRecord(b->fork, s) != hipSuccess || hipStreamWaitEvent(b->light_stream, b->fork, 0) != hipSuccess)
             return hipErrorUnknown;
         sl = b->light_stream;
     }
-    if (nlight && txk::launch_alpha_chunks(b->d_tex, b->d_chunks, b->nheavy, nlight, b->d_counter + 1, b->grid_light,
+    if (nlight && txk::launch_alpha_chunks(b->d_tex, b->d_chunks, b->nheavy, nlight, b->d_counter + 1, b->light,
                                            b->tuning.lanes_per_block, b->tuning.waves_per_group, sl) != hipSuccess)
         return hipErrorUnknown;
     txp::PipeLaunch p{};
@@ -296,7 +306,7 @@ hipError_t launch_batch(tx_batch* b, hipStream_t s)
     p.nchunks = b->nheavy;
     p.nslots = b->pipe_slots;
     p.chunk_blocks = b->tuning.chunk_blocks;
-    p.classify_grid = std::min(b->classify_grid, b->nheavy);
+    p.classify_grid = (uint32_t)std::min<uint64_t>(b->classify_grid, txp::classify_pieces(p));
     p.search_grid = b->pipe_grid;
     p.lists = b->pipe_lists;
     const hipError_t e = txp::launch_pipeline(p, b->pipe, s);
@@ -426,8 +436,8 @@ int tx_batch_create(tx_batch** out, const tx_texture* textures, size_t count, co
     // alpha-only kernel: one block per lane in 4-wave workgroups (up to 8 per
     // CU), or 16 lanes per block in the tuned workgroups
     const uint32_t nlight = b->nchunks - b->nheavy;
-    b->grid_light = txk::alpha_grid((uint32_t)prop.multiProcessorCount, nlight, t.lanes_per_block, t.groups_per_cu,
-                                    t.waves_per_group);
+    b->light = txk::alpha_shape((uint32_t)prop.multiProcessorCount, nlight, t.lanes_per_block, t.groups_per_cu,
+                                t.waves_per_group);
     if (nlight && b->nheavy) {
         if (hipStreamCreateWithFlags(&b->light_stream, hipStreamNonBlocking) != hipSuccess ||
             hipEventCreateWithFlags(&b->fork, hipEventDisableTiming) != hipSuccess ||

@@ -129,12 +129,12 @@ __device__ __forceinline__ void classify_chunk(const Grid& G, const BatchTex& T,
     }
 }
 
-// Classify over the heavy chunks (BC1/BC2/BC3 textures) of a batch, each
-// workgroup taking chunks blockIdx.x, blockIdx.x + gridDim.x, ...  Chunk c
-// covers blocks [first, first + count) of one texture and record slots
-// [slot0, slot0 + count).
+// Classify over the heavy chunks (BC1/BC2/BC3 textures) of a batch in pieces of
+// 64 blocks, each workgroup taking pieces blockIdx.x, blockIdx.x + gridDim.x,
+// ...  A chunk covers blocks [first, first + count) of one texture and record
+// slots [slot0, slot0 + count).
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_pipe_classify(
-    const BatchTex* __restrict__ tex, const uint4* __restrict__ chunks, uint32_t nchunks,
+    const BatchTex* __restrict__ tex, const uint4* __restrict__ chunks, uint32_t nchunks, uint32_t chunk_pieces,
     ClusterRec* __restrict__ recs, uint32_t* __restrict__ keys, PipeCtl* __restrict__ ctl)
 {
     __shared__ LaneTables LT;
@@ -143,10 +143,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
     clear_counters(ctl, lane);
     fill_lane_tables(LT, lane);
     group_sync();
-    // chunks hold similar work, so a plain grid-stride loop balances them
+    // pieces hold similar work, so a plain grid-stride loop balances them
     // (a shared work counter would serialise thousands of atomics at launch)
-    for (uint32_t c = blockIdx.x; c < nchunks; c += gridDim.x) {
-        const uint4 ch = chunks[c];
+    for (uint64_t c = blockIdx.x; c < (uint64_t)nchunks * chunk_pieces; c += gridDim.x) {
+        uint4 ch = chunks[c / chunk_pieces];
+        const uint32_t off = (uint32_t)(c % chunk_pieces) * 64u;
+        if (off >= ch.z) continue;
+        ch = make_uint4(ch.x, ch.y + off, min(64u, ch.z - off), ch.w + off);
         const BatchTex& T = tex[ch.x];
         switch (T.variant) {
         case 0: classify_chunk<BC1, RANGE_FIT>(T, T, ch.x, ch.y, ch.z, ch.w, 0u, LT, LB, lane, recs, keys); break;
@@ -617,7 +620,7 @@ hipError_t launch_classify(const PipeLaunch& p, const PipeBufs& b, hipStream_t s
 {
     if (p.d_tex) {
         hipLaunchKernelGGL(txd::k_pipe_classify, dim3(p.classify_grid), dim3(64), 0, s, p.d_tex, p.d_chunks,
-                           p.nchunks, b.recs, b.keys, b.ctl);
+                           p.nchunks, (p.chunk_blocks + 63u) / 64u, b.recs, b.keys, b.ctl);
         return hipSuccess;
     }
     switch (p.tex0.variant) {

@@ -110,12 +110,21 @@ struct PipeLaunch {
     txk::ChainTable chain;       // count > 0: the levels of a chain, tex0 holding what they share and the
                                  // output; implicit chunks, already numbered
     uint32_t nchunks;            // heavy chunks
-    uint32_t chunk_blocks;       // implicit chunk size
+    uint32_t chunk_blocks;       // chunk size (of a chunk list: the largest)
     uint64_t nslots;             // record slots the chunks cover (<= capacity)
     uint32_t classify_grid;      // persistent 64-thread workgroups of classify
     uint32_t search_grid;        // persistent 64-thread workgroups of each search
     uint32_t lists;              // bit L set: records may go to list L (its search is launched)
 };
+
+// 64-block pieces of a chunk list: classify runs one block per lane, so a wave
+// takes a larger chunk piece by piece, each piece by whichever workgroup's
+// turn it is (a small batch tuned with 128-block chunks would otherwise leave
+// half the waves idle and take the others twice as long).
+inline uint64_t classify_pieces(const PipeLaunch& p)
+{
+    return (uint64_t)p.nchunks * ((p.chunk_blocks + 63u) / 64u);
+}
 
 // The lists a texture's records can go to: ClusterFit -> C; BC1
 // IterativeClusterFit -> A and B; BC2/BC3 IterativeClusterFit -> B; RangeFit

@@ -311,10 +311,10 @@ bool tx_server::start_launch(Launch& L, std::vector<uint64_t>& ids, std::unique_
     // no more persistent workgroups than chunks
     const uint32_t launch_grid = (uint32_t)std::min<uint64_t>(
         grid, std::max<uint64_t>(1, (nheavy + cfg.tuning.waves_per_group - 1) / cfg.tuning.waves_per_group));
-    const uint32_t light_grid = txk::alpha_grid(cus, nlight, alpha_lanes, cfg.tuning.groups_per_cu,
-                                                cfg.tuning.waves_per_group);
+    const txk::AlphaShape light = txk::alpha_shape(cus, nlight, alpha_lanes, cfg.tuning.groups_per_cu,
+                                                   cfg.tuning.waves_per_group);
     if (ok && use_pipe) {
-        if (txk::launch_batch_light(L.d_tex, L.d_chunks, nheavy, nlight, L.d_counter + 2, light_grid, alpha_lanes,
+        if (txk::launch_batch_light(L.d_tex, L.d_chunks, nheavy, nlight, L.d_counter + 2, light, alpha_lanes,
                                     cfg.tuning.waves_per_group, L.stream) !=
             hipSuccess)
             ok = false;
@@ -324,12 +324,12 @@ bool tx_server::start_launch(Launch& L, std::vector<uint64_t>& ids, std::unique_
         p.nchunks = nheavy;
         p.nslots = slot;
         p.chunk_blocks = chunk;
-        p.classify_grid = std::min<uint32_t>(cus * txp::kClassifyWavesPerCu, nheavy);
+        p.classify_grid = (uint32_t)std::min<uint64_t>(cus * txp::kClassifyWavesPerCu, txp::classify_pieces(p));
         p.search_grid = (uint32_t)std::min<uint64_t>((uint64_t)cus * txp::kSearchWavesPerCu, (slot + 3) / 4);
         p.lists = lists;
         if (ok && txp::launch_pipeline(p, L.pipe, L.stream) != hipSuccess) ok = false;
     } else if (ok && c &&
-               txk::launch_batch_raw(L.d_tex, L.d_chunks, nheavy, nlight, L.d_counter, launch_grid, light_grid,
+               txk::launch_batch_raw(L.d_tex, L.d_chunks, nheavy, nlight, L.d_counter, launch_grid, light,
                                      cfg.tuning.waves_per_group, alpha_lanes, L.stream, nullptr, nullptr,
                                      nullptr) != hipSuccess) {
         ok = false;
