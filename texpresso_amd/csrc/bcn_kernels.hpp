@@ -92,14 +92,34 @@ inline AlphaShape alpha_shape(uint32_t cus, uint32_t nlight, uint32_t alpha_lane
     return a;
 }
 
+// Launch shape of the LDS encoder over `nheavy` chunks of up to chunk_blocks
+// blocks with at most max_groups workgroups: with fewer chunks than waves each
+// chunk is cut into per_chunk pieces of `span` blocks (a multiple of 4) so
+// that more of the waves have work.
+struct HeavyShape {
+    uint32_t grid, per_chunk, span;
+};
+inline HeavyShape heavy_shape(uint64_t max_groups, uint32_t nheavy, uint32_t waves_per_group, uint32_t chunk_blocks)
+{
+    const uint64_t waves = max_groups * waves_per_group, quads = (chunk_blocks + 3u) / 4u;
+    uint64_t per = nheavy ? waves / nheavy : 1;
+    per = per < 1 ? 1 : per < quads ? per : quads;
+    HeavyShape h;
+    h.span = 4u * (uint32_t)((quads + per - 1) / per);
+    h.per_chunk = (chunk_blocks + h.span - 1u) / h.span;
+    const uint64_t want = ((uint64_t)nheavy * h.per_chunk + waves_per_group - 1) / waves_per_group;
+    h.grid = (uint32_t)(want < 1 ? 1 : want < max_groups ? want : max_groups);
+    return h;
+}
+
 // Counter reset + persistent kernels over chunks {texture, first block,
 // block count, 0}: the first `nheavy` chunks (any format) go to the LDS
-// encoder (`grid` workgroups of `waves_per_group` = 1, 2 or 4 waves), the
+// encoder (workgroups of `waves_per_group` = 1, 2 or 4 waves), the
 // next `nlight` (BC4/BC5 only) to the alpha-only launch (launch_alpha_chunks),
 // on `s_light` when given (fork/join through the two events) or after the
 // heavy kernel on `s`.  d_counter holds two counters.
 hipError_t launch_batch_raw(const BatchTex* d_tex, const uint4* d_chunks, uint32_t nheavy, uint32_t nlight,
-                            uint32_t* d_counter, uint32_t grid, AlphaShape light, uint32_t waves_per_group,
+                            uint32_t* d_counter, HeavyShape heavy, AlphaShape light, uint32_t waves_per_group,
                             uint32_t alpha_lanes, hipStream_t s, hipStream_t s_light, hipEvent_t fork,
                             hipEvent_t join);
 

@@ -42,15 +42,16 @@ __device__ __forceinline__ void run_chunk(const BatchTex& T, uint32_t first, uin
     }
 }
 
-// Persistent kernel: every wave takes chunks {texture, first block, count},
-// the first by its wave index and the rest from `counter`, until the queue
-// is exhausted.  A chunk's texture fixes the format and algorithm for the
-// whole wave, so the dispatch is wave-uniform.  At most 168 registers (three
-// waves per SIMD, the default 12 workgroups of a CU), without spills.
+// Persistent kernel: every wave takes pieces of `span` blocks of the chunks
+// {texture, first block, count} (per_chunk pieces each), the first by its wave
+// index and the rest from `counter`, until the queue is exhausted.  A chunk's
+// texture fixes the format and algorithm for the whole wave, so the dispatch
+// is wave-uniform.  At most 168 registers (three waves per SIMD, the default
+// 12 workgroups of a CU).
 template <int WAVES>
 __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(3))) void k_batch(
-    const BatchTex* __restrict__ tex, const uint4* __restrict__ chunks, uint32_t nchunks,
-    uint32_t* __restrict__ counter)
+    const BatchTex* __restrict__ tex, const uint4* __restrict__ chunks, uint32_t nchunks, uint32_t per_chunk,
+    uint32_t span, uint32_t* __restrict__ counter)
 {
     __shared__ GroupLds lds[4 * WAVES];
     const int tid = (int)threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -58,9 +59,12 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(3)))
     GroupLds& L = lds[4 * wave + g];
     // first chunk by wave index, later ones from the counter (offset past
     // those), so the launch does not open with one atomic per wave
-    const uint32_t nwaves = gridDim.x * WAVES;
-    for (uint32_t c = blockIdx.x * WAVES + (uint32_t)wave; c < nchunks;) {
-        const uint4 ch = chunks[c];
+    const uint32_t nwaves = gridDim.x * WAVES, npieces = nchunks * per_chunk;
+    for (uint32_t c = blockIdx.x * WAVES + (uint32_t)wave; c < npieces;) {
+        uint4 ch = chunks[c / per_chunk];
+        const uint32_t off = (c % per_chunk) * span;
+        ch.y += off;
+        ch.z = off < ch.z ? min(span, ch.z - off) : 0u;
         const BatchTex& T = tex[ch.x];
         switch (T.variant) {
         case 0: run_chunk<BC1, RANGE_FIT>(T, ch.y, ch.z, L, g, l); break;
@@ -173,13 +177,16 @@ hipError_t launch_alpha_chunks(const BatchTex* d_tex, const uint4* d_chunks, uin
     // alpha-only chunks (it dispatches BC4/BC5 chunks to the group code)
     switch (waves_per_group) {
     case 4:
-        hipLaunchKernelGGL(txd::k_batch<4>, dim3(grid), dim3(256), 0, s, d_tex, d_chunks + first, nlight, d_counter);
+        hipLaunchKernelGGL(txd::k_batch<4>, dim3(grid), dim3(256), 0, s, d_tex, d_chunks + first, nlight, 1u, ~0u,
+                           d_counter);
         break;
     case 2:
-        hipLaunchKernelGGL(txd::k_batch<2>, dim3(grid), dim3(128), 0, s, d_tex, d_chunks + first, nlight, d_counter);
+        hipLaunchKernelGGL(txd::k_batch<2>, dim3(grid), dim3(128), 0, s, d_tex, d_chunks + first, nlight, 1u, ~0u,
+                           d_counter);
         break;
     default:
-        hipLaunchKernelGGL(txd::k_batch<1>, dim3(grid), dim3(64), 0, s, d_tex, d_chunks + first, nlight, d_counter);
+        hipLaunchKernelGGL(txd::k_batch<1>, dim3(grid), dim3(64), 0, s, d_tex, d_chunks + first, nlight, 1u, ~0u,
+                           d_counter);
         break;
     }
     return hipGetLastError();
@@ -196,7 +203,7 @@ hipError_t launch_batch_light(const BatchTex* d_tex, const uint4* d_chunks, uint
 }
 
 hipError_t launch_batch_raw(const BatchTex* d_tex, const uint4* d_chunks, uint32_t nheavy, uint32_t nlight,
-                            uint32_t* d_counter, uint32_t grid, AlphaShape light, uint32_t waves_per_group,
+                            uint32_t* d_counter, HeavyShape heavy, AlphaShape light, uint32_t waves_per_group,
                             uint32_t alpha_lanes, hipStream_t s, hipStream_t s_light, hipEvent_t fork,
                             hipEvent_t join)
 {
@@ -213,13 +220,16 @@ hipError_t launch_batch_raw(const BatchTex* d_tex, const uint4* d_chunks, uint32
     if (nheavy) {
         switch (waves_per_group) {
         case 4:
-            hipLaunchKernelGGL(txd::k_batch<4>, dim3(grid), dim3(256), 0, s, d_tex, d_chunks, nheavy, d_counter);
+            hipLaunchKernelGGL(txd::k_batch<4>, dim3(heavy.grid), dim3(256), 0, s, d_tex, d_chunks, nheavy,
+                               heavy.per_chunk, heavy.span, d_counter);
             break;
         case 2:
-            hipLaunchKernelGGL(txd::k_batch<2>, dim3(grid), dim3(128), 0, s, d_tex, d_chunks, nheavy, d_counter);
+            hipLaunchKernelGGL(txd::k_batch<2>, dim3(heavy.grid), dim3(128), 0, s, d_tex, d_chunks, nheavy,
+                               heavy.per_chunk, heavy.span, d_counter);
             break;
         default:
-            hipLaunchKernelGGL(txd::k_batch<1>, dim3(grid), dim3(64), 0, s, d_tex, d_chunks, nheavy, d_counter);
+            hipLaunchKernelGGL(txd::k_batch<1>, dim3(heavy.grid), dim3(64), 0, s, d_tex, d_chunks, nheavy,
+                               heavy.per_chunk, heavy.span, d_counter);
             break;
         }
     }
@@ -241,7 +251,7 @@ struct tx_batch {
     uint32_t nheavy = 0;
     uint64_t nblocks = 0;
     tx_batch_tuning tuning{};
-    uint32_t grid = 0;
+    txk::HeavyShape heavy{0, 1, 0};
     txk::AlphaShape light{0, 0};
     hipStream_t light_stream = nullptr;  // runs the alpha-only kernel beside the heavy one
     hipEvent_t fork = nullptr, join = nullptr;
@@ -285,7 +295,7 @@ hipError_t launch_batch(tx_batch* b, hipStream_t s)
 {
     if (!b->tuning.pipeline || b->nheavy == 0)
         return txk::launch_batch_raw(b->d_tex, b->d_chunks, b->nheavy, b->nchunks - b->nheavy, b->d_counter,
-                                     b->grid, b->light, b->tuning.waves_per_group, b->tuning.lanes_per_block,
+                                     b->heavy, b->light, b->tuning.waves_per_group, b->tuning.lanes_per_block,
                                      s, b->light_stream, b->fork, b->join);
     // alpha-only chunks on the side stream, the binned pipeline on `s`
     const uint32_t nlight = b->nchunks - b->nheavy;
@@ -430,9 +440,8 @@ int tx_batch_create(tx_batch** out, const tx_texture* textures, size_t count, co
         return TX_ERR_HIP;
     }
     // persistent workgroups: the tuned count, but never more than there are chunks
-    b->grid = (uint32_t)std::min<uint64_t>((uint64_t)prop.multiProcessorCount * t.groups_per_cu,
-                                           std::max<uint64_t>(1, (b->nheavy + t.waves_per_group - 1) /
-                                                                     t.waves_per_group));
+    b->heavy = txk::heavy_shape((uint64_t)prop.multiProcessorCount * t.groups_per_cu, b->nheavy, t.waves_per_group,
+                                t.chunk_blocks);
     // alpha-only kernel: one block per lane in 4-wave workgroups (up to 8 per
     // CU), or 16 lanes per block in the tuned workgroups
     const uint32_t nlight = b->nchunks - b->nheavy;

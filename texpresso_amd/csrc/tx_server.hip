@@ -308,9 +308,7 @@ bool tx_server::start_launch(Launch& L, std::vector<uint64_t>& ids, std::unique_
     if (ok && c && hipMemcpyAsync(L.d_chunks, L.h_chunks, sizeof(uint4) * c, hipMemcpyHostToDevice, L.stream) !=
                        hipSuccess)
         ok = false;
-    // no more persistent workgroups than chunks
-    const uint32_t launch_grid = (uint32_t)std::min<uint64_t>(
-        grid, std::max<uint64_t>(1, (nheavy + cfg.tuning.waves_per_group - 1) / cfg.tuning.waves_per_group));
+    const txk::HeavyShape heavy = txk::heavy_shape(grid, nheavy, cfg.tuning.waves_per_group, chunk);
     const txk::AlphaShape light = txk::alpha_shape(cus, nlight, alpha_lanes, cfg.tuning.groups_per_cu,
                                                    cfg.tuning.waves_per_group);
     if (ok && use_pipe) {
@@ -329,7 +327,7 @@ bool tx_server::start_launch(Launch& L, std::vector<uint64_t>& ids, std::unique_
         p.lists = lists;
         if (ok && txp::launch_pipeline(p, L.pipe, L.stream) != hipSuccess) ok = false;
     } else if (ok && c &&
-               txk::launch_batch_raw(L.d_tex, L.d_chunks, nheavy, nlight, L.d_counter, launch_grid, light,
+               txk::launch_batch_raw(L.d_tex, L.d_chunks, nheavy, nlight, L.d_counter, heavy, light,
                                      cfg.tuning.waves_per_group, alpha_lanes, L.stream, nullptr, nullptr,
                                      nullptr) != hipSuccess) {
         ok = false;
