@@ -538,6 +538,12 @@ __global__ __launch_bounds__(64 * kSearchWaves) __attribute__((amdgpu_waves_per_
 // workgroup's kSearchWaves waves take their positions, four per step, from
 // one shared run, so at the end of the list no wave holds steps that an
 // idle wave could have run.
+// A list too short for refills of four steps (64 positions a workgroup) has no
+// refills: workgroup i of G owns steps i, i + G, i + 2G, ..., and its run
+// counts those.  All waves finish a step at about the same time, and refills of
+// one step queued on the cursor: 31,000 BC3 records took 139 us, now 88.  With
+// full refills the cursor's balance is the better one: 65,000 BC1 and 97,000
+// BC2 records take 203 and 250 us with it, 212 and 255 dealt out.
 __global__ __launch_bounds__(64 * kSearchWaves) __attribute__((amdgpu_waves_per_eu(4))) void k_pipe_cluster(
     const BatchTex* __restrict__ tex, BatchTex tex0, const ClusterRec* __restrict__ recs,
     const uint32_t* __restrict__ slots, uint32_t nslots, PipeCtl* __restrict__ ctl)
@@ -550,15 +556,15 @@ __global__ __launch_bounds__(64 * kSearchWaves) __attribute__((amdgpu_waves_per_
     const int lane = (int)(threadIdx.x & 63u), g = lane >> 4, l = lane & 15;
     GroupLds& L = lds[4 * (threadIdx.x >> 6) + g];
     const uint32_t total = list.total();
-    // refills of up to four steps for one wave (16 positions), at most the
-    // records per wave; the first run of each workgroup is fixed by its
-    // index, refills come from the shared cursor, offset past those runs
-    const uint32_t kRefill = 4u * min(4u, max(1u, total / (4u * kSearchWaves * gridDim.x)));
-    const uint32_t kFirst = kSearchWaves * kRefill;
+    // refills of four steps for one wave; the first run of each workgroup is
+    // fixed by its index, refills come from the shared cursor, offset past
+    // those runs
+    const uint32_t kRefill = 16u, kFirst = kSearchWaves * kRefill;
     const uint32_t cursor_base = gridDim.x * kFirst;
+    const bool dealt = total < kFirst * gridDim.x;
     if (threadIdx.x == 0) {
-        const uint32_t first = blockIdx.x * kFirst;
-        run = ((uint64_t)(first + kFirst) << 32) | first;
+        const uint32_t first = dealt ? 0u : blockIdx.x * kFirst;
+        run = ((uint64_t)(dealt ? ~0u : first + kFirst) << 32) | first;
         refilling = 0u;
     }
     __syncthreads();
@@ -566,7 +572,8 @@ __global__ __launch_bounds__(64 * kSearchWaves) __attribute__((amdgpu_waves_per_
         uint32_t pos[4] = {0u, 0u, 0u, 0u};
         if (lane == 0) take_positions(&run, &refilling, cursor, cursor_base, kRefill, 4u, pos);
         const uint32_t p0 = lane0(pos[0]), p1 = lane0(pos[1]), p2 = lane0(pos[2]), p3 = lane0(pos[3]);
-        const uint32_t p = g == 0 ? p0 : g == 1 ? p1 : g == 2 ? p2 : p3;
+        uint32_t p = g == 0 ? p0 : g == 1 ? p1 : g == 2 ? p2 : p3;
+        if (dealt) p = ((p >> 2) * gridDim.x + blockIdx.x) * 4u + (p & 3u);
         const bool has = p < total;
         if (!wave_any(has)) break;
         ColourSet cs{0, -1, false};
