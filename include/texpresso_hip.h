@@ -296,11 +296,17 @@ int tx_util_time_phases(int format, const uint8_t* d_rgba, size_t width, size_t 
                         uint8_t* d_output, size_t out_len, int iters, float ms_phase[4], int* used_pipeline);
 
 /* BC2/BC3 IterativeClusterFit textures with at least `min_blocks` blocks are
- * encoded by the binned pipeline (classify, counting sort by colour count,
+ * encoded by the binned pipeline (classify, binning by colour count,
  * per-block independent searches), smaller ones by the single direct kernel;
+ * other formats and algorithms use a multiple of this threshold (the measured
+ * crossovers).  On a caller's stream, and in tx_compress_device_noalloc,
  * BC2/BC3 ClusterFit use 1.25x, BC1 ClusterFit 1.5x and BC1
- * IterativeClusterFit 3x this threshold (the measured crossovers).  Both
- * paths give identical bytes.  0 = always the pipeline, UINT64_MAX = never.
+ * IterativeClusterFit 3x; on the library's own stream, where calls do not
+ * overlap, ClusterFit uses 0.5625x and BC1 IterativeClusterFit 1.75x.  A
+ * stream being captured into a graph always gets the direct kernels (except
+ * in tx_compress_device_noalloc).  A mip chain counts as one texture of all
+ * its levels' blocks.  Both paths give identical bytes.  0 = always the
+ * pipeline, UINT64_MAX = never.
  * Process-wide; returns the previous value (default 32768). */
 uint64_t tx_set_pipeline_threshold(uint64_t min_blocks);
 

@@ -172,26 +172,39 @@ static txk::EncodeArgs encode_args(int format, const tx_params* p, const uint8_t
     return a;
 }
 
-// Blocks from which a texture goes through the binned pipeline: the set
-// threshold for BC2/BC3 IterativeClusterFit, 1.25x for BC2/BC3 ClusterFit,
-// 1.5x for BC1 ClusterFit and 3x for BC1 IterativeClusterFit (measured
-// crossovers against the direct kernel, 256^2-1448^2: BC1's two search
-// passes and single-ordering blocks gain less from independent per-block
-// scheduling).
-static uint64_t pipeline_threshold(int format, int algorithm)
+// Blocks from which a texture goes through the binned pipeline, as a share of
+// the set threshold (default 32,768), in sixteenths: the measured crossings
+// against the direct kernels (square seeded textures, pipeline / direct us).
+// On the library's own stream calls run one after another: BC2/BC3
+// IterativeClusterFit 205 / 196 at 30,976 blocks, 220 / 239 at 36,864; BC1
+// IterativeClusterFit 253 / 250 at 50,176, 263 / 263 at 57,600; ClusterFit BC1
+// 58 / 59 at 16,384 (the direct kernel's last full round of waves), 68 / 84 at
+// 25,600, BC3 54 / 52 and 78 / 82.  Calls on a caller's stream may overlap
+// those on other streams, which only the direct kernels allow (three streams,
+// BC1 ClusterFit, per call: 100 / 73 at 40,000 blocks), so there the pipeline
+// starts later.
+static uint64_t pipeline_threshold(int format, int algorithm, bool own_stream)
 {
     const uint64_t t = txc::pipeline_min_blocks();
     const bool bc1 = format == TX_BC1, iterative = algorithm == TX_ITERATIVE_CLUSTER_FIT;
-    const uint64_t quarters = bc1 ? (iterative ? 12 : 6) : (iterative ? 4 : 5);
-    return t > UINT64_MAX / quarters ? UINT64_MAX : t * quarters / 4;
+    uint64_t sixteenths = bc1 ? (iterative ? 48 : 24) : (iterative ? 16 : 20);
+    if (own_stream) sixteenths = iterative ? (bc1 ? 28 : 16) : 9;
+    return t > UINT64_MAX / sixteenths ? UINT64_MAX : t * sixteenths / 16;
 }
 
 // Whether a texture goes through the binned pipeline: ClusterFit or
 // IterativeClusterFit in BC1-BC3 with at least pipeline_threshold() blocks.
-static bool takes_pipeline(const txk::EncodeArgs& a)
+static bool takes_pipeline(const txk::EncodeArgs& a, bool own_stream)
 {
     const bool cluster = a.format <= TX_BC3 && a.algorithm != TX_RANGE_FIT;
-    return cluster && a.nblocks >= pipeline_threshold(a.format, a.algorithm) && a.nblocks <= 0xFFFFFFFFull;
+    return cluster && a.nblocks >= pipeline_threshold(a.format, a.algorithm, own_stream) && a.nblocks <= 0xFFFFFFFFull;
+}
+
+// Whether `s` is being captured into a graph.
+static bool capturing(hipStream_t s)
+{
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(s, &status) == hipSuccess && status != hipStreamCaptureStatusNone;
 }
 
 // Launch shape of the binned pipeline for one texture, or for the levels of
@@ -244,7 +257,11 @@ static hipError_t encode_on(txc::DeviceContext* ctx, const txk::EncodeArgs& a, h
                             bool* used_pipeline = nullptr)
 {
     if (used_pipeline) *used_pipeline = false;
-    if (!takes_pipeline(a)) return chain ? txk::launch_encode_chain(a, *chain, s) : txk::launch_encode(a, s);
+    // the pipeline's shared buffers are ordered between streams by events, which
+    // a captured stream cannot wait for
+    const bool own = s == ctx->stream;
+    if (!takes_pipeline(a, own) || (!own && capturing(s)))
+        return chain ? txk::launch_encode_chain(a, *chain, s) : txk::launch_encode(a, s);
     if (used_pipeline) *used_pipeline = true;
     std::lock_guard<std::mutex> lock(ctx->pipe_mu);
     txp::PipeBufs bufs;
@@ -373,7 +390,7 @@ int tx_compress_device_noalloc(int format, const uint8_t* d_rgba, size_t width, 
     if (rc != TX_OK) return rc;
     const hipStream_t s = (hipStream_t)stream;
     const txk::EncodeArgs a = encode_args(format, params, d_rgba, width, height, d_output, out_len);
-    if (!takes_pipeline(a)) return txk::launch_encode(a, s) == hipSuccess ? TX_OK : TX_ERR_HIP;
+    if (!takes_pipeline(a, false)) return txk::launch_encode(a, s) == hipSuccess ? TX_OK : TX_ERR_HIP;
     if (a.nblocks > TX_NOALLOC_MAX_PIPELINE_BLOCKS) return TX_ERR_TOO_LARGE;
     txp::PipeBufs bufs;
     bufs.carve(dev->ptr, TX_NOALLOC_MAX_PIPELINE_BLOCKS);
