@@ -260,12 +260,17 @@ static hipError_t encode_on(txc::DeviceContext* ctx, const txk::EncodeArgs& a, h
     // the pipeline's shared buffers are ordered between streams by events, which
     // a captured stream cannot wait for
     const bool own = s == ctx->stream;
-    if (!takes_pipeline(a, own) || (!own && capturing(s)))
-        return chain ? txk::launch_encode_chain(a, *chain, s) : txk::launch_encode(a, s);
-    if (used_pipeline) *used_pipeline = true;
+    const auto direct = [&] { return chain ? txk::launch_encode_chain(a, *chain, s) : txk::launch_encode(a, s); };
+    if (!takes_pipeline(a, own) || (!own && capturing(s))) return direct();
     std::lock_guard<std::mutex> lock(ctx->pipe_mu);
     txp::PipeBufs bufs;
-    if (!ctx->pipe_scratch(a.nblocks, &bufs)) return hipErrorOutOfMemory;
+    if (!ctx->pipe_scratch(a.nblocks, &bufs)) {
+        // no memory for the records; the direct kernels need none.  The failed
+        // allocation must not be taken for a failed launch.
+        (void)hipGetLastError();
+        return direct();
+    }
+    if (used_pipeline) *used_pipeline = true;
     if (!ctx->pipe_before(s)) return hipErrorUnknown;
     const hipError_t e = txp::launch_pipeline(pipe_launch_for(a, chain, (uint32_t)ctx->cus), bufs, s, marks);
     if (!ctx->pipe_after(s)) return hipErrorUnknown;
