@@ -156,7 +156,8 @@ typedef struct {
 } tx_texture;
 
 typedef struct {
-    uint32_t chunk_blocks;     /* blocks per work-queue chunk (multiple of 4) */
+    uint32_t chunk_blocks;     /* blocks per work-queue chunk: any multiple of 4 up to 2^32 - 4
+                                  (a size above a texture's does not split it) */
     uint32_t waves_per_group;  /* waves per workgroup: 1, 2 or 4 (4 blocks per wave) */
     uint32_t groups_per_cu;    /* persistent workgroups per compute unit */
     uint32_t use_graph;        /* 1: capture the launch in a hipGraph and replay it */
@@ -183,7 +184,7 @@ int tx_batch_run(tx_batch* batch, void* stream);
 /* Enqueues the pass and waits for it; returns the elapsed ms (HIP events). */
 int tx_batch_run_timed(tx_batch* batch, int iters, float* ms_total);
 int tx_batch_destroy(tx_batch* batch);
-/* Number of chunks and blocks in the batch. */
+/* Number of chunks (of the tuned sizes) and blocks in the batch. */
 int tx_batch_info(const tx_batch* batch, uint64_t* chunks, uint64_t* blocks);
 
 /* Autotuner: times every tuning of the candidate grid on these textures and

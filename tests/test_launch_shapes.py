@@ -1,0 +1,58 @@
+"""Launch shapes computed on the host, without a GPU: for every chunk size and
+number of chunks a batch may have, the pieces of the lockstep encoder's launch
+cover each chunk, and the piece count fits the kernel's 32 bits."""
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+SOURCE = r"""
+#include <stdio.h>
+#include "bcn_kernels.hpp"
+int main()
+{
+    unsigned long long groups; unsigned n, wpg, largest;
+    while (scanf("%llu %u %u %u", &groups, &n, &wpg, &largest) == 4) {
+        const txk::HeavyShape h = txk::heavy_shape(groups, n, wpg, largest);
+        printf("%u %u %u\n", h.grid, h.per_chunk, h.span);
+    }
+    return 0;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def shapes(tmp_path_factory):
+    d = tmp_path_factory.mktemp("shapes")
+    src, exe = d / "shapes.cpp", d / "shapes"
+    src.write_text(SOURCE)
+    subprocess.run([os.environ.get("CXX", "g++"), "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    "-I" + os.path.join(ROOT, "texpresso_amd", "csrc"), str(src), "-o", str(exe)], check=True)
+
+    def run(rows):
+        out = subprocess.run([str(exe)], input="".join("%d %d %d %d\n" % r for r in rows), text=True, check=True,
+                             stdout=subprocess.PIPE).stdout
+        return [tuple(map(int, line.split())) for line in out.splitlines()]
+
+    return run
+
+
+def test_heavy_pieces_cover_every_chunk(shapes):
+    sizes = [4, 8, 60, 64, 68, 128, 4096, 1 << 20, 1 << 30, (1 << 31) - 4, 1 << 31, (1 << 31) + 4, 0xFFFFFFC0,
+             0xFFFFFFC4, 0xFFFFFFF8, 0xFFFFFFFC]
+    rows = [(256 * g, n, w, c) for g in (1, 12, 64) for w in (1, 2, 4) for c in sizes
+            for n in (1, 2, 3, 7, 100, 2000, 3071, 3072, 3073, 100000)]
+    for (groups, n, wpg, chunk), (grid, per_chunk, span) in zip(rows, shapes(rows)):
+        case = (groups, n, wpg, chunk, grid, per_chunk, span)
+        assert per_chunk >= 1 and span >= 4 and span % 4 == 0, case
+        assert per_chunk * span >= chunk > (per_chunk - 1) * span, case
+        assert n * per_chunk < 1 << 32 and n * per_chunk <= max(n, groups * wpg), case
+        assert 1 <= grid <= groups, case
+
+
+def test_no_chunks_and_single_blocks(shapes):
+    # no chunks at all (a batch without colour textures), and chunks below one step
+    for grid, per_chunk, span in shapes([(3072, 0, 1, 0), (3072, 0, 4, 0), (3072, 1, 1, 1), (3072, 1, 2, 3)]):
+        assert (grid, per_chunk, span) == (1, 1, 4)

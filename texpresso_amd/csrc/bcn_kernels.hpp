@@ -92,21 +92,24 @@ inline AlphaShape alpha_shape(uint32_t cus, uint32_t nlight, uint32_t alpha_lane
     return a;
 }
 
-// Launch shape of the LDS encoder over `nheavy` chunks of up to chunk_blocks
-// blocks with at most max_groups workgroups: with fewer chunks than waves each
-// chunk is cut into per_chunk pieces of `span` blocks (a multiple of 4) so
-// that more of the waves have work.
+// Launch shape of the LDS encoder over `nheavy` chunks, the largest of
+// `largest` blocks, with at most max_groups workgroups: with fewer chunks than
+// waves each chunk is cut into per_chunk pieces of `span` blocks (a multiple of
+// 4) so that more of the waves have work.  `largest` counts the chunks as they
+// are: a tuning may name any size up to 2^32 - 4, and sizes this near 2^32 are
+// rounded up in 64 bits.
 struct HeavyShape {
     uint32_t grid, per_chunk, span;
 };
-inline HeavyShape heavy_shape(uint64_t max_groups, uint32_t nheavy, uint32_t waves_per_group, uint32_t chunk_blocks)
+inline HeavyShape heavy_shape(uint64_t max_groups, uint32_t nheavy, uint32_t waves_per_group, uint32_t largest)
 {
-    const uint64_t waves = max_groups * waves_per_group, quads = (chunk_blocks + 3u) / 4u;
-    uint64_t per = nheavy ? waves / nheavy : 1;
+    const uint64_t quads = largest ? ((uint64_t)largest + 3) / 4 : 1;
+    uint64_t per = nheavy ? max_groups * waves_per_group / nheavy : 1;
     per = per < 1 ? 1 : per < quads ? per : quads;
+    const uint64_t span = 4 * ((quads + per - 1) / per);
     HeavyShape h;
-    h.span = 4u * (uint32_t)((quads + per - 1) / per);
-    h.per_chunk = (chunk_blocks + h.span - 1u) / h.span;
+    h.span = (uint32_t)(span < 0xFFFFFFFCull ? span : 0xFFFFFFFCull);
+    h.per_chunk = (uint32_t)((4 * quads + h.span - 1) / h.span);
     const uint64_t want = ((uint64_t)nheavy * h.per_chunk + waves_per_group - 1) / waves_per_group;
     h.grid = (uint32_t)(want < 1 ? 1 : want < max_groups ? want : max_groups);
     return h;

@@ -247,7 +247,8 @@ struct tx_batch {
     txd::BatchTex* d_tex = nullptr;
     uint4* d_chunks = nullptr;
     uint32_t* d_counter = nullptr;
-    uint32_t nchunks = 0;  // heavy chunks first, then the alpha-only ones
+    uint32_t nchunks = 0;  // listed: heavy chunks first, then the alpha-only ones
+    uint64_t tuned_chunks = 0;  // of the tuned size (tx_batch_info)
     uint32_t nheavy = 0;
     uint64_t nblocks = 0;
     tx_batch_tuning tuning{};
@@ -315,8 +316,7 @@ hipError_t launch_batch(tx_batch* b, hipStream_t s)
     p.d_chunks = b->d_chunks;
     p.nchunks = b->nheavy;
     p.nslots = b->pipe_slots;
-    p.chunk_blocks = b->tuning.chunk_blocks;
-    p.classify_grid = (uint32_t)std::min<uint64_t>(b->classify_grid, txp::classify_pieces(p));
+    p.classify_grid = std::min(b->classify_grid, b->nheavy);
     p.search_grid = b->pipe_grid;
     p.lists = b->pipe_lists;
     const hipError_t e = txp::launch_pipeline(p, b->pipe, s);
@@ -378,7 +378,7 @@ int tx_batch_create(tx_batch** out, const tx_texture* textures, size_t count, co
     std::vector<txd::BatchTex> tex(count);
     std::vector<uint4> chunks;
     std::vector<uint32_t> cls;
-    uint64_t nblocks = 0;
+    uint64_t nblocks = 0, tuned_chunks = 0;
     for (size_t i = 0; i < count; ++i) {
         const tx_texture& s = textures[i];
         if (!valid_texture(s)) return TX_ERR_INVALID;
@@ -401,9 +401,12 @@ int tx_batch_create(tx_batch** out, const tx_texture* textures, size_t count, co
         d.wb = s.params.weights[2];
         d.weigh_alpha = s.params.weigh_colour_by_alpha ? 1u : 0u;
         // alpha-only textures one block per lane take larger chunks
-        const uint32_t cb = (cost_class(s) == 0 && t.lanes_per_block == 1) ? txk::kLightChunkBlocks : t.chunk_blocks;
-        for (uint32_t f = 0; f < d.nblocks; f += cb) {
-            chunks.push_back(make_uint4((uint32_t)i, f, std::min(cb, d.nblocks - f), 0u));
+        uint32_t cb = (cost_class(s) == 0 && t.lanes_per_block == 1) ? txk::kLightChunkBlocks : t.chunk_blocks;
+        tuned_chunks += (nb + cb - 1) / cb;
+        // the pipeline's classify pass works in steps of kClassifyBlocks
+        if (t.pipeline && cost_class(s) > 0) cb = std::min(cb, txp::kClassifyBlocks);
+        for (uint64_t f = 0; f < nb; f += cb) {
+            chunks.push_back(make_uint4((uint32_t)i, (uint32_t)f, (uint32_t)std::min<uint64_t>(cb, nb - f), 0u));
             cls.push_back(cost_class(s));
         }
         nblocks += nb;
@@ -416,9 +419,11 @@ int tx_batch_create(tx_batch** out, const tx_texture* textures, size_t count, co
     // heavy chunks also get their first record slot of the binned pipeline
     std::vector<uint4> sorted(chunks.size());
     uint64_t slots = 0;
+    uint32_t largest = 0;
     for (size_t i = 0; i < order.size(); ++i) {
         sorted[i] = chunks[order[i]];
         if (cls[order[i]] > 0) {
+            largest = std::max(largest, sorted[i].z);
             sorted[i].w = (uint32_t)slots;
             slots += sorted[i].z;
         }
@@ -433,6 +438,7 @@ int tx_batch_create(tx_batch** out, const tx_texture* textures, size_t count, co
     b->nheavy = 0;
     for (size_t i = 0; i < order.size(); ++i) b->nheavy += cls[order[i]] > 0 ? 1u : 0u;
     b->nblocks = nblocks;
+    b->tuned_chunks = tuned_chunks;
     hipDeviceProp_t prop;
     if (hipEventCreateWithFlags(&b->done, hipEventDisableTiming) != hipSuccess ||
         hipGetDeviceProperties(&prop, ctx->device) != hipSuccess) {
@@ -441,7 +447,7 @@ int tx_batch_create(tx_batch** out, const tx_texture* textures, size_t count, co
     }
     // persistent workgroups: the tuned count, but never more than there are chunks
     b->heavy = txk::heavy_shape((uint64_t)prop.multiProcessorCount * t.groups_per_cu, b->nheavy, t.waves_per_group,
-                                t.chunk_blocks);
+                                largest);
     // alpha-only kernel: one block per lane in 4-wave workgroups (up to 8 per
     // CU), or 16 lanes per block in the tuned workgroups
     const uint32_t nlight = b->nchunks - b->nheavy;
@@ -561,7 +567,7 @@ int tx_batch_destroy(tx_batch* b)
 int tx_batch_info(const tx_batch* b, uint64_t* chunks, uint64_t* blocks)
 {
     if (!b) return TX_ERR_INVALID;
-    if (chunks) *chunks = b->nchunks;
+    if (chunks) *chunks = b->tuned_chunks;
     if (blocks) *blocks = b->nblocks;
     return TX_OK;
 }

@@ -129,12 +129,12 @@ __device__ __forceinline__ void classify_chunk(const Grid& G, const BatchTex& T,
     }
 }
 
-// Classify over the heavy chunks (BC1/BC2/BC3 textures) of a batch in pieces of
-// 64 blocks, each workgroup taking pieces blockIdx.x, blockIdx.x + gridDim.x,
-// ...  A chunk covers blocks [first, first + count) of one texture and record
-// slots [slot0, slot0 + count).
+// Classify over the heavy chunks (BC1/BC2/BC3 textures) of a batch, each
+// workgroup taking chunks blockIdx.x, blockIdx.x + gridDim.x, ...  A chunk
+// covers blocks [first, first + count) of one texture and record slots
+// [slot0, slot0 + count).
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_pipe_classify(
-    const BatchTex* __restrict__ tex, const uint4* __restrict__ chunks, uint32_t nchunks, uint32_t chunk_pieces,
+    const BatchTex* __restrict__ tex, const uint4* __restrict__ chunks, uint32_t nchunks,
     ClusterRec* __restrict__ recs, uint32_t* __restrict__ keys, PipeCtl* __restrict__ ctl)
 {
     __shared__ LaneTables LT;
@@ -143,13 +143,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
     clear_counters(ctl, lane);
     fill_lane_tables(LT, lane);
     group_sync();
-    // pieces hold similar work, so a plain grid-stride loop balances them
+    // chunks hold similar work, so a plain grid-stride loop balances them
     // (a shared work counter would serialise thousands of atomics at launch)
-    for (uint64_t c = blockIdx.x; c < (uint64_t)nchunks * chunk_pieces; c += gridDim.x) {
-        uint4 ch = chunks[c / chunk_pieces];
-        const uint32_t off = (uint32_t)(c % chunk_pieces) * 64u;
-        if (off >= ch.z) continue;
-        ch = make_uint4(ch.x, ch.y + off, min(64u, ch.z - off), ch.w + off);
+    for (uint32_t c = blockIdx.x; c < nchunks; c += gridDim.x) {
+        const uint4 ch = chunks[c];
         const BatchTex& T = tex[ch.x];
         switch (T.variant) {
         case 0: classify_chunk<BC1, RANGE_FIT>(T, T, ch.x, ch.y, ch.z, ch.w, 0u, LT, LB, lane, recs, keys); break;
@@ -627,18 +624,19 @@ hipError_t launch_classify(const PipeLaunch& p, const PipeBufs& b, hipStream_t s
 {
     if (p.d_tex) {
         hipLaunchKernelGGL(txd::k_pipe_classify, dim3(p.classify_grid), dim3(64), 0, s, p.d_tex, p.d_chunks,
-                           p.nchunks, (p.chunk_blocks + 63u) / 64u, b.recs, b.keys, b.ctl);
-        return hipSuccess;
+                           p.nchunks, b.recs, b.keys, b.ctl);
+        return hipGetLastError();
     }
     switch (p.tex0.variant) {
-    case 1: launch_classify_one<0, 1>(p, b, s); return hipSuccess;
-    case 2: launch_classify_one<0, 2>(p, b, s); return hipSuccess;
-    case 4: launch_classify_one<1, 1>(p, b, s); return hipSuccess;
-    case 5: launch_classify_one<1, 2>(p, b, s); return hipSuccess;
-    case 7: launch_classify_one<2, 1>(p, b, s); return hipSuccess;
-    case 8: launch_classify_one<2, 2>(p, b, s); return hipSuccess;
+    case 1: launch_classify_one<0, 1>(p, b, s); break;
+    case 2: launch_classify_one<0, 2>(p, b, s); break;
+    case 4: launch_classify_one<1, 1>(p, b, s); break;
+    case 5: launch_classify_one<1, 2>(p, b, s); break;
+    case 7: launch_classify_one<2, 1>(p, b, s); break;
+    case 8: launch_classify_one<2, 2>(p, b, s); break;
     default: return hipErrorInvalidValue;
     }
+    return hipGetLastError();
 }
 
 }  // namespace
@@ -653,12 +651,15 @@ hipError_t launch_pipeline(const PipeLaunch& p, const PipeBufs& b, hipStream_t s
         return hipGetLastError();
     }
     if (mark(0) != hipSuccess) return hipErrorUnknown;
-    if (launch_classify(p, b, s) != hipSuccess) return hipErrorInvalidValue;
+    // no pass is launched on the counters, keys or lists of one that was not
+    hipError_t e = launch_classify(p, b, s);
+    if (e != hipSuccess) return e;
     if (mark(1) != hipSuccess) return hipErrorUnknown;
     const uint32_t bin_grid = (uint32_t)((p.nslots + kBinSeg - 1) / kBinSeg);
     const uint32_t search_wgs = (p.search_grid + kSearchWaves - 1) / kSearchWaves;
     hipLaunchKernelGGL(txd::k_pipe_bin, dim3(bin_grid), dim3(256), 0, s, b.keys, (uint32_t)p.nslots, b.ctl, b.list[kListA],
                        b.list[kListB], b.list[kListC]);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
     if (mark(2) != hipSuccess) return hipErrorUnknown;
     if (p.lists & (1u << kListC))
         hipLaunchKernelGGL(txd::k_pipe_cluster, dim3(search_wgs), dim3(64 * kSearchWaves), 0, s, p.d_tex, p.tex0, b.recs,

@@ -105,26 +105,24 @@ constexpr uint32_t kSearchWaves = 4;  // waves per search workgroup (sharing one
 struct PipeLaunch {
     const txk::BatchTex* d_tex;  // texture descriptors, with d_chunks (null: only `tex0`)
     txk::BatchTex tex0;          // the texture when d_tex is null (ClusterFit or IterativeClusterFit)
-    const uint4* d_chunks;       // heavy chunks (texture, first block, count, first record slot);
-                                 // null with d_tex: implicit chunks of tex0
+    const uint4* d_chunks;       // heavy chunks (texture, first block, count, first record slot) of
+                                 // at most kClassifyBlocks blocks; null with d_tex: implicit chunks of tex0
     txk::ChainTable chain;       // count > 0: the levels of a chain, tex0 holding what they share and the
                                  // output; implicit chunks, already numbered
     uint32_t nchunks;            // heavy chunks
-    uint32_t chunk_blocks;       // chunk size (of a chunk list: the largest)
+    uint32_t chunk_blocks;       // size of the implicit chunks
     uint64_t nslots;             // record slots the chunks cover (<= capacity)
     uint32_t classify_grid;      // persistent 64-thread workgroups of classify
     uint32_t search_grid;        // persistent 64-thread workgroups of each search
     uint32_t lists;              // bit L set: records may go to list L (its search is launched)
 };
 
-// 64-block pieces of a chunk list: classify runs one block per lane, so a wave
-// takes a larger chunk piece by piece, each piece by whichever workgroup's
-// turn it is (a small batch tuned with 128-block chunks would otherwise leave
-// half the waves idle and take the others twice as long).
-inline uint64_t classify_pieces(const PipeLaunch& p)
-{
-    return (uint64_t)p.nchunks * ((p.chunk_blocks + 63u) / 64u);
-}
+// Blocks of a chunk that the classify pass takes in one step, one per lane of
+// its wave.  Larger chunks are listed as chunks of this size, so that the steps
+// are shared out among the workgroups (a small batch tuned with 128-block
+// chunks would otherwise leave half the waves idle and take the others twice
+// as long) and a large tuned size costs nothing.
+constexpr uint32_t kClassifyBlocks = 64;
 
 // The lists a texture's records can go to: ClusterFit -> C; BC1
 // IterativeClusterFit -> A and B; BC2/BC3 IterativeClusterFit -> B; RangeFit

@@ -225,19 +225,20 @@ bool tx_server::start_launch(Launch& L, std::vector<uint64_t>& ids, std::unique_
     uint64_t want = (colour_blocks + waves - 1) / std::max<uint64_t>(1, waves);
     want = std::max<uint64_t>(4, (want + 3) & ~(uint64_t)3);
     const uint32_t chunk = (uint32_t)std::min<uint64_t>(cfg.tuning.chunk_blocks, want);
+    const bool pipeline = cfg.tuning.pipeline && colour_blocks >= txc::pipeline_min_blocks() &&
+                          colour_blocks <= kServerPipeMaxBlocks;
+    const uint32_t heavy_chunk = pipeline ? std::min(chunk, txp::kClassifyBlocks) : chunk;
     // BC4/BC5 jobs: one block per lane in chunks of 512, or 16 lanes per block
     // in the colour chunks' size
     const uint32_t alpha_lanes = cfg.tuning.lanes_per_block == 16 ? 16u : 1u;
     const uint32_t light_chunk = alpha_lanes == 16 ? chunk : txk::kLightChunkBlocks;
-    const bool pipeline = cfg.tuning.pipeline && colour_blocks >= txc::pipeline_min_blocks() &&
-                          colour_blocks <= kServerPipeMaxBlocks;
     size_t nchunks = 0;
     std::vector<tx_job> specs;
     std::vector<size_t> in_offs, out_offs;
     for (uint64_t id : ids) {
         Job& j = jobs[id];
         const uint64_t nb = (uint64_t)((j.spec.width + 3) / 4) * ((j.spec.height + 3) / 4);
-        const uint32_t cb = j.spec.format >= TX_BC4 ? light_chunk : chunk;
+        const uint32_t cb = j.spec.format >= TX_BC4 ? light_chunk : heavy_chunk;
         nchunks += (size_t)((nb + cb - 1) / cb);
         specs.push_back(j.spec);
         in_offs.push_back(j.in_off);
@@ -291,7 +292,7 @@ bool tx_server::start_launch(Launch& L, std::vector<uint64_t>& ids, std::unique_
         const size_t k = order[q];
         const txk::BatchTex& t = L.h_tex[k];
         const bool light = t.variant >= 9u;
-        const uint32_t cb = light ? light_chunk : chunk;
+        const uint32_t cb = light ? light_chunk : heavy_chunk;
         for (uint32_t f = 0; f < t.nblocks; f += cb) {
             const uint32_t n = std::min(cb, t.nblocks - f);
             L.h_chunks[c++] = make_uint4((uint32_t)k, f, n, light ? 0u : slot);
@@ -308,7 +309,7 @@ bool tx_server::start_launch(Launch& L, std::vector<uint64_t>& ids, std::unique_
     if (ok && c && hipMemcpyAsync(L.d_chunks, L.h_chunks, sizeof(uint4) * c, hipMemcpyHostToDevice, L.stream) !=
                        hipSuccess)
         ok = false;
-    const txk::HeavyShape heavy = txk::heavy_shape(grid, nheavy, cfg.tuning.waves_per_group, chunk);
+    const txk::HeavyShape heavy = txk::heavy_shape(grid, nheavy, cfg.tuning.waves_per_group, heavy_chunk);
     const txk::AlphaShape light = txk::alpha_shape(cus, nlight, alpha_lanes, cfg.tuning.groups_per_cu,
                                                    cfg.tuning.waves_per_group);
     if (ok && use_pipe) {
@@ -321,8 +322,7 @@ bool tx_server::start_launch(Launch& L, std::vector<uint64_t>& ids, std::unique_
         p.d_chunks = L.d_chunks;
         p.nchunks = nheavy;
         p.nslots = slot;
-        p.chunk_blocks = chunk;
-        p.classify_grid = (uint32_t)std::min<uint64_t>(cus * txp::kClassifyWavesPerCu, txp::classify_pieces(p));
+        p.classify_grid = std::min<uint32_t>(cus * txp::kClassifyWavesPerCu, nheavy);
         p.search_grid = (uint32_t)std::min<uint64_t>((uint64_t)cus * txp::kSearchWavesPerCu, (slot + 3) / 4);
         p.lists = lists;
         if (ok && txp::launch_pipeline(p, L.pipe, L.stream) != hipSuccess) ok = false;
@@ -468,7 +468,7 @@ int tx_server_create(tx_server** out, const tx_server_config* config)
         // at the tuned chunk size, or one chunk per resident wave for small
         // launches, without growing while serving
         ok = ok && grow_chunks(L, (size_t)s->grid * cfg.tuning.waves_per_group +
-                                      ((size_t)1 << 20) / cfg.tuning.chunk_blocks +
+                                      ((size_t)1 << 20) / std::min(cfg.tuning.chunk_blocks, txp::kClassifyBlocks) +
                                       2 * (size_t)cfg.max_jobs_per_launch);
         // record scratch for the largest launch the arena can hold (its
         // inputs take 64 bytes per block), allocated once: a later free would
