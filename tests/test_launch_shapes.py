@@ -1,6 +1,7 @@
 """Launch shapes computed on the host, without a GPU: for every chunk size and
 number of chunks a batch may have, the pieces of the lockstep encoder's launch
-cover each chunk, and the piece count fits the kernel's 32 bits."""
+cover each chunk, and the piece count fits the kernel's 32 bits; the grid of
+the mip levels stays within a launch's limits for every image size."""
 import os
 import subprocess
 
@@ -15,6 +16,20 @@ int main()
 {
     unsigned long long groups; unsigned n, wpg, largest;
     while (scanf("%llu %u %u %u", &groups, &n, &wpg, &largest) == 4) {
+        if (groups == 0) {  // the mip levels of an n x wpg image: launches, widest grid, its rows
+            unsigned launches = 0, x = 0, y = 0;
+            unsigned long long covered = 0;
+            while (covered * txk::kMipTile < n) {
+                const dim3 g = txk::mip_grid(n, wpg, covered);
+                x = g.x > x ? g.x : x;
+                y = g.y;
+                covered += g.x;
+                ++launches;
+            }
+            if (covered != (n + 63ull) / 64) launches = 0;
+            printf("%u %u %u\n", launches, x, y);
+            continue;
+        }
         const txk::HeavyShape h = txk::heavy_shape(groups, n, wpg, largest);
         printf("%u %u %u\n", h.grid, h.per_chunk, h.span);
     }
@@ -56,3 +71,11 @@ def test_no_chunks_and_single_blocks(shapes):
     # no chunks at all (a batch without colour textures), and chunks below one step
     for grid, per_chunk, span in shapes([(3072, 0, 1, 0), (3072, 0, 4, 0), (3072, 1, 1, 1), (3072, 1, 2, 3)]):
         assert (grid, per_chunk, span) == (1, 1, 4)
+
+
+def test_mip_grid_within_launch_limits(shapes):
+    sides = [1, 63, 64, 65, 4096, (1 << 29) - 1, 1 << 29, (1 << 29) + 1, 1 << 30, (1 << 30) + 1, 0x7FFFFFFF]
+    rows = [(0, w, h, 0) for w in sides for h in sides]
+    for (_, w, h, _), (launches, widest, y) in zip(rows, shapes(rows)):
+        assert widest * 256 < 1 << 32 and 1 <= y < 1 << 16 and y <= (h + 63) // 64, (w, h)
+        assert launches == ((w + 63) // 64 + (1 << 23) - 1) >> 23, (w, h)

@@ -157,11 +157,14 @@ hipError_t reset_counters(uint32_t* d_counter, hipStream_t s);
 // most 2^16 and index workgroup y * gridDim.x + x (a grid-stride loop
 // instead made the compiler keep more registers live and cost the lockstep
 // kernel a wave per SIMD); the decoder caps its tile grid and walks larger
-// images grid-stride.
+// images grid-stride; the mip levels take a launch per 2^23 columns of
+// tiles (more than one above 2^29 texels wide) and walk rows grid-stride.
 constexpr uint64_t kGroupsPerRow = 1ull << 16;
 constexpr uint64_t kMaxGroups2d = kGroupsPerRow * 65535ull;
 constexpr uint64_t kMaxDecodeTilesX = 1ull << 16;  // 256-block tiles of the decoder per grid row
 constexpr uint64_t kMaxDecodeTilesY = 1ull << 14;
+constexpr uint64_t kMaxMipTilesX = 1ull << 23;     // 64 x 64 source tiles of the mip levels per grid row
+constexpr uint64_t kMaxMipTilesY = 1ull << 14;
 
 inline uint32_t capped_grid(uint64_t groups, uint64_t cap) { return (uint32_t)(groups < cap ? groups : cap); }
 
@@ -185,6 +188,13 @@ hipError_t launch_elementary(const float* d_in, uint32_t n, float* d_tables, flo
 // (w x h, 4-byte aligned) back to back into dst: 2x2 box of the level above,
 // edge clamp, (sum + 2) >> 2; level k is max(1, w >> k) x max(1, h >> k).
 constexpr uint32_t kMipLevelsPerLaunch = 6;
+constexpr uint32_t kMipTile = 64;  // source texels per side of a workgroup's tile
+// Grid of the launch that starts at tile column col0 (col0 * kMipTile < w).
+inline dim3 mip_grid(uint32_t w, uint32_t h, uint64_t col0)
+{
+    return dim3(capped_grid(((uint64_t)w + kMipTile - 1) / kMipTile - col0, kMaxMipTilesX),
+                capped_grid(((uint64_t)h + kMipTile - 1) / kMipTile, kMaxMipTilesY));
+}
 hipError_t launch_mip_levels(const uint8_t* src, uint32_t w, uint32_t h, uint32_t nout, uint8_t* dst, hipStream_t s);
 
 }  // namespace txk

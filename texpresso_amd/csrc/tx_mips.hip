@@ -9,13 +9,11 @@
 // texels of level 0 at its place only, and the clamp acts on sides of 1 alone.
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
-
 #include "bcn_kernels.hpp"
 
 namespace txd {
 
-constexpr uint32_t kTile = 64;  // source texels per side of a workgroup's tile
+constexpr uint32_t kTile = txk::kMipTile;  // source texels per side of a workgroup's tile
 
 typedef uint32_t mip4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint32_t mip2 __attribute__((ext_vector_type(2), aligned(4)));
@@ -30,8 +28,8 @@ __device__ __forceinline__ uint32_t mean4(uint32_t a, uint32_t b, uint32_t c, ui
     return ((e >> 2) & m) | (((o >> 2) & m) << 8);
 }
 
-// Levels 1..nout (nout <= 6) of the w x h image src, one 64 x 64 source tile
-// per workgroup: each thread averages 4 x 4 texels into 2 x 2 of level 1 and
+// Levels 1..nout (nout <= 6) of the w x h image src in the columns of tiles
+// from col0 on, one 64 x 64 source tile per workgroup: each thread averages 4 x 4 texels into 2 x 2 of level 1 and
 // one of level 2, and the tile's 16 x 16 texels of level 2 go down to one
 // texel of level 6 through LDS on the first wave.  The levels lie back to
 // back in dst.  Bound by memory: the source is read once and no level is read
@@ -39,12 +37,12 @@ __device__ __forceinline__ uint32_t mean4(uint32_t a, uint32_t b, uint32_t c, ui
 // dependent launch per level, a texel per thread with four 4-byte loads, took
 // 44.6 us.
 __global__ __launch_bounds__(256) void k_mip_levels(const uint32_t* __restrict__ src, uint32_t w, uint32_t h,
-                                                    uint32_t nout, uint32_t* __restrict__ dst)
+                                                    uint32_t nout, uint32_t* __restrict__ dst, uint32_t col0)
 {
     __shared__ uint32_t lds[16][17];
     const uint32_t tx = threadIdx.x & 15u, ty = threadIdx.x >> 4;
     const uint32_t w1 = max(1u, w >> 1), h1 = max(1u, h >> 1), w2 = max(1u, w1 >> 1), h2 = max(1u, h1 >> 1);
-    const uint32_t x0 = blockIdx.x * kTile + 4u * tx;
+    const uint32_t col = col0 + blockIdx.x, x0 = col * kTile + 4u * tx;
     for (uint64_t tile = blockIdx.y; tile * kTile < h; tile += gridDim.y) {
         const uint32_t y0 = (uint32_t)tile * kTile + 4u * ty;
         uint32_t p[4][4];
@@ -104,7 +102,7 @@ __global__ __launch_bounds__(256) void k_mip_levels(const uint32_t* __restrict__
                 if (in) lds[ly][lx] = m;
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                 __builtin_amdgcn_wave_barrier();
-                const uint32_t ox = blockIdx.x * side + lx, oy = (uint32_t)tile * side + ly;
+                const uint32_t ox = col * side + lx, oy = (uint32_t)tile * side + ly;
                 if (in && ox < nw && oy < nh) out[(size_t)oy * nw + ox] = m;
                 pw = nw;
                 ph = nh;
@@ -121,11 +119,14 @@ namespace txk {
 hipError_t launch_mip_levels(const uint8_t* src, uint32_t w, uint32_t h, uint32_t nout, uint8_t* dst, hipStream_t s)
 {
     if (w == 0 || h == 0 || nout == 0 || nout > kMipLevelsPerLaunch) return hipErrorInvalidValue;
-    const dim3 grid((w + txd::kTile - 1u) / txd::kTile,
-                    (uint32_t)std::min<uint64_t>(((uint64_t)h + txd::kTile - 1) / txd::kTile, 16384));
-    hipLaunchKernelGGL(txd::k_mip_levels, grid, dim3(256), 0, s, reinterpret_cast<const uint32_t*>(src), w, h, nout,
-                       reinterpret_cast<uint32_t*>(dst));
-    return hipGetLastError();
+    for (uint64_t col0 = 0; col0 * kMipTile < w; col0 += kMaxMipTilesX) {
+        hipLaunchKernelGGL(txd::k_mip_levels, mip_grid(w, h, col0), dim3(256), 0, s,
+                           reinterpret_cast<const uint32_t*>(src), w, h, nout, reinterpret_cast<uint32_t*>(dst),
+                           (uint32_t)col0);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 }  // namespace txk
