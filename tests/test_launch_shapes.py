@@ -1,7 +1,8 @@
 """Launch shapes computed on the host, without a GPU: for every chunk size and
 number of chunks a batch may have, the pieces of the lockstep encoder's launch
 cover each chunk, and the piece count fits the kernel's 32 bits; the grid of
-the mip levels stays within a launch's limits for every image size."""
+the mip levels stays within a launch's limits for every image size; and the
+lines of the direct kernels' teams."""
 import os
 import subprocess
 
@@ -28,6 +29,10 @@ int main()
             }
             if (covered != (n + 63ull) / 64) launches = 0;
             printf("%u %u %u\n", launches, x, y);
+            continue;
+        }
+        if (groups == 1) {  // the team of algorithm n for wpg blocks, on the library's and on a caller's stream
+            printf("%d %d 0\n", txk::team_groups(n, wpg, false), txk::team_groups(n, wpg, true));
             continue;
         }
         const txk::HeavyShape h = txk::heavy_shape(groups, n, wpg, largest);
@@ -79,3 +84,12 @@ def test_mip_grid_within_launch_limits(shapes):
     for (_, w, h, _), (launches, widest, y) in zip(rows, shapes(rows)):
         assert widest * 256 < 1 << 32 and 1 <= y < 1 << 16 and y <= (h + 63) // 64, (w, h)
         assert launches == ((w + 63) // 64 + (1 << 23) - 1) >> 23, (w, h)
+
+
+def test_team_lines(shapes):
+    # (algorithm, blocks): team on the library's own stream, team on a caller's
+    want = {(1, 1): (4, 4), (1, 2560): (4, 4), (1, 2561): (2, 2), (1, 6144): (2, 2), (1, 6145): (1, 1),
+            (2, 1): (4, 4), (2, 7168): (4, 4), (2, 7169): (4, 2), (2, 10240): (4, 2), (2, 10241): (2, 2),
+            (2, 32768): (2, 2), (2, 32769): (1, 1)}
+    got = shapes([(1, alg, n, 0) for alg, n in want])
+    assert {k: v[:2] for k, v in zip(want, got)} == want

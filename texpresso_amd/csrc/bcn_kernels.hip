@@ -413,23 +413,6 @@ __global__ __launch_bounds__(64) void k_elementary(const float* __restrict__ in,
 
 namespace {
 
-// Groups per block of the direct kernels.  A split search on 16 lanes takes a
-// wave 17 us (30-100 us for IterativeClusterFit) however few blocks there are;
-// on 32 or 64 lanes it takes half or a quarter, but a wave then holds 2 or 1
-// blocks and repeats what comes before the search.  Measured us for teams of 1
-// / 2 / 4 groups (BC1 ClusterFit): 27.5 / 18.5 / 14.4 at 256 blocks, 28.2 /
-// 23.4 / 20.8 at 2304, 27.9 / 23.4 / 24.8 at 3136, 33.8 / 29.0 / 35.2 at 5184,
-// 34.2 / 33.9 / 40.3 at 6400.  BC1 and BC3 IterativeClusterFit, several
-// searches a block: 120 / 68 / 48 and 99 / 61 / 39 at 256 blocks, 174 / 137 /
-// 130 and 174 / 134 / 116 at 9216, 164 / 140 / 150 and 178 / 147 / 136 at
-// 12544, 190 / 170 / 190 and 197 / 169 / 168 at 16384.
-int team_groups(int algorithm, uint64_t nblocks)
-{
-    const bool iterative = algorithm == 2;
-    if (nblocks <= (iterative ? 10240u : 2560u)) return 4;
-    return nblocks <= (iterative ? 32768u : 6144u) ? 2 : 1;
-}
-
 txd::Image image_of(const txk::EncodeArgs& a)
 {
     return txd::Image{a.rgba, a.width, a.height, a.blocks_wide, a.nblocks, a.out};
@@ -464,7 +447,7 @@ hipError_t launch_encode_n(const txk::EncodeArgs& a, txk::ChainTable* chain, hip
 template <int FMT, int ALG>
 hipError_t launch_encode_t(const txk::EncodeArgs& a, txk::ChainTable* chain, hipStream_t s)
 {
-    switch (team_groups(ALG, a.nblocks)) {
+    switch (txk::team_groups(ALG, a.nblocks, a.may_overlap)) {
     case 4: return launch_encode_n<FMT, ALG, 4>(a, chain, s);
     case 2: return launch_encode_n<FMT, ALG, 2>(a, chain, s);
     default: return launch_encode_n<FMT, ALG, 1>(a, chain, s);
@@ -536,7 +519,7 @@ template <int FMT, int ALG>
 hipError_t launch_blocks_t(const txk::BlockListArgs& a, hipStream_t s)
 {
     if constexpr (ALG != 0) {
-        const int t = team_groups(ALG, a.nblocks);
+        const int t = txk::team_groups(ALG, a.nblocks, false);
         if (t == 4) return launch_blocks_n<FMT, ALG, 4>(a, s);
         if (t == 2) return launch_blocks_n<FMT, ALG, 2>(a, s);
     }

@@ -15,7 +15,36 @@ struct EncodeArgs {
     uint8_t* out;      // device, nblocks * block_size bytes
     float wr, wg, wb;
     uint32_t weigh_alpha;
+    bool may_overlap;  // on a caller's stream, where calls on others may run beside this one
 };
+
+// Groups per block of the direct kernels.  A split search on 16 lanes takes a
+// wave 17 us (30-100 us for IterativeClusterFit) however few blocks there are;
+// on 32 or 64 lanes it takes half or a quarter, but a wave then holds 2 or 1
+// blocks and repeats what comes before the search.  Measured us for teams of 1
+// / 2 / 4 groups (BC1 ClusterFit): 27.5 / 18.5 / 14.4 at 256 blocks, 28.2 /
+// 23.4 / 20.8 at 2304, 27.9 / 23.4 / 24.8 at 3136, 33.8 / 29.0 / 35.2 at 5184,
+// 34.2 / 33.9 / 40.3 at 6400.  BC1 and BC3 IterativeClusterFit, several
+// searches a block: 120 / 68 / 48 and 99 / 61 / 39 at 256 blocks, 174 / 137 /
+// 130 and 174 / 134 / 116 at 9216, 164 / 140 / 150 and 178 / 147 / 136 at
+// 12544, 190 / 170 / 190 and 197 / 169 / 168 at 16384.
+// Those times are of calls one after another.  A longer team does more work in
+// all (its groups repeat the front), which calls that overlap on several
+// streams pay for: IterativeClusterFit on 8 streams, us a call for teams of 1 /
+// 2 / 4, BC1 37 / 28 / 36 and BC3 46 / 36 / 43 at 7056 blocks, 38 / 31 / 39 and
+// 47 / 39 / 48 at 7744, 42 / 39 / 50 and 53 / 47 / 59 at 9216.  So where a call
+// may overlap others (a texture on a caller's stream) the line of four lies
+// where teams of four still beat single groups on 8 streams; alone, such a call
+// of 7168..10240 blocks takes up to 1.3 times as long as with four (BC1 64 -> 71
+// us and BC3 70 -> 90 at 7744 blocks, 75 -> 76 and 79 -> 89 at 9216; single
+// groups took 121 and 172, 129 and 169).  The other lines hold for 8 streams too,
+// and a chain's one launch, which replaces its levels in series, for any.
+inline int team_groups(int algorithm, uint64_t nblocks, bool may_overlap)
+{
+    const bool iterative = algorithm == 2;
+    if (nblocks <= (iterative ? (may_overlap ? 7168u : 10240u) : 2560u)) return 4;
+    return nblocks <= (iterative ? 32768u : 6144u) ? 2 : 1;
+}
 
 struct BlockListArgs {
     int format;

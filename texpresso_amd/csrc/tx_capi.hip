@@ -169,6 +169,7 @@ static txk::EncodeArgs encode_args(int format, const tx_params* p, const uint8_t
     a.wg = p->weights[1];
     a.wb = p->weights[2];
     a.weigh_alpha = p->weigh_colour_by_alpha ? 1u : 0u;
+    a.may_overlap = false;
     return a;
 }
 
@@ -252,7 +253,7 @@ static txp::PipeLaunch pipe_launch_for(const txk::EncodeArgs& a, const txk::Chai
 // With `marks` (5 events) the pipeline records them between its kernels;
 // `used_pipeline` says which path ran.  With `chain`, the levels of a chain
 // instead of one texture (a.nblocks counts the blocks of them all).
-static hipError_t encode_on(txc::DeviceContext* ctx, const txk::EncodeArgs& a, hipStream_t s,
+static hipError_t encode_on(txc::DeviceContext* ctx, txk::EncodeArgs a, hipStream_t s,
                             const txk::ChainTable* chain = nullptr, hipEvent_t* marks = nullptr,
                             bool* used_pipeline = nullptr)
 {
@@ -260,6 +261,7 @@ static hipError_t encode_on(txc::DeviceContext* ctx, const txk::EncodeArgs& a, h
     // the pipeline's shared buffers are ordered between streams by events, which
     // a captured stream cannot wait for
     const bool own = s == ctx->stream;
+    a.may_overlap = !own && !chain;
     const auto direct = [&] { return chain ? txk::launch_encode_chain(a, *chain, s) : txk::launch_encode(a, s); };
     if (!takes_pipeline(a, own) || (!own && capturing(s))) return direct();
     std::lock_guard<std::mutex> lock(ctx->pipe_mu);
@@ -394,7 +396,8 @@ int tx_compress_device_noalloc(int format, const uint8_t* d_rgba, size_t width, 
     rc = noalloc_device(&dev);
     if (rc != TX_OK) return rc;
     const hipStream_t s = (hipStream_t)stream;
-    const txk::EncodeArgs a = encode_args(format, params, d_rgba, width, height, d_output, out_len);
+    txk::EncodeArgs a = encode_args(format, params, d_rgba, width, height, d_output, out_len);
+    a.may_overlap = true;
     if (!takes_pipeline(a, false)) return txk::launch_encode(a, s) == hipSuccess ? TX_OK : TX_ERR_HIP;
     if (a.nblocks > TX_NOALLOC_MAX_PIPELINE_BLOCKS) return TX_ERR_TOO_LARGE;
     txp::PipeBufs bufs;
