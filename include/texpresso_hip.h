@@ -283,6 +283,10 @@ int tx_util_copy(void* d_dst, const void* d_src, size_t bytes);
  * host pointers. */
 int tx_util_elementary(const float* in, size_t n, float u8f[256], float sqrt_counts[17], float sqrt_alpha[4096],
                        float* snap31, float* snap63, int32_t* round255);
+/* The split search's reciprocal of each of the n values (n <= 2^26): 1 / in[i],
+ * correctly rounded, for zeros, infinities, NaN and every |in[i]| in [2^-126,
+ * 2^126).  Synchronous; host pointers. */
+int tx_util_reciprocal(const float* in, size_t n, float* out);
 /* Enqueues `iters` tx_compress_device launches between two events on the
  * library stream, waits, and stores the elapsed milliseconds. */
 int tx_util_time_compress(int format, const uint8_t* d_rgba, size_t width, size_t height, const tx_params* params,

@@ -172,6 +172,7 @@ def lib():
             "tx_util_download": (c_int, [c_vp, c_vp, c_sz]),
             "tx_util_copy": (c_int, [c_vp, c_vp, c_sz]),
             "tx_util_elementary": (c_int, [c_vp, c_sz, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp]),
+            "tx_util_reciprocal": (c_int, [c_vp, c_sz, c_vp]),
             "tx_set_pipeline_threshold": (ctypes.c_uint64, [ctypes.c_uint64]),
             "tx_util_time_compress": (c_int, [c_int, c_vp, c_sz, c_sz, pp, c_vp, c_sz, c_int,
                                               ctypes.POINTER(ctypes.c_float)]),
@@ -437,6 +438,16 @@ def elementary(values):
            "elementary")
     return {"u8f": u8f, "sqrt_counts": sqc, "sqrt_alpha": sqa, "snap31": s31[:n], "snap63": s63[:n],
             "round255": r255[:n]}
+
+
+def reciprocal(values):
+    """The split search's reciprocal of each float32 in `values`, as the device
+    evaluates it (tx_util_reciprocal)."""
+    import numpy as np
+    v = np.ascontiguousarray(values, dtype=np.float32)
+    out = np.empty_like(v)
+    _check(lib().tx_util_reciprocal(v.ctypes.data, v.size, out.ctypes.data), "reciprocal")
+    return out
 
 
 def time_compress(fmt, d_rgba, width, height, params, d_out, out_len, iters):

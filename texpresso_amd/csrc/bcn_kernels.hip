@@ -407,6 +407,12 @@ __global__ __launch_bounds__(64) void k_elementary(const float* __restrict__ in,
     }
 }
 
+// recip() of each input, for the same check.
+__global__ __launch_bounds__(64) void k_reciprocal(const float* __restrict__ in, uint32_t n, float* __restrict__ out)
+{
+    for (uint32_t i = blockIdx.x * 64u + threadIdx.x; i < n; i += gridDim.x * 64u) out[i] = recip(in[i]);
+}
+
 }  // namespace txd
 
 // ---------------------------------------------------------------- launchers
@@ -580,6 +586,13 @@ hipError_t launch_elementary(const float* d_in, uint32_t n, float* d_tables, flo
     const uint32_t groups = (uint32_t)std::min<uint64_t>(4096, std::max<uint64_t>(1, ((uint64_t)n + 63) / 64));
     hipLaunchKernelGGL(txd::k_elementary, dim3(groups), dim3(64), 0, s, d_in, n, d_tables, d_snap31, d_snap63,
                        d_round255);
+    return hipGetLastError();
+}
+
+hipError_t launch_reciprocal(const float* d_in, uint32_t n, float* d_out, hipStream_t s)
+{
+    const uint32_t groups = (uint32_t)std::min<uint64_t>(4096, std::max<uint64_t>(1, ((uint64_t)n + 63) / 64));
+    hipLaunchKernelGGL(txd::k_reciprocal, dim3(groups), dim3(64), 0, s, d_in, n, d_out);
     return hipGetLastError();
 }
 

@@ -213,6 +213,8 @@ hipError_t launch_decode(int format, const uint8_t* data, uint32_t w, uint32_t h
 // 256 + 17 + 4096 floats; the three per-value outputs hold n entries each.
 hipError_t launch_elementary(const float* d_in, uint32_t n, float* d_tables, float* d_snap31, float* d_snap63,
                              int32_t* d_round255, hipStream_t s);
+// The reciprocal check (tx_util_reciprocal): n values in and out.
+hipError_t launch_reciprocal(const float* d_in, uint32_t n, float* d_out, hipStream_t s);
 // Levels 1..nout (1 <= nout <= kMipLevelsPerLaunch) of the RGBA8 image src
 // (w x h, 4-byte aligned) back to back into dst: 2x2 box of the level above,
 // edge clamp, (sum + 2) >> 2; level k is max(1, w >> k) x max(1, h >> k).

@@ -758,6 +758,24 @@ int tx_util_elementary(const float* in, size_t n, float u8f[256], float sqrt_cou
     return rc;
 }
 
+int tx_util_reciprocal(const float* in, size_t n, float* out)
+{
+    if (n > ((size_t)1 << 26) || (n && (!in || !out))) return TX_ERR_INVALID;
+    int rc = TX_OK;
+    txc::DeviceContext* ctx = txc::current_context(&rc);
+    if (!ctx) return rc;
+    if (n == 0) return TX_OK;
+    float* d = nullptr;
+    if (hipMalloc(&d, 8 * n) != hipSuccess) return TX_ERR_NOMEM;
+    if (hipMemcpyAsync(d, in, 4 * n, hipMemcpyHostToDevice, ctx->stream) != hipSuccess ||
+        txk::launch_reciprocal(d, (uint32_t)n, d + n, ctx->stream) != hipSuccess ||
+        hipMemcpyAsync(out, d + n, 4 * n, hipMemcpyDeviceToHost, ctx->stream) != hipSuccess)
+        rc = TX_ERR_HIP;
+    if (hipStreamSynchronize(ctx->stream) != hipSuccess) rc = TX_ERR_HIP;
+    (void)hipFree(d);
+    return rc;
+}
+
 int tx_util_time_compress(int format, const uint8_t* d_rgba, size_t width, size_t height, const tx_params* params,
                           uint8_t* d_output, size_t out_len, int iters, float* ms_total)
 {
