@@ -9,6 +9,8 @@
 // texels of level 0 at its place only, and the clamp acts on sides of 1 alone.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "bcn_kernels.hpp"
 
 namespace txd {
@@ -46,10 +48,11 @@ __global__ __launch_bounds__(256) void k_mip_levels(const uint32_t* __restrict__
     for (uint64_t tile = blockIdx.y; tile * kTile < h; tile += gridDim.y) {
         const uint32_t y0 = (uint32_t)tile * kTile + 4u * ty;
         uint32_t p[4][4];
-        if (x0 + 4u <= w && y0 + 4u <= h) {
+        if (x0 + 4u <= w) {
+            // past the last row, that row again
 #pragma unroll
             for (uint32_t y = 0; y < 4; ++y) {
-                const mip4 v = *reinterpret_cast<const mip4*>(src + (size_t)(y0 + y) * w + x0);
+                const mip4 v = *reinterpret_cast<const mip4*>(src + (size_t)min(y0 + y, h - 1u) * w + x0);
 #pragma unroll
                 for (uint32_t x = 0; x < 4; ++x) p[y][x] = v[x];
             }
@@ -112,13 +115,65 @@ __global__ __launch_bounds__(256) void k_mip_levels(const uint32_t* __restrict__
     }
 }
 
+// One level, a texel per thread with four 4-byte loads: where the tiles serve
+// badly (mip_levels_apart).
+__global__ __launch_bounds__(256) void k_mip_level(const uint32_t* __restrict__ src, uint32_t w, uint32_t h,
+                                                   uint32_t* __restrict__ dst, uint32_t nw, uint32_t nh)
+{
+    const uint32_t x = blockIdx.x * 64u + (threadIdx.x & 63u);
+    if (x >= nw) return;
+    const uint32_t x0 = min(2u * x, w - 1u), x1 = min(2u * x + 1u, w - 1u);
+    for (uint32_t y = blockIdx.y * 4u + (threadIdx.x >> 6); y < nh; y += gridDim.y * 4u) {
+        const size_t y0 = (size_t)min(2u * y, h - 1u) * w, y1 = (size_t)min(2u * y + 1u, h - 1u) * w;
+        dst[(size_t)y * nw + x] = mean4(src[y0 + x0], src[y0 + x1], src[y1 + x0], src[y1 + x1]);
+    }
+}
+
 }  // namespace txd
 
 namespace txk {
 
+namespace {
+
+// Whether nout levels of a w x h image go by a launch each.  A tile's threads
+// read 16-byte runs, which straddle cache lines when rows start at any 4-byte
+// address: where one level is all, so that reading the source once saves
+// nothing, a texel per thread is faster (4095 x 2047 8.6 us, 11.0 in tiles; 4096
+// x 2048 7.3 and 5.8).  And of an image below 16 rows a tile uses 64 threads or
+// fewer, so its time grows with the width where a launch stays at its 3 us (10^6
+// x 2, three levels 9.4 us, 19.2 in tiles; 300,000 x 7 9.3 and 7.5, one level 3.6
+// and 6.2; 100,000 x 1, three levels 9.5 and 4.1).
+bool mip_levels_apart(uint32_t w, uint32_t h, uint32_t nout)
+{
+    if (w >= 1u << 29) return false;  // the tiles' launches are cut by width
+    if (nout == 1 && w >= 64 && (w & 3u)) return true;
+    return h < 16 && w >= nout << 18;
+}
+
+hipError_t launch_mips_apart(const uint32_t* src, uint32_t w, uint32_t h, uint32_t nout, uint32_t* dst, hipStream_t s)
+{
+    for (uint32_t k = 0; k < nout; ++k) {
+        const uint32_t nw = std::max(1u, w >> 1), nh = std::max(1u, h >> 1);
+        const dim3 grid((nw + 63u) / 64u, capped_grid(((uint64_t)nh + 3) / 4, kMaxMipTilesY));
+        hipLaunchKernelGGL(txd::k_mip_level, grid, dim3(256), 0, s, src, w, h, dst, nw, nh);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        src = dst;
+        dst += (size_t)nw * nh;
+        w = nw;
+        h = nh;
+    }
+    return hipSuccess;
+}
+
+}  // namespace
+
 hipError_t launch_mip_levels(const uint8_t* src, uint32_t w, uint32_t h, uint32_t nout, uint8_t* dst, hipStream_t s)
 {
     if (w == 0 || h == 0 || nout == 0 || nout > kMipLevelsPerLaunch) return hipErrorInvalidValue;
+    if (mip_levels_apart(w, h, nout))
+        return launch_mips_apart(reinterpret_cast<const uint32_t*>(src), w, h, nout, reinterpret_cast<uint32_t*>(dst),
+                                 s);
     for (uint64_t col0 = 0; col0 * kMipTile < w; col0 += kMaxMipTilesX) {
         hipLaunchKernelGGL(txd::k_mip_levels, mip_grid(w, h, col0), dim3(256), 0, s,
                            reinterpret_cast<const uint32_t*>(src), w, h, nout, reinterpret_cast<uint32_t*>(dst),
