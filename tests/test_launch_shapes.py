@@ -2,7 +2,7 @@
 number of chunks a batch may have, the pieces of the lockstep encoder's launch
 cover each chunk, and the piece count fits the kernel's 32 bits; the grid of
 the mip levels stays within a launch's limits for every image size; and the
-lines of the direct kernels' teams."""
+lines of the direct kernels' teams and of RangeFit's groups."""
 import os
 import subprocess
 
@@ -29,6 +29,15 @@ int main()
             }
             if (covered != (n + 63ull) / 64) launches = 0;
             printf("%u %u %u\n", launches, x, y);
+            continue;
+        }
+        if (groups == 2) {  // blocks up to which RangeFit takes groups: format, width, height + 2^31 if weighed
+            txk::EncodeArgs a{};
+            a.format = n;
+            a.width = wpg;
+            a.height = largest & 0x7FFFFFFFu;
+            a.weigh_alpha = largest >> 31;
+            printf("%u 0 0\n", (unsigned)txk::range_group_blocks(a));
             continue;
         }
         if (groups == 1) {  // the team of algorithm n for wpg blocks, on the library's and on a caller's stream
@@ -93,3 +102,12 @@ def test_team_lines(shapes):
             (2, 32768): (2, 2), (2, 32769): (1, 1)}
     got = shapes([(1, alg, n, 0) for alg, n in want])
     assert {k: v[:2] for k, v in zip(want, got)} == want
+
+
+def test_range_lines(shapes):
+    w = 1 << 31  # weighed by alpha
+    want = {(0, 256, 256): 2560, (1, 256, 256): 2560, (2, 256, 256): 5120, (0, 257, 255): 2560, (2, 257, 256): 10240,
+            (2, 256, 255): 10240, (0, 3, 8192): 8192, (1, 8192, 1): 8192, (2, 3, 8192): 10240, (0, 256, 256 + w): 12288,
+            (1, 1, 64 + w): 12288, (2, 257, 256 + w): 12288}
+    got = shapes([(2, fmt, width, height) for fmt, width, height in want])
+    assert {k: v[0] for k, v in zip(want, got)} == want

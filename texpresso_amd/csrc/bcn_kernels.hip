@@ -115,8 +115,7 @@ __global__ __launch_bounds__(256) void k_encode_alpha_chain(txk::ChainTable chai
 // classify pass (alpha, colour set, principal axis, then the single-colour or
 // range fit) without its record path.  A RangeFit block is a few thousand
 // mostly serial operations; on a 16-lane group every fold would run on all 16
-// lanes (measured, BC1: 10.0 us against 9.0 at 256 blocks, 12.0 / 9.1 at 4096,
-// 18.3 / 9.2 at 16384).  Single-wave workgroups (the wave's LDS copies of the
+// lanes, which pays below range_group_blocks() only.  Single-wave workgroups (the wave's LDS copies of the
 // block pixels and weights): of four waves they were 3-5 % faster where the
 // blocks fill whole rounds of the GPU (2048^2 23.6 -> 22.8 us) and 3 % slower
 // between (344,000 blocks 31.1 -> 32.0 us).
@@ -442,11 +441,14 @@ hipError_t launch_encode_n(const txk::EncodeArgs& a, txk::ChainTable* chain, hip
     hipError_t e;
     const uint64_t groups = groups_for(a, chain, 4 / T, e);
     if (groups == 0) return e;
-    if (chain)
-        hipLaunchKernelGGL((txd::k_encode_chain<FMT, ALG, T>), txk::grid_2d(groups), dim3(64), 0, s, *chain, a.out,
-                           fit_of(a));
-    else
-        hipLaunchKernelGGL((txd::k_encode<FMT, ALG, T>), txk::grid_2d(groups), dim3(64), 0, s, image_of(a), fit_of(a));
+    if constexpr (ALG != 0) {  // a chain's RangeFit blocks are encoded one per lane
+        if (chain) {
+            hipLaunchKernelGGL((txd::k_encode_chain<FMT, ALG, T>), txk::grid_2d(groups), dim3(64), 0, s, *chain, a.out,
+                               fit_of(a));
+            return hipGetLastError();
+        }
+    }
+    hipLaunchKernelGGL((txd::k_encode<FMT, ALG, T>), txk::grid_2d(groups), dim3(64), 0, s, image_of(a), fit_of(a));
     return hipGetLastError();
 }
 
@@ -479,7 +481,9 @@ template <int FMT>
 hipError_t launch_encode_f(const txk::EncodeArgs& a, txk::ChainTable* chain, hipStream_t s)
 {
     switch (a.algorithm) {
-    case 0: return launch_encode_range<FMT>(a, chain, s);
+    case 0:
+        if (!chain && a.nblocks <= txk::range_group_blocks(a)) return launch_encode_n<FMT, 0, 1>(a, nullptr, s);
+        return launch_encode_range<FMT>(a, chain, s);
     case 1: return launch_encode_t<FMT, 1>(a, chain, s);
     default: return launch_encode_t<FMT, 2>(a, chain, s);
     }

@@ -46,6 +46,34 @@ inline int team_groups(int algorithm, uint64_t nblocks, bool may_overlap)
     return nblocks <= (iterative ? 32768u : 6144u) ? 2 : 1;
 }
 
+// RangeFit textures of up to this many blocks take the 16-lane groups, larger
+// ones a block per lane.  A wave of 64 blocks takes the time of their longest
+// serial chain, 9-10 us however few they are, 3 us more with point weights from
+// alpha (each lane then compares its 16 pixels pair by pair) and, for BC3, 3 us
+// more with partly masked blocks; a group's time follows its block's colours.
+// Measured us, groups / lanes, of seeded noise, and of the same with three
+// quarters of its tiles flat ("mixed"):
+//   BC1          2304 blocks 10.9 /  9.8, mixed 10.2 / 11.5;  4096 11.1 /  9.8, mixed 10.3 / 9.9
+//   BC2          1024 blocks  8.9 /  9.1;  2304  9.4 /  9.1;  4096  9.7 /  9.1
+//   BC3          2304 blocks  9.7 / 10.0, mixed  9.6 / 11.4;  4096 10.0 / 10.0;  6400 10.5 /  9.9
+//   BC3, a side no multiple of 4
+//                6561 blocks 10.5 / 12.4;  9409 13.3 / 12.7, 10,201 mixed 12.3 / 14.2;  12,321 14.3 / 12.7
+//   weighed by alpha, BC1 / BC2 / BC3
+//                8100 blocks 11.4 / 12.8,  9.9 / 12.0, 10.5 / 12.9;  12,100 12.9 / 12.8, 11.8 / 12.1,
+//                13.4 / 13.0;  14,400 16.2 / 12.8, 14.9 / 12.0, 16.3 / 13.0
+//   a side below 4, BC1 / BC2
+//                 512 blocks  5.9 / 9.4,  5.3 / 8.6;  5000 8.1 / 9.6, 7.5 / 8.8;  10,000 9.6 / 9.3, 9.4 / 8.5
+// Pictures of few colours keep the groups ahead to 12,000 blocks and more (BC1
+// with 8 levels a channel 6.9 / 11.3 at 2304, 8.5 / 10.1 at 12,100).
+inline uint64_t range_group_blocks(const EncodeArgs& a)
+{
+    const bool bc3 = a.format == 2;
+    if (a.weigh_alpha) return 12288;
+    if (bc3 && ((a.width | a.height) & 3u)) return 10240;
+    if (a.width < 4 || a.height < 4) return 8192;
+    return bc3 ? 5120 : 2560;
+}
+
 struct BlockListArgs {
     int format;
     int algorithm;
