@@ -307,10 +307,11 @@ int tx_util_time_phases(int format, const uint8_t* d_rgba, size_t width, size_t 
  * crossovers).  On a caller's stream, and in tx_compress_device_noalloc,
  * BC2/BC3 ClusterFit use 1.25x, BC1 ClusterFit 1.5x and BC1
  * IterativeClusterFit 3x; on the library's own stream, where calls do not
- * overlap, ClusterFit uses 0.5625x and BC1 IterativeClusterFit 1.75x.  A
- * stream being captured into a graph always gets the direct kernels (except
- * in tx_compress_device_noalloc).  A mip chain counts as one texture of all
- * its levels' blocks.  Both paths give identical bytes.  0 = always the
+ * overlap, ClusterFit uses 0.5625x (textures with weigh_colour_by_alpha 0.875x
+ * for BC1 and 1.25x for BC2/BC3), and BC1 IterativeClusterFit of a mip chain
+ * 1.75x.  A stream being captured into a graph always gets the direct kernels
+ * (except in tx_compress_device_noalloc).  A mip chain counts as one texture of
+ * all its levels' blocks.  Both paths give identical bytes.  0 = always the
  * pipeline, UINT64_MAX = never.
  * Process-wide; returns the previous value (default 32768). */
 uint64_t tx_set_pipeline_threshold(uint64_t min_blocks);

@@ -176,29 +176,43 @@ static txk::EncodeArgs encode_args(int format, const tx_params* p, const uint8_t
 // Blocks from which a texture goes through the binned pipeline, as a share of
 // the set threshold (default 32,768), in sixteenths: the measured crossings
 // against the direct kernels (square seeded textures, pipeline / direct us).
-// On the library's own stream calls run one after another: BC2/BC3
-// IterativeClusterFit 205 / 196 at 30,976 blocks, 220 / 239 at 36,864; BC1
-// IterativeClusterFit 253 / 250 at 50,176, 263 / 263 at 57,600; ClusterFit BC1
-// 58 / 59 at 16,384 (the direct kernel's last full round of waves), 68 / 84 at
-// 25,600, BC3 54 / 52 and 78 / 82.  Calls on a caller's stream may overlap
-// those on other streams, which only the direct kernels allow (three streams,
-// BC1 ClusterFit, per call: 100 / 73 at 40,000 blocks), so there the pipeline
-// starts later.
-static uint64_t pipeline_threshold(int format, int algorithm, bool own_stream)
+// BC2/BC3 IterativeClusterFit 205 / 196 at 30,976 blocks, 220 / 239 at 36,864.
+// BC1 IterativeClusterFit runs two searches after classify, which textures with
+// flat areas or few colours do not repay: of noise 250 / 247 at 57,600 blocks,
+// 284 / 282 at 73,984, 344 / 348 at 92,416 (of 1024 x 1024 259 / 315), of the
+// same with three quarters of its tiles flat 157 / 127, 172 / 140 and 189 / 154
+// (161 / 141), with 8 levels a channel 149 / 52, 153 / 63 and 133 / 74 (152 / 67).
+// ClusterFit on the library's own stream, where calls run one after another: BC1
+// 52 / 61 at 16,384 blocks (the direct kernel's last full round of waves), 51 /
+// 58 at 18,769, 60 / 63 at 25,600, 68 / 82 at 33,856, with flat tiles 38 / 38,
+// 39 / 49 and 40 / 56; BC3 55 / 52, 59 / 70, 76 / 83 and 91 / 102, with flat
+// tiles 40 / 43, 46 / 51 and 47 / 56.  (With 8 levels a channel the direct
+// kernels stay ahead by 4-11 us up to 40,000 blocks, BC3 28 / 18 at 18,769.)
+// With point weights from alpha classify takes longer: BC1 59 / 59 at 18,769, 71 /
+// 64 at 25,600, 72 / 78 at 29,584; BC3 71 / 71 at 20,736, 86 / 86 at 25,600, 97 /
+// 95 at 29,584 and 125 / 123 at 40,804.  A chain's small levels fill the direct
+// launch badly, so there the pipeline starts as early as without weights and for
+// BC1 IterativeClusterFit too (chains of noise of 61,801 blocks 274 / 316, 83,460
+// 318 / 354, with flat tiles 229 / 189 and 234 / 212).
+// Calls on a caller's stream may overlap those on other streams, which only the
+// direct kernels allow (three streams, BC1 ClusterFit, per call: 100 / 73 at
+// 40,000 blocks), so there the pipeline starts later.
+static uint64_t pipeline_threshold(const txk::EncodeArgs& a, bool is_chain, bool own_stream)
 {
     const uint64_t t = txc::pipeline_min_blocks();
-    const bool bc1 = format == TX_BC1, iterative = algorithm == TX_ITERATIVE_CLUSTER_FIT;
+    const bool bc1 = a.format == TX_BC1, iterative = a.algorithm == TX_ITERATIVE_CLUSTER_FIT;
     uint64_t sixteenths = bc1 ? (iterative ? 48 : 24) : (iterative ? 16 : 20);
-    if (own_stream) sixteenths = iterative ? (bc1 ? 28 : 16) : 9;
+    if (own_stream && !iterative) sixteenths = is_chain || !a.weigh_alpha ? 9 : bc1 ? 14 : 20;
+    if (own_stream && iterative && bc1 && is_chain) sixteenths = 28;
     return t > UINT64_MAX / sixteenths ? UINT64_MAX : t * sixteenths / 16;
 }
 
 // Whether a texture goes through the binned pipeline: ClusterFit or
 // IterativeClusterFit in BC1-BC3 with at least pipeline_threshold() blocks.
-static bool takes_pipeline(const txk::EncodeArgs& a, bool own_stream)
+static bool takes_pipeline(const txk::EncodeArgs& a, bool is_chain, bool own_stream)
 {
     const bool cluster = a.format <= TX_BC3 && a.algorithm != TX_RANGE_FIT;
-    return cluster && a.nblocks >= pipeline_threshold(a.format, a.algorithm, own_stream) && a.nblocks <= 0xFFFFFFFFull;
+    return cluster && a.nblocks >= pipeline_threshold(a, is_chain, own_stream) && a.nblocks <= 0xFFFFFFFFull;
 }
 
 // Whether `s` is being captured into a graph.
@@ -263,7 +277,7 @@ static hipError_t encode_on(txc::DeviceContext* ctx, txk::EncodeArgs a, hipStrea
     const bool own = s == ctx->stream;
     a.may_overlap = !own && !chain;
     const auto direct = [&] { return chain ? txk::launch_encode_chain(a, *chain, s) : txk::launch_encode(a, s); };
-    if (!takes_pipeline(a, own) || (!own && capturing(s))) return direct();
+    if (!takes_pipeline(a, chain != nullptr, own) || (!own && capturing(s))) return direct();
     std::lock_guard<std::mutex> lock(ctx->pipe_mu);
     txp::PipeBufs bufs;
     if (!ctx->pipe_scratch(a.nblocks, &bufs)) {
@@ -398,7 +412,7 @@ int tx_compress_device_noalloc(int format, const uint8_t* d_rgba, size_t width, 
     const hipStream_t s = (hipStream_t)stream;
     txk::EncodeArgs a = encode_args(format, params, d_rgba, width, height, d_output, out_len);
     a.may_overlap = true;
-    if (!takes_pipeline(a, false)) return txk::launch_encode(a, s) == hipSuccess ? TX_OK : TX_ERR_HIP;
+    if (!takes_pipeline(a, false, false)) return txk::launch_encode(a, s) == hipSuccess ? TX_OK : TX_ERR_HIP;
     if (a.nblocks > TX_NOALLOC_MAX_PIPELINE_BLOCKS) return TX_ERR_TOO_LARGE;
     txp::PipeBufs bufs;
     bufs.carve(dev->ptr, TX_NOALLOC_MAX_PIPELINE_BLOCKS);
