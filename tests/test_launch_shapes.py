@@ -1,6 +1,7 @@
 """Launch shapes computed on the host, without a GPU: for every chunk size and
 number of chunks a batch may have, the pieces of the lockstep encoder's launch
-cover each chunk, and the piece count fits the kernel's 32 bits; the grid of
+cover each chunk, and the piece count fits the kernel's 32 bits; alpha-only chunks are cut
+only as far as each wave gets at most one piece; the grid of
 the mip levels stays within a launch's limits for every image size; and the
 lines of the direct kernels' teams and of RangeFit's groups."""
 import os
@@ -29,6 +30,11 @@ int main()
             }
             if (covered != (n + 63ull) / 64) launches = 0;
             printf("%u %u %u\n", launches, x, y);
+            continue;
+        }
+        if (groups == 3) {  // the alpha-only launch of n chunks on wpg CUs: grid, steps, whether it draws work
+            const txk::AlphaShape s = txk::alpha_shape(wpg, n, 1, 12, 1);
+            printf("%u %u %u\n", s.grid, s.steps, (unsigned)txk::alpha_needs_counter(s, n, 1));
             continue;
         }
         if (groups == 2) {  // blocks up to which RangeFit takes groups: format, width, height + 2^31 if weighed
@@ -111,3 +117,15 @@ def test_range_lines(shapes):
             (1, 1, 64 + w): 12288, (2, 257, 256 + w): 12288}
     got = shapes([(2, fmt, width, height) for fmt, width, height in want])
     assert {k: v[0] for k, v in zip(want, got)} == want
+
+
+def test_alpha_pieces(shapes):
+    rows = [(3, n, cus, 0) for cus in (256, 304) for n in (1, 2, 3, 24, 1023, 1024, 1025, 1500, 2048, 2049, 4096, 4097,
+                                                           8192, 8193, 20000, 1 << 23)]
+    for (_, n, cus, _), (grid, steps, draws) in zip(rows, shapes(rows)):
+        waves, pieces = 32 * cus, n * (8 // steps)
+        case = (n, cus, grid, steps, draws)
+        assert steps in (1, 2, 4, 8) and grid == min((pieces + 3) // 4, waves // 4), case
+        assert bool(draws) == (pieces > 4 * grid) == (n > waves), case
+        if steps > 1:  # a finer cut would leave a wave more than one piece
+            assert 2 * pieces > waves, case

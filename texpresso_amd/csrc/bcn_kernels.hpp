@@ -127,8 +127,12 @@ constexpr uint32_t kLightChunkBlocks = 512;
 
 // Launch shape of the alpha-only kernel.  One block per lane: 4-wave
 // workgroups, up to 8 per CU, whose waves take pieces of `steps` steps (1, 2, 4
-// or 8) of a chunk: as large as leaves every wave one (a whole chunk takes a
-// wave 35 us, so a small batch is cut finer).  16 lanes per block: the LDS
+// or 8) of a chunk: as small as leaves each wave at most one (a whole chunk
+// takes a wave 35 us, so a small batch is cut finer).  More pieces than waves
+// would be drawn from the counter, whose thousands of atomics take longer than
+// the work, so only whole chunks are (BC4, 540,672 blocks in chunks of 512: 117
+// us in pieces of one step from the counter, 55 in whole chunks, 35 in pieces of
+// two).  16 lanes per block: the LDS
 // encoder's workgroups over whole chunks.
 struct AlphaShape {
     uint32_t grid, steps;
@@ -140,7 +144,7 @@ inline AlphaShape alpha_shape(uint32_t cus, uint32_t nlight, uint32_t alpha_lane
     AlphaShape a{0, 0};
     if (alpha_lanes != 16) {
         a.steps = kLightChunkBlocks / 64u;
-        while (a.steps > 1 && (uint64_t)a.pieces(nlight) < (uint64_t)cus * 32) a.steps /= 2;
+        while (a.steps > 1 && 2 * (uint64_t)a.pieces(nlight) <= (uint64_t)cus * 32) a.steps /= 2;
     }
     const uint64_t want = alpha_lanes == 16 ? ((uint64_t)nlight + waves_per_group - 1) / waves_per_group
                                             : ((uint64_t)a.pieces(nlight) + 3) / 4;
