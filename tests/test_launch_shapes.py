@@ -37,6 +37,11 @@ int main()
             printf("%u %u %u\n", s.grid, s.steps, (unsigned)txk::alpha_needs_counter(s, n, 1));
             continue;
         }
+        if (groups == 4) {  // the same beside the lockstep encoder
+            const txk::AlphaShape s = txk::alpha_shape(wpg, n, 1, 12, 1, true);
+            printf("%u %u %u\n", s.grid, s.steps, (unsigned)txk::alpha_needs_counter(s, n, 1));
+            continue;
+        }
         if (groups == 2) {  // blocks up to which RangeFit takes groups: format, width, height + 2^31 if weighed
             txk::EncodeArgs a{};
             a.format = n;
@@ -129,3 +134,11 @@ def test_alpha_pieces(shapes):
         assert bool(draws) == (pieces > 4 * grid) == (n > waves), case
         if steps > 1:  # a finer cut would leave a wave more than one piece
             assert 2 * pieces > waves, case
+
+
+def test_alpha_chunks_whole_beside_the_lockstep_encoder(shapes):
+    rows = [(4, n, cus, 0) for cus in (256, 304) for n in (1, 2, 3, 24, 460, 1024, 8192, 8193, 20000)]
+    for (_, n, cus, _), (grid, steps, draws) in zip(rows, shapes(rows)):
+        case = (n, cus, grid, steps, draws)
+        assert steps == 8 and grid == min((n + 3) // 4, 8 * cus), case
+        assert bool(draws) == (n > 32 * cus), case

@@ -132,19 +132,23 @@ constexpr uint32_t kLightChunkBlocks = 512;
 // would be drawn from the counter, whose thousands of atomics take longer than
 // the work, so only whole chunks are (BC4, 540,672 blocks in chunks of 512: 117
 // us in pieces of one step from the counter, 55 in whole chunks, 35 in pieces of
-// two).  16 lanes per block: the LDS
-// encoder's workgroups over whole chunks.
+// two).  Nor is a chunk cut `beside` the lockstep encoder of the same batch,
+// whose waves stay where they are placed: thousands of short waves that fill the
+// GPU ahead of them leave some SIMDs a wave more than others (12 textures of four
+// formats, 229,086 colour blocks in 1790 chunks of 128, ClusterFit 1125 us with
+// the alpha-only chunks cut, 904 with whole ones, RangeFit 394 / 347).  16 lanes
+// per block: the LDS encoder's workgroups over whole chunks.
 struct AlphaShape {
     uint32_t grid, steps;
     uint32_t pieces(uint32_t nlight) const { return steps ? nlight * (kLightChunkBlocks / 64u / steps) : nlight; }
 };
 inline AlphaShape alpha_shape(uint32_t cus, uint32_t nlight, uint32_t alpha_lanes, uint32_t groups_per_cu,
-                              uint32_t waves_per_group)
+                              uint32_t waves_per_group, bool beside = false)
 {
     AlphaShape a{0, 0};
     if (alpha_lanes != 16) {
         a.steps = kLightChunkBlocks / 64u;
-        while (a.steps > 1 && 2 * (uint64_t)a.pieces(nlight) <= (uint64_t)cus * 32) a.steps /= 2;
+        while (!beside && a.steps > 1 && 2 * (uint64_t)a.pieces(nlight) <= (uint64_t)cus * 32) a.steps /= 2;
     }
     const uint64_t want = alpha_lanes == 16 ? ((uint64_t)nlight + waves_per_group - 1) / waves_per_group
                                             : ((uint64_t)a.pieces(nlight) + 3) / 4;
