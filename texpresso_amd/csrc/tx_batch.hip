@@ -298,7 +298,11 @@ hipError_t launch_batch(tx_batch* b, hipStream_t s)
         return txk::launch_batch_raw(b->d_tex, b->d_chunks, b->nheavy, b->nchunks - b->nheavy, b->d_counter,
                                      b->heavy, b->light, b->tuning.waves_per_group, b->tuning.lanes_per_block,
                                      s, b->light_stream, b->fork, b->join);
-    // alpha-only chunks on the side stream, the binned pipeline on `s`
+    // alpha-only chunks on the side stream, the binned pipeline on `s`; the
+    // 16-lane alpha kernel ends before the searches start: four workgroups of a
+    // search take all of a CU's LDS and stay, and what the alpha kernel's smaller
+    // pieces leave free in between does not hold a fourth (a ClusterFit search
+    // of 252,178 blocks 385 us, 500 when it started beside them)
     const uint32_t nlight = b->nchunks - b->nheavy;
     if (nlight && txk::alpha_needs_counter(b->light, nlight, b->tuning.lanes_per_block))
         hipLaunchKernelGGL(txd::k_reset_counter, dim3(1), dim3(1), 0, s, b->d_counter);
@@ -311,7 +315,9 @@ hipError_t launch_batch(tx_batch* b, hipStream_t s)
     if (nlight && txk::launch_alpha_chunks(b->d_tex, b->d_chunks, b->nheavy, nlight, b->d_counter + 1, b->light,
                                            b->tuning.lanes_per_block, b->tuning.waves_per_group, sl) != hipSuccess)
         return hipErrorUnknown;
+    if (sl != s && hipEventRecord(b->join, sl) != hipSuccess) return hipErrorUnknown;
     txp::PipeLaunch p{};
+    if (sl != s && b->tuning.lanes_per_block == 16) p.before_search = b->join;
     p.d_tex = b->d_tex;
     p.d_chunks = b->d_chunks;
     p.nchunks = b->nheavy;
@@ -321,10 +327,7 @@ hipError_t launch_batch(tx_batch* b, hipStream_t s)
     p.lists = b->pipe_lists;
     const hipError_t e = txp::launch_pipeline(p, b->pipe, s);
     if (e != hipSuccess) return e;
-    if (nlight && b->light_stream) {
-        if (hipEventRecord(b->join, b->light_stream) != hipSuccess || hipStreamWaitEvent(s, b->join, 0) != hipSuccess)
-            return hipErrorUnknown;
-    }
+    if (sl != s && hipStreamWaitEvent(s, b->join, 0) != hipSuccess) return hipErrorUnknown;
     return hipGetLastError();
 }
 

@@ -661,6 +661,7 @@ hipError_t launch_pipeline(const PipeLaunch& p, const PipeBufs& b, hipStream_t s
                        b.list[kListB], b.list[kListC]);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if (mark(2) != hipSuccess) return hipErrorUnknown;
+    if (p.before_search && (e = hipStreamWaitEvent(s, p.before_search, 0)) != hipSuccess) return e;
     if (p.lists & (1u << kListC))
         hipLaunchKernelGGL(txd::k_pipe_cluster, dim3(search_wgs), dim3(64 * kSearchWaves), 0, s, p.d_tex, p.tex0, b.recs,
                            b.list[kListC], (uint32_t)p.nslots, b.ctl);

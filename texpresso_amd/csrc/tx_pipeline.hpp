@@ -115,6 +115,7 @@ struct PipeLaunch {
     uint32_t classify_grid;      // persistent 64-thread workgroups of classify
     uint32_t search_grid;        // persistent 64-thread workgroups of each search
     uint32_t lists;              // bit L set: records may go to list L (its search is launched)
+    hipEvent_t before_search;    // when given, the searches start after it
 };
 
 // Blocks of a chunk that the classify pass takes in one step, one per lane of
