@@ -51,6 +51,16 @@ int main()
             printf("%u 0 0\n", (unsigned)txk::range_group_blocks(a));
             continue;
         }
+        if (groups == 5) {  // the same for input read over the bus
+            txk::EncodeArgs a{};
+            a.format = n;
+            a.width = wpg;
+            a.height = largest & 0x7FFFFFFFu;
+            a.weigh_alpha = largest >> 31;
+            a.over_bus = true;
+            printf("%u 0 0\n", (unsigned)txk::range_group_blocks(a));
+            continue;
+        }
         if (groups == 1) {  // the team of algorithm n for wpg blocks, on the library's and on a caller's stream
             printf("%d %d 0\n", txk::team_groups(n, wpg, false), txk::team_groups(n, wpg, true));
             continue;
@@ -142,3 +152,11 @@ def test_alpha_chunks_whole_beside_the_lockstep_encoder(shapes):
         case = (n, cus, grid, steps, draws)
         assert steps == 8 and grid == min((n + 3) // 4, 8 * cus), case
         assert bool(draws) == (n > 32 * cus), case
+
+
+def test_range_lines_over_the_bus(shapes):
+    w = 1 << 31  # weighed by alpha
+    want = {(0, 256, 256): 512, (2, 256, 256): 512, (2, 257, 256): 512, (1, 256, 256 + w): 1280, (0, 4, 4): 512,
+            (0, 3, 8192): 8192, (1, 8192, 1): 8192, (2, 3, 8192): 10240, (1, 1, 64 + w): 12288}
+    got = shapes([(5, fmt, width, height) for fmt, width, height in want])
+    assert {k: v[0] for k, v in zip(want, got)} == want

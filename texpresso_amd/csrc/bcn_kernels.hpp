@@ -16,6 +16,7 @@ struct EncodeArgs {
     float wr, wg, wb;
     uint32_t weigh_alpha;
     bool may_overlap;  // on a caller's stream, where calls on others may run beside this one
+    bool over_bus;     // rgba is host memory that the kernels read over the bus
 };
 
 // Groups per block of the direct kernels.  A split search on 16 lanes takes a
@@ -65,9 +66,16 @@ inline int team_groups(int algorithm, uint64_t nblocks, bool may_overlap)
 //                 512 blocks  5.9 / 9.4,  5.3 / 8.6;  5000 8.1 / 9.6, 7.5 / 8.8;  10,000 9.6 / 9.3, 9.4 / 8.5
 // Pictures of few colours keep the groups ahead to 12,000 blocks and more (BC1
 // with 8 levels a channel 6.9 / 11.3 at 2304, 8.5 / 10.1 at 12,100).
+// Input read over the bus is fetched 16 bytes at a time by a group and in long
+// runs by the lanes, so there the line lies lower (whole host calls, groups /
+// lanes: BC1 25.7 / 24.4 at 256 blocks, 26.9 / 25.3 at 576, 28.2 / 25.7 at 1024,
+// of few colours 22.1 / 25.2, 23.0 / 25.4 and 23.7 / 26.0; weighed 28.2 / 28.6
+// at 1024, 30.6 / 29.4 at 1600; BC3 67.6 / 48.2 at 8281), except for sides below
+// 4, whose rows are long (2000 blocks 24.2 / 26.0, 4000 weighed 27.6 / 32.4).
 inline uint64_t range_group_blocks(const EncodeArgs& a)
 {
     const bool bc3 = a.format == 2;
+    if (a.over_bus && a.width >= 4 && a.height >= 4) return a.weigh_alpha ? 1280 : 512;
     if (a.weigh_alpha) return 12288;
     if (bc3 && ((a.width | a.height) & 3u)) return 10240;
     if (a.width < 4 || a.height < 4) return 8192;

@@ -170,6 +170,7 @@ static txk::EncodeArgs encode_args(int format, const tx_params* p, const uint8_t
     a.wb = p->weights[2];
     a.weigh_alpha = p->weigh_colour_by_alpha ? 1u : 0u;
     a.may_overlap = false;
+    a.over_bus = false;
     return a;
 }
 
@@ -296,7 +297,8 @@ static hipError_t encode_on(txc::DeviceContext* ctx, txk::EncodeArgs a, hipStrea
 // Kernels read pinned input themselves up to this size.  The decoder and the
 // one-block-per-lane encoders read it once in long runs: no copy is faster at
 // every staged size (RangeFit 512^2 71 us against 83 with one, 64^2 24 / 27;
-// decoding 512^2 68 / 80, 64^2 16 / 21).  The 16-lane groups of the cluster
+// decoding 512^2 68 / 80, 64^2 16 / 21), and RangeFit takes its groups for few
+// blocks of such input only (txk::range_group_blocks).  The 16-lane groups of the cluster
 // fits fetch 16 bytes at a time over the bus, which a copy beats from about 64
 // KiB on (BC1 ClusterFit 64^2 31 us against 32 with a copy, 128^2 41 / 40,
 // 256^2 64 / 59).
@@ -333,6 +335,8 @@ public:
         }
         return hipMemcpyAsync(d_buf, src, n, hipMemcpyHostToDevice, ctx->stream) == hipSuccess ? d_buf : nullptr;
     }
+    // Whether upload() hands out the pinned memory itself.
+    bool reads_pinned() const { return direct_in; }
     // Where kernels write the output: d_buf, or the pinned memory.
     uint8_t* output(uint8_t* d_buf) { return stage_out ? pin + txc::kStageBytes : d_buf; }
     // Waits for the call's work and leaves its n bytes of output in dst.
@@ -372,9 +376,9 @@ int tx_compress(int format, const uint8_t* rgba, size_t rgba_len, size_t width, 
     const uint8_t* d_in = call.upload(d, rgba, in_bytes);
     uint8_t* d_out = call.output(d + in_cap);
     if (!d_in) return TX_ERR_HIP;
-    if (encode_on(ctx, encode_args(format, params, d_in, width, height, d_out, out_len), ctx->stream) !=
-        hipSuccess)
-        return TX_ERR_HIP;
+    txk::EncodeArgs a = encode_args(format, params, d_in, width, height, d_out, out_len);
+    a.over_bus = call.reads_pinned();
+    if (encode_on(ctx, a, ctx->stream) != hipSuccess) return TX_ERR_HIP;
     return call.finish(output, d_out, out_len);
 }
 
