@@ -140,11 +140,13 @@ constexpr uint32_t kLightChunkBlocks = 512;
 // would be drawn from the counter, whose thousands of atomics take longer than
 // the work, so only whole chunks are (BC4, 540,672 blocks in chunks of 512: 117
 // us in pieces of one step from the counter, 55 in whole chunks, 35 in pieces of
-// two).  Nor is a chunk cut `beside` the lockstep encoder of the same batch,
-// whose waves stay where they are placed: thousands of short waves that fill the
-// GPU ahead of them leave some SIMDs a wave more than others (12 textures of four
-// formats, 229,086 colour blocks in 1790 chunks of 128, ClusterFit 1125 us with
-// the alpha-only chunks cut, 904 with whole ones, RangeFit 394 / 347).  16 lanes
+// two).  Nor is a chunk cut `beside` the lockstep encoder over whole chunks of the
+// same batch, whose waves stay where they are placed: thousands of short waves
+// that fill the GPU ahead of them leave some SIMDs a wave more than others (12
+// textures of four formats, 229,086 colour blocks in 1790 chunks of 128,
+// ClusterFit 1125 us with the alpha-only chunks cut, 904 with whole ones, RangeFit
+// 394 / 347).  Where the colour chunks are cut as well, the shorter waves are the
+// better ones (6 textures, 96,455 colour blocks, RangeFit 135 / 149).  16 lanes
 // per block: the LDS encoder's workgroups over whole chunks.
 struct AlphaShape {
     uint32_t grid, steps;

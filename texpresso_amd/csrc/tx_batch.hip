@@ -455,7 +455,7 @@ int tx_batch_create(tx_batch** out, const tx_texture* textures, size_t count, co
     // CU), or 16 lanes per block in the tuned workgroups
     const uint32_t nlight = b->nchunks - b->nheavy;
     b->light = txk::alpha_shape((uint32_t)prop.multiProcessorCount, nlight, t.lanes_per_block, t.groups_per_cu,
-                                t.waves_per_group, b->nheavy && !t.pipeline);
+                                t.waves_per_group, b->nheavy && !t.pipeline && b->heavy.per_chunk == 1);
     if (nlight && b->nheavy) {
         if (hipStreamCreateWithFlags(&b->light_stream, hipStreamNonBlocking) != hipSuccess ||
             hipEventCreateWithFlags(&b->fork, hipEventDisableTiming) != hipSuccess ||
