@@ -42,17 +42,6 @@ struct FitParams {
     uint32_t weigh_alpha;  // Params::weigh_colour_by_alpha
 };
 
-// LDS of the front half of a block (colour set, principal axis, single and
-// range fits): the pixels and the distinct colours, 320 bytes.  The front
-// functions take any LDS type with `pts` and the put_pix / pix accessors.
-struct __align__(16) FrontLds {
-    float4 pts[16];       // distinct colours: x, y, z, sqrt(weight)
-    uint32_t pixels[16];  // the block's RGBA8 pixels
-
-    __device__ void put_pix(int l, uint32_t px) { pixels[l] = px; }
-    __device__ uint32_t pix(int m) const { return pixels[m]; }
-};
-
 // Per-group LDS (one per 4x4 block in flight), 2544 bytes, so that 16
 // single-wave workgroups (64 groups) fit in a CU's 160 KiB.  The first 80
 // bytes of the prefix table are also scratch while they hold nothing live:
@@ -312,8 +301,7 @@ struct ColourSet {
 
 // lib/src/math.rs:44-97: weighted covariance of the n points in LDS, then
 // eight power-iteration steps.  Folds run in point order on every lane.
-template <class LDS>
-__device__ __forceinline__ void principal_axis(const LDS& L, int n, float& vx, float& vy, float& vz)
+__device__ __forceinline__ void principal_axis(const GroupLds& L, int n, float& vx, float& vy, float& vz)
 {
     float total = 0.0f, cx = 0.0f, cy = 0.0f, cz = 0.0f;
 #pragma unroll
@@ -384,8 +372,8 @@ __device__ __forceinline__ uint32_t single_endpoints(int tr, int tg, int cr, int
 }
 
 // single.rs:100-164
-template <int FMT, class LDS>
-__device__ __forceinline__ void single_fit(const LDS& L, const ColourSet& cs, int l, uint32_t& lo, uint32_t& hi)
+template <int FMT>
+__device__ __forceinline__ void single_fit(const GroupLds& L, const ColourSet& cs, int l, uint32_t& lo, uint32_t& hi)
 {
     const float4 q = L.pts[0];
     const int cr = f32_to_i32_clamped(q.x * 255.0f, 255);
@@ -481,8 +469,8 @@ __device__ __forceinline__ void ends_axis(uint32_t a, uint32_t b, float& x, floa
 }
 
 // range.rs:44-192
-template <int FMT, class LDS>
-__device__ __forceinline__ void range_fit(const LDS& L, const ColourSet& cs, int l, const FitParams& fp,
+template <int FMT>
+__device__ __forceinline__ void range_fit(const GroupLds& L, const ColourSet& cs, int l, const FitParams& fp,
                                           float px, float py, float pz, uint32_t& lo, uint32_t& hi)
 {
     const int n = cs.n;
@@ -1419,8 +1407,8 @@ __device__ __forceinline__ void set_colour(uint32_t (&out)[4], uint32_t lo, uint
 // Returns the fit kind; for KIND_CLUSTER the principal axis comes back in
 // (vx, vy, vz) and the colour half is left to the caller.  Every lane of the
 // wave must call this (LDS hand-offs inside).
-template <int FMT, int ALG, class LDS>
-__device__ __forceinline__ int encode_front(uint32_t px, bool valid, const FitParams& fp, LDS& L, int g, int l,
+template <int FMT, int ALG>
+__device__ __forceinline__ int encode_front(uint32_t px, bool valid, const FitParams& fp, GroupLds& L, int g, int l,
                                             uint32_t (&out)[4], ColourSet& cs, float& vx, float& vy, float& vz)
 {
     const int gshift = 16 * g;
