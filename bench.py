@@ -42,14 +42,21 @@ def split_counts(n):
 C3 = np.array([split_counts(n)[0] for n in range(17)], np.float64)
 C4 = np.array([split_counts(n)[1] for n in range(17)], np.float64)
 
+# FP32 operations of one split (a fused multiply-add counts two): the terms
+# that splits of one tile of 2 x 2 have in common are counted once for the
+# tile, and the weight terms not at all, which 16 colours of weight 1 take from
+# a table.  Per split: the three channels' error 92, alphax and betax 18, a
+# quarter of the tile's 30 common ones; 3-colour splits have no tiles (92 + 18).
+OPS4, OPS3 = 92 + 18 + 30 / 4, 92 + 18
+
 
 def search_flops(stats):
     """The part of algorithmic_flops spent in the split searches (per-split
     costs plus the per-ordering work), split by pass: (3-colour, 4-colour)."""
     n = stats["count"].clip(0, 16)
     cl = stats["fit"] == 2
-    f3 = np.where(cl, C3[n] * 138 * stats["searched3"] + 450 * stats["searched3"], 0.0)
-    f4 = np.where(cl, C4[n] * 159 * stats["searched4"] + 450 * stats["searched4"], 0.0)
+    f3 = np.where(cl, C3[n] * OPS3 * stats["searched3"] + 450 * stats["searched3"], 0.0)
+    f4 = np.where(cl, C4[n] * OPS4 * stats["searched4"] + 450 * stats["searched4"], 0.0)
     return float(f3.sum()), float(f4.sum())
 
 
@@ -69,14 +76,13 @@ def profiled_traffic(kernel, workload):
 
 
 def algorithmic_flops(stats):
-    """Counted FP32 operations of the colour fits (per-split costs of the
-    reference expression tree: 138 for a 3-colour split, 159 for a 4-colour
+    """FP32 operations that the colour fits cannot do without (OPS3 and OPS4 per
     split, plus ~1.4k per ClusterFit block and 0.45k per ordering; RangeFit
     ~1.5k per block)."""
     n = stats["count"].clip(0, 16)
     cl = stats["fit"] == 2
     orders = stats["searched3"] + stats["searched4"]
-    f = np.where(cl, C3[n] * 138 * stats["searched3"] + C4[n] * 159 * stats["searched4"] + 1400 + 450 * orders, 0.0)
+    f = np.where(cl, C3[n] * OPS3 * stats["searched3"] + C4[n] * OPS4 * stats["searched4"] + 1400 + 450 * orders, 0.0)
     f += np.where(stats["fit"] == 1, 1500.0, 0.0)
     return float(f.sum())
 
