@@ -4,9 +4,9 @@
 //
 // classify: alpha, colour set and fit choice for every block, one block per
 //   lane; single-colour and range-fit blocks are finished here, ClusterFit
-//   blocks become a ClusterRec and are counted by distinct-colour count n.
+//   blocks become a ClusterRec.
 // bin: the records into one list per pass, many-coloured ones first and
-//   neighbours of one colour count
+//   neighbours of nearly one distinct-colour count n
 //   (list A: BC1 IterativeClusterFit records for the 3-colour search; list
 //   B: records that need the 4-colour search -- BC1 IterativeClusterFit
 //   without transparency, BC2/BC3 IterativeClusterFit; list C: ClusterFit
@@ -14,8 +14,8 @@
 // search<NC>: persistent waves; each 16-lane group pulls the next record
 //   from its list and runs that block's ordering iterations on its own, so
 //   blocks with one ordering and blocks with several share a wave without
-//   waiting for each other, and neighbouring records have the same n (the
-//   same number of candidate rounds).
+//   waiting for each other, and neighbouring records have about the same n
+//   (the same number of candidate rounds).
 // cluster: ClusterFit (a single ordering per search): each group pulls a
 //   record and runs its searches on it (BC1: 3-colour then 4-colour).
 #pragma once
@@ -95,9 +95,9 @@ struct PipeBufs {
 
 // Resident waves per CU: classify (single-wave workgroups, one block per
 // lane) is limited by registers and LDS (8 KiB of pixel and weight copies
-// per workgroup), the searches by LDS and registers (4 x 2512 B per wave);
-// both fit 4 waves per SIMD.  The 16-colour searches run kSearchWaves waves
-// per workgroup (k_pipe_search), ClusterFit's single wave (k_pipe_cluster).
+// per workgroup), the searches by LDS and registers (4 x 2544 B per wave,
+// so that four search workgroups of kSearchWaves waves take a CU's 160 KiB);
+// both fit 4 waves per SIMD.
 constexpr uint32_t kClassifyWavesPerCu = 16;
 constexpr uint32_t kSearchWavesPerCu = 16;
 constexpr uint32_t kSearchWaves = 4;  // waves per search workgroup (sharing one run of list positions)

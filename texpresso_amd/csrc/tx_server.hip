@@ -121,8 +121,8 @@ struct Launch {
 };
 
 // Largest number of BC1-BC3 blocks a launch sends through the binned
-// pipeline (records: 192 bytes each, so 0.8 GB per launch slot at most);
-// larger launches use the lockstep persistent kernel.
+// pipeline (232 bytes a block for record, key and lists, so 0.97 GB per launch
+// slot at most); larger launches use the lockstep persistent kernel.
 constexpr uint64_t kServerPipeMaxBlocks = 4u << 20;
 
 }  // namespace
