@@ -38,8 +38,16 @@ struct EncodeArgs {
 // where teams of four still beat single groups on 8 streams; alone, such a call
 // of 7168..10240 blocks takes up to 1.3 times as long as with four (BC1 64 -> 71
 // us and BC3 70 -> 90 at 7744 blocks, 75 -> 76 and 79 -> 89 at 9216; single
-// groups took 121 and 172, 129 and 169).  The other lines hold for 8 streams too,
-// and a chain's one launch, which replaces its levels in series, for any.
+// groups took 121 and 172, 129 and 169).  The other lines are those of calls one
+// after another, since what teams of two gain alone is more than they lose on 8
+// streams (groups of 1 / 2, alone and on 8: IterativeClusterFit BC3 16,384 blocks
+// 147 / 127 and 87 / 90, 30,625 210 / 197 and 151 / 164, BC1 30,625 171 / 150 and
+// 109 / 117; ClusterFit BC3 6084 30.8 / 28.0 and 19.0 / 21.5, BC1 34.7 / 30.0 and
+// 18.0 / 15.9).  Pictures of few colours have short searches and pay for the front
+// alone (8 levels a channel, IterativeClusterFit BC3, groups of 1 / 2 / 4: 5625
+// blocks 22.7 / 21.2 / 24.2 and on 8 streams 8.5 / 9.7 / 13.7, 16,384 23.9 / 30.5
+// and 14.6 / 22.1).  A chain's one launch, which replaces its levels in series,
+// keeps these lines on any stream.
 inline int team_groups(int algorithm, uint64_t nblocks, bool may_overlap)
 {
     const bool iterative = algorithm == 2;
